@@ -117,9 +117,9 @@ int tvh_batch_plan_create(const tvh_table_desc* tables, size_t count, tvh_batch_
         u64 m = t.target_len;
         u64* leaves = t.tree + 5 * merkle_level_base(m, 0, t.layout);
         h.push_back(HashArgs{t.codewords, m, (u32)t.num_cols, leaves});
-        hb.push_back((u32)((m + 255) / 256));
+        hb.push_back(sponge_blocks(m));
         std::vector<MerkleGroup> groups;
-        merkle_groups(t.tree, m, t.layout, groups);
+        merkle_groups(t.tree, m, t.layout, true, groups);
         for (size_t g = 0; g < groups.size(); g++) {
             if (ma.size() <= g) {
                 ma.resize(g + 1);

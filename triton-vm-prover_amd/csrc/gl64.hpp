@@ -234,6 +234,182 @@ __host__ __device__ __forceinline__ u64 mul_lazy(u64 a, u64 b) {
 // a, b any u64 -> canonical
 __host__ __device__ __forceinline__ u64 mul(u64 a, u64 b) { return canon_raw(mul_lazy(a, b)); }
 
+// ---- products with the unlikely borrow set aside (device only) -----------------
+// The product l + h*2^64 (h = h1:h0) folds to (l + h0*(2^32 - 1)) - h1.  Its
+// 64-bit sum u carries about every second time (the carry c adds 2^32 - 1 back),
+// but u < h1 with c = 0 needs u below 2^32: one product in 2^32 of random
+// operands.  The *_rare forms leave that case to the caller: they add the lane
+// to `bad` and their result is then wrong; the caller branches on `bad` once for
+// many products and redoes them with the exact forms (mul_lazy, ...).  A fold is
+// then 4 VALU operations (a multiply-add and three carry operations) where
+// montyred and fold128 take 8 and more.
+//
+// Carries are lane masks in SGPR pairs, named by asm because the language has
+// no word for the carry out of v_mad_u64_u32 and the compiler turns sums with
+// two carries in into selects.  gfx950 wants two wait states between a VALU
+// write of an SGPR and a VALU read of it, and the compiler does not look into
+// asm: the forms take N >= 3 values at a time and do each step for all of them,
+// so that two other instructions lie between (volatile asm keeps its order).
+typedef u64 mask;  // a bit per lane, uniform
+
+__device__ __forceinline__ bool in_mask(mask m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+// r = a + b, a + b + k, a - b - k, ... and the carry (borrow) out
+#define GL_ADD_CO(r, k, a, b) \
+    asm volatile("v_add_co_u32 %0, %1, %2, %3" : "=v"(r), "=s"(k) : "v"(a), "v"(b))
+#define GL_ADDC_CO(r, ko, a, b, k) \
+    asm volatile("v_addc_co_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(ko) : "v"(a), "v"(b), "s"(k))
+#define GL_ADDC_0(r, ko, a, k) \
+    asm volatile("v_addc_co_u32 %0, %1, %2, 0, %3" : "=v"(r), "=s"(ko) : "v"(a), "s"(k))
+#define GL_SUB_CO(r, k, a, b) \
+    asm volatile("v_sub_co_u32 %0, %1, %2, %3" : "=v"(r), "=s"(k) : "v"(a), "v"(b))
+#define GL_SUBB_CO(r, ko, a, b, k) \
+    asm volatile("v_subb_co_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(ko) : "v"(a), "v"(b), "s"(k))
+#define GL_SUBB_0(r, ko, a, k) \
+    asm volatile("v_subb_co_u32 %0, %1, %2, 0, %3" : "=v"(r), "=s"(ko) : "v"(a), "s"(k))
+// bad |= k & ~c (k is overwritten); kept on the scalar unit
+#define GL_NOTE(bad, k, c) \
+    asm volatile("s_andn2_b64 %1, %1, %2\n\ts_or_b64 %0, %0, %1" : "+s"(bad), "+s"(k) : "s"(c) : "scc")
+// r = a * b + c (64 bits) and the carry out; the second form has b = 2^32 - 1
+#define GL_MAD_CO(r, k, a, b, c) \
+    asm volatile("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(k) : "v"(a), "v"(b), "v"(c))
+#define GL_MAD_EPS_CO(r, k, a, c) \
+    asm volatile("v_mad_u64_u32 %0, %1, %2, -1, %3" : "=v"(r), "=s"(k) : "v"(a), "v"(c))
+
+// l + (h1:h0) * 2^64 -> lazy u64, or bad
+template <int N>
+__device__ __forceinline__ void fold128_rare(u64 (&r)[N], const u64 (&l)[N], const u32 (&h0)[N],
+                                             const u32 (&h1)[N], mask& bad) {
+    static_assert(N >= 3, "wait states");
+    u64 u[N];
+    u32 r0[N], r1[N];
+    mask c[N], k[N], none;
+#pragma unroll
+    for (int i = 0; i < N; i++) GL_MAD_EPS_CO(u[i], c[i], h0[i], l[i]);
+#pragma unroll
+    for (int i = 0; i < N; i++) GL_SUBB_CO(r0[i], k[i], (u32)u[i], h1[i], c[i]);  // - h1 - c
+#pragma unroll
+    for (int i = 0; i < N; i++) GL_SUBB_0(r1[i], k[i], (u32)(u[i] >> 32), k[i]);
+#pragma unroll
+    for (int i = 0; i < N; i++) GL_ADDC_0(r1[i], none, r1[i], c[i]);              // + c * 2^32
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        GL_NOTE(bad, k[i], c[i]);
+        r[i] = mk64(r0[i], r1[i]);
+    }
+}
+
+// r = a * b, any u64 -> lazy u64, or bad
+template <int N>
+__device__ __forceinline__ void mul_rare(u64 (&r)[N], const u64 (&a)[N], const u64 (&b)[N],
+                                         mask& bad) {
+    static_assert(N >= 3, "wait states");
+    u64 p[N], q[N], y[N], l[N];
+    u32 l1[N], h0[N], h1[N];
+    mask cm[N], k[N], none;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const u64 x = (u64)(u32)(a[i] >> 32) * (u32)b[i];
+        GL_MAD_CO(y[i], cm[i], (u32)a[i], (u32)(b[i] >> 32), x);  // cross sum y + cm * 2^64
+        p[i] = (u64)(u32)a[i] * (u32)b[i];
+        q[i] = (u64)(u32)(a[i] >> 32) * (u32)(b[i] >> 32);
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) GL_ADD_CO(l1[i], k[i], (u32)(p[i] >> 32), (u32)y[i]);
+#pragma unroll
+    for (int i = 0; i < N; i++) GL_ADDC_CO(h0[i], k[i], (u32)q[i], (u32)(y[i] >> 32), k[i]);
+#pragma unroll
+    for (int i = 0; i < N; i++) GL_ADDC_0(h1[i], none, (u32)(q[i] >> 32), k[i]);
+#pragma unroll
+    for (int i = 0; i < N; i++) GL_ADDC_0(h1[i], none, h1[i], cm[i]);
+#pragma unroll
+    for (int i = 0; i < N; i++) l[i] = mk64((u32)p[i], l1[i]);
+    fold128_rare(r, l, h0, h1, bad);
+}
+
+// r = a * a, any u64 -> lazy u64, or bad
+template <int N>
+__device__ __forceinline__ void sqr_rare(u64 (&r)[N], const u64 (&a)[N], mask& bad) {
+    static_assert(N >= 3, "wait states");
+    u64 p[N], q[N], x[N], l[N];
+    u32 l1[N], h0[N], h1[N];
+    mask k[N], none;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const u32 a0 = (u32)a[i], a1 = (u32)(a[i] >> 32);
+        p[i] = (u64)a0 * a0;
+        x[i] = (u64)a0 * a1;
+        q[i] = (u64)a1 * a1;
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        u32 x2;  // (a plain add: half the cost of a shift)
+        asm("v_add_u32 %0, %1, %1" : "=v"(x2) : "v"((u32)x[i]));
+        GL_ADD_CO(l1[i], k[i], (u32)(p[i] >> 32), x2);
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const u32 x0 = (u32)x[i], x1 = (u32)(x[i] >> 32);
+        GL_ADDC_CO(h0[i], k[i], (u32)q[i], (u32)__builtin_amdgcn_alignbit(x1, x0, 31), k[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const u32 x1 = (u32)(x[i] >> 32);
+        GL_ADDC_CO(h1[i], none, (u32)(q[i] >> 32), x1 >> 31, k[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) l[i] = mk64((u32)p[i], l1[i]);
+    fold128_rare(r, l, h0, h1, bad);
+}
+
+// x * 2^64 (into Montgomery form), any u64 -> lazy u64, or bad (only when the
+// low word of x is 0 and the high one is not)
+template <int N>
+__device__ __forceinline__ void to_mont_rare(u64 (&r)[N], const u64 (&x)[N], mask& bad) {
+    static_assert(N >= 3, "wait states");
+    u64 t[N];
+    u32 r0[N], r1[N];
+    mask k[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) t[i] = (u64)(u32)x[i] * EPS;
+#pragma unroll
+    for (int i = 0; i < N; i++) GL_SUB_CO(r0[i], k[i], (u32)t[i], (u32)(x[i] >> 32));
+#pragma unroll
+    for (int i = 0; i < N; i++) GL_SUBB_0(r1[i], k[i], (u32)(t[i] >> 32), k[i]);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        asm volatile("s_or_b64 %0, %0, %1" : "+s"(bad) : "s"(k[i]) : "scc");
+        r[i] = mk64(r0[i], r1[i]);
+    }
+}
+
+// Constants of join_bytes that the compiler must not see through (it would
+// replace the multiply-adds by shifts and carries).
+struct JoinConsts {
+    u32 two16, eps;
+};
+__device__ __forceinline__ JoinConsts join_consts() {
+    JoinConsts c{65536u, 0xFFFFFFFFu};
+    asm volatile("" : "+s"(c.two16), "+s"(c.eps));
+    return c;
+}
+
+// Sum of d[t] * 256^t over eight byte places whose pair sums A = d[0] + 256 d[1],
+// B, C, D lie in [0, 2^31): A + B 2^16 + C 2^32 + D 2^48 -> u64 congruent to it.
+// With H = C + D 2^16 < 2^48 the value is (A + B 2^16) + H0 2^32 + H1 (2^32 - 1),
+// whose 64-bit sum carries only when H0 is within 2^17 of 2^32 (once in 2^15):
+// `carry` then says that 2^32 - 1 has to be added.  Three multiply-adds and one
+// add with carry after the four shift-adds.
+__device__ __forceinline__ u64 join_bytes_rare(const JoinConsts& J, u32 d0, u32 d1, u32 d2, u32 d3,
+                                               u32 d4, u32 d5, u32 d6, u32 d7, bool& carry) {
+    const u32 A = d0 + (d1 << 8), B = d2 + (d3 << 8), C = d4 + (d5 << 8), D = d6 + (d7 << 8);
+    const u64 L = (u64)B * J.two16 + A, H = (u64)D * J.two16 + C;
+    const u64 L2 = (u64)(u32)(H >> 32) * J.eps + L;
+    u32 k;
+    const u32 r1 = __builtin_addc((u32)(L2 >> 32), (u32)H, 0u, &k);
+    carry = k != 0;
+    return mk64((u32)L2, r1);
+}
 // 2^e mod p for 0 <= e < 192 (compile-time usable)
 __host__ __device__ constexpr u64 pow2_mod_p(int e) {
     u64 r = 1;

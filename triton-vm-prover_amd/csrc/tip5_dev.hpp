@@ -1,24 +1,38 @@
-// Tip5 permutation for one sponge per lane on gfx950.
+// Tip5 permutation of 16 sponges per wavefront on gfx950, with the MDS layer on
+// the matrix cores.
 //
 // Follows the reference permutation (src/hash/tip5.cpp:92-203): 5 rounds of
 // S-box -> circulant MDS -> round constants; S-box = split-and-lookup on lanes
-// 0..3 and x^7 on lanes 4..15.  The arithmetic is re-derived for VALU:
+// 0..3 and x^7 on lanes 4..15.  The arithmetic is re-derived for the GPU:
 //
-//  * the state is kept in Montgomery form x_M = x * 2^64 mod p (the form the
-//    reference's split-and-lookup is defined on): the reference forms the
-//    canonical Montgomery value montyred(v * R^2) = v * 2^64 mod p, looks up each
-//    byte and maps back with montyred(0, o) = o * 2^-64, so in Montgomery form
-//    the S-box is the byte lookup of the canonical value alone, and x^7 uses
-//    Montgomery products (montyred is cheaper than the 2^64 = 2^32 - 1 fold).
-//    Callers convert absorbed elements in (to_mont) and digests out
-//    (montyred(y, 0), canonical).  The 256-byte table sits in LDS.
-//  * MDS: the 16x16 circulant has 16-bit entries, so each state word is split
-//    into 32-bit halves and both halves are multiplied in f64 (exact: every
-//    partial sum is below 2^52), using the x^8 - 1 / x^8 + 1 split of the
-//    cyclic convolution.  The two 52-bit results are recombined modulo p with
-//    integer ops.
-//  * state words stay "lazy" (any u64 congruent mod p) inside the permutation;
+//  * Layout.  Lane 16g + n of a wave holds words g, 4 + g, 8 + g, 12 + g of
+//    sponge n (registers s[0..3]).  That is where v_mfma_i32_16x16x64_i8 takes
+//    its second operand from and leaves its result, so the state never moves
+//    between lanes; the four lookup words share register 0, so nothing diverges.
+//  * The state is kept in Montgomery form x_M = x * 2^64 mod p (the form the
+//    reference's split-and-lookup is defined on): the S-box of words 0..3 is the
+//    byte lookup of the canonical value alone.  x^7 takes plain products on the
+//    same values: (x 2^64)^7 = x^7 2^64 * 2^384, and 2^192 = 1 (mod p), so no
+//    Montgomery reduction occurs at all.  Callers convert absorbed elements in
+//    (to_m) and digests out (from_m, canonical).  The 256-byte table sits in LDS.
+//  * MDS.  The 16x16 circulant has 16-bit entries m = m0 + 256 m1 + 65536 m2
+//    with signed byte digits, the state words are 8 bytes, and 2^64 = 2^32 - 1,
+//    so every output word is a sum of eight byte places whose coefficients are
+//    fixed signed bytes: twelve 16x16x64 i8 products per round (the low words'
+//    bytes reach six of the places, the high words' six).  Bytes are made
+//    signed by flipping their top bits (x - kKappa in value); the constant that
+//    takes this back, the round constant and a bias that keeps every sum
+//    positive start the accumulators.  Sums stay below 2^31 (checked below).
+//  * Products and the final join leave their unlikely borrow or carry to one
+//    branch per round (gl64.hpp, *_rare).
+//  * State words stay "lazy" (any u64 congruent mod p) inside the permutation;
 //    callers canonicalise what they store.
+//
+// What bounds it: VALU issue.  The kernels issue a VALU instruction every 4
+// cycles per SIMD (2 for a few plain 32-bit ones); matrix instructions of one
+// wave run beside the VALU instructions of the others.  Rows of 2^22 x 379
+// (1.6e8 permutations): 19.7 ms, against 29.2 ms with one sponge per lane, the
+// MDS in f64 FMAs and Montgomery products.
 #pragma once
 
 #include "gl64.hpp"
@@ -33,186 +47,233 @@ constexpr int STATE = 16;
 constexpr int RATE = 10;
 constexpr int ROUNDS = 5;
 constexpr int DIGEST = 5;
+constexpr int WORDS = 4;        // state words per lane
+constexpr int GROUP = 16;       // sponges per wave
 
 // Round constants of the Tip5 specification: tip5_constants.hpp.
 using tip5c::kRoundConstants;
 
-struct RoundConstantsM {
-    u64 v[ROUNDS * STATE];
-};
-constexpr RoundConstantsM mont_round_constants() {
-    RoundConstantsM t{};
-    for (int i = 0; i < ROUNDS * STATE; i++)
-        t.v[i] = (u64)(((unsigned __int128)kRoundConstants[i] * gl::EPS) % gl::P);
-    return t;
-}
-// (the round constants in Montgomery form: c * 2^64 mod p, 2^64 = 2^32 - 1 mod p)
+typedef int v4i __attribute__((ext_vector_type(4)));
 
 // 1 in Montgomery form (2^64 mod p)
 constexpr u64 kOneM = gl::EPS;
 
-// First column of the circulant MDS matrix: tip5c::kMdsFirstColumn (SHA-256
-// of "Tip5" as 16 LE u16), folded into kMdsP / kMdsQ below.
+// ---- the MDS layer as byte products (first column: SHA-256 of "Tip5") --------
+constexpr int kProducts = 12;
+// product p adds to place kPlace[p]; the first six take the low words' bytes
+constexpr int kPlace[kProducts] = {0, 1, 2, 3, 4, 5, 0, 1, 4, 5, 6, 7};
+constexpr u64 kKappa = 0x8080808080808080ull;
+constexpr u32 kBias = 1u << 29;
 
-// Fill a 256-byte LDS table with the S-box ((x+1)^3 mod 257) - 1.
-__device__ __forceinline__ void load_lut(uint8_t* lut) {
+// signed byte digit d (0..2) of a 16-bit entry: digits 0 and 1 in [-128, 127]
+constexpr int mds_digit(int m, int d) {
+    int d0 = m & 255;
+    if (d0 > 127) d0 -= 256;
+    int r = (m - d0) >> 8, d1 = r & 255;
+    if (d1 > 127) d1 -= 256;
+    return d == 0 ? d0 : d == 1 ? d1 : (r - d1) >> 8;
+}
+// coefficient of byte b (0..7) of word j in byte place t of output word i:
+// 256^(b + d), with places 8 and 9 folded by 2^64 = 2^32 - 1
+constexpr int mds_coefficient(int i, int j, int b, int t) {
+    const int m = tip5c::kMdsFirstColumn[(i - j) & 15];
+    int c = 0;
+    for (int d = 0; d < 3; d++) {
+        const int pos = b + d;
+        if (pos == t) c += mds_digit(m, d);
+        if (pos >= 8 && pos - 4 == t) c += mds_digit(m, d);
+        if (pos >= 8 && pos - 8 == t) c -= mds_digit(m, d);
+    }
+    return c;
+}
+
+// First operands: lane 16g + r of product p holds row r's coefficients of the
+// bytes that lane group g feeds in (register v: word 4v + g).  Row r = 4g' + v'
+// is the output word 4v' + g', which lands in register v' of lane group g'.
+struct MdsOperands {
+    u32 w[kProducts * 64 * 4];
+};
+constexpr MdsOperands mds_operands() {
+    MdsOperands t{};
+    for (int p = 0; p < kProducts; p++)
+        for (int g = 0; g < 4; g++)
+            for (int r = 0; r < 16; r++)
+                for (int v = 0; v < 4; v++) {
+                    u32 x = 0;
+                    for (int b = 0; b < 4; b++)
+                        x |= (u32)(mds_coefficient(4 * (r & 3) + (r >> 2), 4 * v + g,
+                                                   b + (p < 6 ? 0 : 4), kPlace[p]) &
+                                   255)
+                             << (8 * b);
+                    t.w[(p * 64 + 16 * g + r) * 4 + v] = x;
+                }
+    return t;
+}
+__device__ const MdsOperands kMdsOperands = mds_operands();
+
+// Largest magnitude a place's sum can take, over signed bytes.
+constexpr int mds_bound(int t) {
+    int s = 0;
+    for (int j = 0; j < STATE; j++)
+        for (int b = 0; b < 8; b++) {
+            const int c = mds_coefficient(0, j, b, t);
+            s += 128 * (c < 0 ? -c : c);
+        }
+    return s;
+}
+constexpr bool mds_fits() {
+    for (int t = 0; t < 8; t += 2)
+        if ((u64)mds_bound(t) + 256ull * (u64)mds_bound(t + 1) + 65536 >= kBias) return false;
+    for (int j = 0; j < STATE; j++)
+        for (int b = 0; b < 8; b++)
+            for (int t = 0; t < 8; t++) {
+                const int c = mds_coefficient(0, j, b, t);
+                if (c < -128 || c > 127) return false;
+            }
+    return true;
+}
+static_assert(mds_fits(), "MDS byte sums leave their range");
+
+// Accumulator starts of the even byte places: bias + 16 bits of
+// (round constant in Montgomery form) + kKappa * (sum of the circulant) - biases.
+// start[round][place / 2][g][v] for word 4v + g.
+struct MdsStarts {
+    u32 w[ROUNDS * 4 * 16];
+};
+constexpr MdsStarts mds_starts() {
+    MdsStarts t{};
+    typedef unsigned __int128 u128;
+    u64 sum = 0;
+    for (int i = 0; i < STATE; i++) sum += tip5c::kMdsFirstColumn[i];
+    const u64 back = (u64)(((u128)kKappa * sum) % gl::P);
+    const u128 bias = (u128)kBias * (1 + (1ull << 16) + (1ull << 32) + (1ull << 48));
+    const u64 minus = gl::P - (u64)(bias % gl::P);
+    for (int r = 0; r < ROUNDS; r++)
+        for (int i = 0; i < STATE; i++) {
+            const u64 rc = (u64)(((u128)kRoundConstants[r * STATE + i] * gl::EPS) % gl::P);
+            const u64 c = (u64)(((u128)rc + back + minus) % gl::P);
+            for (int q = 0; q < 4; q++)
+                t.w[((r * 4 + q) * 4 + (i & 3)) * 4 + (i >> 2)] = kBias + (u32)((c >> (16 * q)) & 0xFFFF);
+        }
+    return t;
+}
+__device__ const MdsStarts kMdsStarts = mds_starts();
+
+// ---- LDS tables of a block -----------------------------------------------------
+struct alignas(16) Tables {
+    u32 start[ROUNDS * 4 * 16];
+    uint8_t lut[256];  // the S-box ((x+1)^3 mod 257) - 1
+};
+// Fills them (the caller synchronises the block before use).
+__device__ __forceinline__ void load_tables(Tables& T) {
+    for (u32 i = threadIdx.x; i < ROUNDS * 64; i += blockDim.x) T.start[i] = kMdsStarts.w[i];
     for (u32 x = threadIdx.x; x < 256; x += blockDim.x) {
         u32 t = x + 1;
-        lut[x] = (uint8_t)(((t * t % 257) * t % 257) - 1);
+        T.lut[x] = (uint8_t)(((t * t % 257) * t % 257) - 1);
     }
 }
 
-// S-box of lanes 0..3 on a Montgomery-form value: bytes of the canonical
-// Montgomery value through the table; the result is the Montgomery form of the
-// reference's output (tip5.cpp split_and_lookup).
-__device__ __forceinline__ u64 split_and_lookup_m(u64 v, const uint8_t* lut) {
-    u64 m = gl::canon(v);
+// The wave's constant operands, and where the lane sits.
+struct Wave {
+    v4i mds[kProducts];
+    gl::JoinConsts J;
+    const Tables* T;
+    u32 g, n;  // lane = 16 g + n
+};
+__device__ __forceinline__ Wave make_wave(const Tables& T) {
+    Wave W;
+    const u32 lane = threadIdx.x & 63;
+    W.J = gl::join_consts();
+    W.T = &T;
+    W.g = lane >> 4;
+    W.n = lane & 15;
+#pragma unroll
+    for (int p = 0; p < kProducts; p++)
+        W.mds[p] = *(const v4i*)(kMdsOperands.w + (p * 64 + lane) * 4);
+    return W;
+}
+
+// ---- S-box ----------------------------------------------------------------------
+// x^7, exact (the products' unlikely case)
+__device__ __forceinline__ u64 pow7(u64 x) {
+    const u64 x2 = gl::mul_lazy(x, x), x4 = gl::mul_lazy(x2, x2);
+    return gl::mul_lazy(gl::mul_lazy(x, x2), x4);
+}
+template <int N>
+__device__ __forceinline__ void pow7_rare(u64 (&y)[N], const u64 (&x)[N], gl::mask& bad) {
+    u64 x2[N], x3[N], x4[N];
+    gl::sqr_rare(x2, x, bad);
+    gl::mul_rare(x3, x, x2, bad);
+    gl::sqr_rare(x4, x2, bad);
+    gl::mul_rare(y, x3, x4, bad);
+}
+
+// S-box of words 0..3 on a Montgomery-form value: bytes of the canonical value
+// through the table; the result is the Montgomery form of the reference's
+// output (tip5.cpp split_and_lookup).
+__device__ __forceinline__ u64 split_and_lookup(u64 m, const uint8_t* lut) {
     u32 lo = (u32)m, hi = (u32)(m >> 32);
-    u32 olo = (u32)lut[lo & 0xff] | ((u32)lut[(lo >> 8) & 0xff] << 8) |
-              ((u32)lut[(lo >> 16) & 0xff] << 16) | ((u32)lut[lo >> 24] << 24);
-    u32 ohi = (u32)lut[hi & 0xff] | ((u32)lut[(hi >> 8) & 0xff] << 8) |
-              ((u32)lut[(hi >> 16) & 0xff] << 16) | ((u32)lut[hi >> 24] << 24);
+    // p <= m < 2^64 only with a high word of ones and a nonzero low word
+    if (__builtin_expect(hi == 0xFFFFFFFFu, 0)) {
+        if (lo) {
+            lo -= 1;
+            hi = 0;
+        }
+    }
+    const u32 olo = (u32)lut[lo & 0xff] | ((u32)lut[(lo >> 8) & 0xff] << 8) |
+                    ((u32)lut[(lo >> 16) & 0xff] << 16) | ((u32)lut[lo >> 24] << 24);
+    const u32 ohi = (u32)lut[hi & 0xff] | ((u32)lut[(hi >> 8) & 0xff] << 8) |
+                    ((u32)lut[(hi >> 16) & 0xff] << 16) | ((u32)lut[hi >> 24] << 24);
     return ((u64)ohi << 32) | olo;
 }
 
-__device__ __forceinline__ u64 pow7_m(u64 x) {
-    u64 x2 = gl::mont_sqr(x);
-    u64 x4 = gl::mont_sqr(x2);
-    u64 x3 = gl::mont_mul(x, x2);
-    return gl::mont_mul(x3, x4);
-}
-
-// integer-valued double a >= 0 and bias = 2^52 + c with a + c < 2^52 -> a + c
-__device__ __forceinline__ u64 f2u52(double a, double bias) {
-    return (u64)__double_as_longlong(a + bias) & 0x000FFFFFFFFFFFFFull;
-}
-
-// Round constants as f64 biases for the MDS recombination: adding the 32-bit
-// halves c0, c1 of the Montgomery-form constant to the exact MDS outputs
-// (L + c0) + (H + c1) * 2^32 adds the constant itself; 2^52 + c is exact in f64
-// and L + c0, H + c1 stay below 2^52.
-struct RcBias {
-    double v[ROUNDS * STATE * 2];
-};
-constexpr RcBias rc_bias_table() {
-    RcBias t{};
-    const RoundConstantsM m = mont_round_constants();
-    for (int i = 0; i < ROUNDS * STATE; i++) {
-        u64 c = m.v[i];
-        t.v[2 * i] = 4503599627370496.0 + (double)(u32)c;
-        t.v[2 * i + 1] = 4503599627370496.0 + (double)(u32)(c >> 32);
-    }
-    return t;
-}
-__constant__ RcBias kRcBias = rc_bias_table();
-
-// Circulant MDS y_r = sum_c M[(r - c) & 15] s_c on the two 32-bit halves of the
-// state, each via x^16 - 1 = (x^8 - 1)(x^8 + 1): a cyclic 8-term product of
-// (s_lo + s_hi) with kMdsP = (m_lo + m_hi)/2 and a negacyclic one of
-// (s_lo - s_hi) with kMdsQ = (m_lo - m_hi)/2 give A and B with y_lo = A + B,
-// y_hi = A - B.  Every partial sum is a multiple of 1/2 below 2^52 in
-// magnitude, so all f64 arithmetic is exact (128 FMAs per half instead of 256).
-struct MdsHalves {
-    double v[8];
-};
-constexpr MdsHalves mds_halves(int sign) {
-    MdsHalves t{};
-    for (int i = 0; i < 8; i++)
-        t.v[i] = ((double)tip5c::kMdsFirstColumn[i] + sign * (double)tip5c::kMdsFirstColumn[i + 8]) / 2.0;
-    return t;
-}
-constexpr MdsHalves kMdsP = mds_halves(1);
-constexpr MdsHalves kMdsQ = mds_halves(-1);
-
-__device__ __forceinline__ void mds_half(const double x[STATE], double y[STATE]) {
-    double sp[8], sm[8];
+// ---- one round, the permutation --------------------------------------------------
+// Round r (tip5.cpp:115-125: S-box layer, MDS, round constants) on the wave's
+// Montgomery-form states (any u64 words congruent to x_M).  All 64 lanes take
+// part; lanes of unused sponges carry any values.
+__device__ __forceinline__ void round_m(u64 s[WORDS], int r, const Wave& W) {
+    const u64 x[3] = {s[1], s[2], s[3]};
+    u64 y7[3];
+    gl::mask bad = 0;
+    pow7_rare(y7, x, bad);
+    s[0] = split_and_lookup(s[0], W.T->lut);
+    if (__builtin_expect(gl::in_mask(bad), 0)) {
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-        sp[c] = x[c] + x[c + 8];
-        sm[c] = x[c] - x[c + 8];
+        for (int i = 0; i < 3; i++) y7[i] = pow7(x[i]);
     }
 #pragma unroll
-    for (int r = 0; r < 8; r++) {
-        double A = 0.0, B = 0.0;
+    for (int i = 0; i < 3; i++) s[1 + i] = y7[i];
+    v4i lo, hi;
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
-            A = __fma_rn(kMdsP.v[(r - c) & 7], sp[c], A);
-            B = __fma_rn(r >= c ? kMdsQ.v[r - c] : -kMdsQ.v[r - c + 8], sm[c], B);
-        }
-        y[r] = A + B;
-        y[r + 8] = A - B;
+    for (int v = 0; v < WORDS; v++) {
+        lo[v] = (int)((u32)s[v] ^ (u32)kKappa);
+        hi[v] = (int)((u32)(s[v] >> 32) ^ (u32)kKappa);
+    }
+    const v4i* start = (const v4i*)(W.T->start + r * 64) + W.g;
+    v4i y[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) y[t] = t & 1 ? v4i{0, 0, 0, 0} : start[2 * t];
+#pragma unroll
+    for (int p = 0; p < kProducts; p++)
+        y[kPlace[p]] = __builtin_amdgcn_mfma_i32_16x16x64_i8(W.mds[p], p < 6 ? lo : hi,
+                                                             y[kPlace[p]], 0, 0, 0);
+    bool carry[WORDS];
+#pragma unroll
+    for (int v = 0; v < WORDS; v++)
+        s[v] = gl::join_bytes_rare(W.J, (u32)y[0][v], (u32)y[1][v], (u32)y[2][v], (u32)y[3][v],
+                                   (u32)y[4][v], (u32)y[5][v], (u32)y[6][v], (u32)y[7][v],
+                                   carry[v]);
+    if (__builtin_expect(carry[0] | carry[1] | carry[2] | carry[3], 0)) {
+#pragma unroll
+        for (int v = 0; v < WORDS; v++)
+            if (carry[v]) s[v] += gl::EPS;
     }
 }
 
-// MDS followed by the round constants of round `round` (any u64 in, < 2^64 out).
-__device__ __forceinline__ void mds_rc(u64 s[STATE], int round) {
-    double lo[STATE], hi[STATE], ylo[STATE], yhi[STATE];
-#pragma unroll
-    for (int c = 0; c < STATE; c++) {
-        lo[c] = (double)(u32)s[c];
-        hi[c] = (double)(u32)(s[c] >> 32);
-    }
-    mds_half(lo, ylo);
-    mds_half(hi, yhi);
-    const double* bias = kRcBias.v + round * STATE * 2;
-#pragma unroll
-    for (int r = 0; r < STATE; r++) {  // (L + c0) + (H + c1) * 2^32
-        s[r] = gl::lin52(f2u52(ylo[r], bias[2 * r]), f2u52(yhi[r], bias[2 * r + 1]));
-    }
-}
-
-// Round r of the permutation (tip5.cpp:115-125: S-box layer, MDS, round
-// constants) on a Montgomery-form state (any u64 words congruent to x_M).
-__device__ __forceinline__ void round_m(u64 s[STATE], int r, const uint8_t* lut) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) s[i] = split_and_lookup_m(s[i], lut);
-#pragma unroll
-    for (int i = 4; i < STATE; i++) s[i] = pow7_m(s[i]);
-    mds_rc(s, r);
-}
-
-// The permutation on a Montgomery-form state.
-__device__ __forceinline__ void permutation_m(u64 s[STATE], const uint8_t* lut) {
+// The permutation on the wave's Montgomery-form states.
+__device__ __forceinline__ void permutation_m(u64 s[WORDS], const Wave& W) {
 #pragma unroll 1
-    for (int r = 0; r < ROUNDS; r++) round_m(s, r, lut);
-}
-
-// The permutation spread over a group of 16 lanes (16-aligned within the wave),
-// for latency-bound work such as the top levels of a Merkle tree: lane w of the
-// group holds state word w (Montgomery form).  The S-box acts lane-wise; the
-// circulant MDS y_w = sum_c M[(w - c) & 15] s_c gathers the group's words with
-// lane shuffles and sums each 32-bit half in f64, exact because sum_c M_c <
-// 2^20 keeps both sums below 2^52.  Every lane of the group must take part.
-struct MdsColumnF64 {
-    double v[STATE];
-};
-constexpr MdsColumnF64 mds_column_f64() {
-    MdsColumnF64 t{};
-    for (int i = 0; i < STATE; i++) t.v[i] = (double)tip5c::kMdsFirstColumn[i];
-    return t;
-}
-__constant__ MdsColumnF64 kMdsColumnF64 = mds_column_f64();
-
-__device__ __forceinline__ u64 permutation_group16(u64 s, u32 w, const uint8_t* lut) {
-    double m[STATE];
-#pragma unroll
-    for (int c = 0; c < STATE; c++) m[c] = kMdsColumnF64.v[(w - (u32)c) & 15];
-#pragma unroll 1
-    for (int r = 0; r < ROUNDS; r++) {
-        s = w < 4 ? split_and_lookup_m(s, lut) : pow7_m(s);
-        const u32 lo = (u32)s, hi = (u32)(s >> 32);
-        double l0 = 0.0, l1 = 0.0, h0 = 0.0, h1 = 0.0;  // two chains per half
-#pragma unroll
-        for (int c = 0; c < STATE; c += 2) {
-            l0 = __fma_rn(m[c], (double)__shfl(lo, c, 16), l0);
-            h0 = __fma_rn(m[c], (double)__shfl(hi, c, 16), h0);
-            l1 = __fma_rn(m[c + 1], (double)__shfl(lo, c + 1, 16), l1);
-            h1 = __fma_rn(m[c + 1], (double)__shfl(hi, c + 1, 16), h1);
-        }
-        const double* bias = kRcBias.v + (r * STATE + w) * 2;
-        s = gl::lin52(f2u52(l0 + l1, bias[0]), f2u52(h0 + h1, bias[1]));
-    }
-    return s;
+    for (int r = 0; r < ROUNDS; r++) round_m(s, r, W);
 }
 
 // Montgomery form <-> canonical

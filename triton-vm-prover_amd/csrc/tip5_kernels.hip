@@ -1,19 +1,20 @@
 // Tip5 hashing kernels: row digests, pair hashing, Merkle trees, auth paths.
 //
-// Row hashing restates Tip5::hash_varlen (src/hash/tip5.cpp:246-282) for one
-// row per lane over a column-major table (element (r, c) at c*rows + r, the
-// reference GPU layout, include/gpu/kernels/row_hash_kernel.cuh:18-33): zero
-// state, overwrite absorb of 10 elements per permutation, last block padded
-// [rest, 1, 0...].  Reads of one column by a wavefront are 64 consecutive
-// u64, so HBM traffic is coalesced without staging.
+// Every kernel runs 16 sponges per wave (tip5_dev.hpp): lane 16g + n holds
+// words 4v + g (v = 0..3) of sponge n.  State words 0..9 are the rate.
+//
+// Row hashing restates Tip5::hash_varlen (src/hash/tip5.cpp:246-282) over a
+// column-major table (element (r, c) at c*rows + r, the reference GPU layout,
+// include/gpu/kernels/row_hash_kernel.cuh:18-33): zero state, overwrite absorb
+// of 10 elements per permutation, last block padded [rest, 1, 0...].  A wave
+// reads 16 consecutive u64 (one 128-byte line) of four columns at a time.
 //
 // Merkle trees follow merkle_tree.cpp:41-61 (parent = hash_pair(left,right)).
 // Node (level l, index i) of an n-leaf tree lives at base(l) + i with
 //   level order (merkle_kernel.cu:60-102): base(l) = 2n - (2n >> l)
 //   heap        (merkle_tree.cpp:12-33):   base(l) = n >> l      (1-indexed)
-// Levels of more than 2^16 parents take a launch each, one hash per thread.
-// Above them a block hashes up to 16 parents on 16 lanes each, keeps them in
-// LDS and continues to their subtree root (up to 5 levels per launch).
+// Large levels take a launch each; below them a block hashes up to 256 parents,
+// keeps them in LDS and continues to their subtree root.
 #include "tvh_internal.hpp"
 
 namespace tvh {
@@ -21,10 +22,12 @@ namespace tvh {
 using gl::u32;
 using gl::u64;
 
-// Sponge states are kept in Montgomery form (tip5_dev.hpp); digests leave canonical.
-__device__ __forceinline__ void store_digest(u64* dst, const u64 s[tip5::STATE]) {
-#pragma unroll
-    for (int i = 0; i < tip5::DIGEST; i++) dst[i] = tip5::from_m(s[i]);
+// Sponge states are kept in Montgomery form (tip5_dev.hpp); digests leave
+// canonical.  Word 4v + g < 5 of the lane's sponge goes to dst[4v + g].
+__device__ __forceinline__ void store_digest(u64* dst, const u64 s[tip5::WORDS],
+                                             const tip5::Wave& W) {
+    dst[W.g] = tip5::from_m(s[0]);
+    if (W.g == 0) dst[4] = tip5::from_m(s[1]);
 }
 
 // Segment lookup for multi-table launches (start[nseg] = total blocks).
@@ -38,50 +41,75 @@ __device__ __forceinline__ u32 find_seg(const u32* __restrict__ start, u32 nseg,
     return lo;
 }
 
+// First sponge of the wave: block blk of kSpongesPerBlock sponges.
+__device__ __forceinline__ u64 wave_first(u64 blk) {
+    return blk * kSpongesPerBlock + (threadIdx.x >> 6) * tip5::GROUP;
+}
+
+// Absorbs one full rate block: elem(i) is element i (0..9), canonical.
+template <class F>
+__device__ __forceinline__ void absorb(u64 s[tip5::WORDS], const tip5::Wave& W, const F& elem) {
+    const u64 x[3] = {elem(W.g), elem(4 + W.g), W.g < 2 ? elem(8 + W.g) : 0};
+    u64 m[3];
+    gl::mask bad = 0;
+    gl::to_mont_rare(m, x, bad);
+    if (__builtin_expect(gl::in_mask(bad), 0)) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) m[i] = tip5::to_m(x[i]);
+    }
+    s[0] = m[0];
+    s[1] = m[1];
+    s[2] = W.g < 2 ? m[2] : s[2];
+}
+
+// Absorbs the padding block [rest elements, 1, 0...], rest < 10.
+template <class F>
+__device__ __forceinline__ void absorb_last(u64 s[tip5::WORDS], const tip5::Wave& W, u32 rest,
+                                            const F& elem) {
+#pragma unroll
+    for (int v = 0; v < 3; v++) {
+        const u32 i = 4 * v + W.g;
+        if (i < (u32)tip5::RATE)
+            s[v] = i < rest ? tip5::to_m(elem(i)) : (i == rest ? tip5::kOneM : 0ull);
+    }
+}
+
 // rows x cols column-major table -> rows digests (5 u64 each, row-major).
-__device__ __forceinline__ void hash_rows_body(const HashArgs& A, u64 blk, const uint8_t* lut) {
-    u64 row = blk * 256 + threadIdx.x;
-    if (row >= A.rows) return;
+__device__ __forceinline__ void hash_rows_body(const HashArgs& A, u64 blk, const tip5::Wave& W) {
+    const u64 row = wave_first(blk) + W.n;
     const u64 rows = A.rows;
     const u32 cols = A.cols;
-    u64 s[tip5::STATE];
-#pragma unroll
-    for (int i = 0; i < tip5::STATE; i++) s[i] = 0;
-    const u64* p = A.tab + row;
+    // lanes past the last row hash it again (they take part in the matrix products)
+    const u64* p = A.tab + (row < rows ? row : rows - 1);
+    u64 s[tip5::WORDS] = {0, 0, 0, 0};
     u32 used = 0;
     for (; used + tip5::RATE <= cols; used += tip5::RATE) {
-#pragma unroll
-        for (int i = 0; i < tip5::RATE; i++)
-            s[i] = tip5::to_m(__builtin_nontemporal_load(p + (u64)(used + i) * rows));
-        tip5::permutation_m(s, lut);
+        absorb(s, W, [&](u32 i) { return __builtin_nontemporal_load(p + (u64)(used + i) * rows); });
+        tip5::permutation_m(s, W);
     }
-    u32 rest = cols - used;
-#pragma unroll
-    for (int i = 0; i < tip5::RATE; i++) {
-        u32 ui = (u32)i;
-        s[i] = ui < rest ? tip5::to_m(__builtin_nontemporal_load(p + (u64)(used + ui) * rows))
-                         : (ui == rest ? tip5::kOneM : 0ull);
-    }
-    tip5::permutation_m(s, lut);
-    store_digest(A.dig + row * tip5::DIGEST, s);
+    absorb_last(s, W, cols - used,
+                [&](u32 i) { return __builtin_nontemporal_load(p + (u64)(used + i) * rows); });
+    tip5::permutation_m(s, W);
+    if (row < rows) store_digest(A.dig + row * tip5::DIGEST, s, W);
 }
 
-// At least 4 waves per SIMD (<= 128 VGPRs; 4 to 6 waves time the same).
-__global__ void __launch_bounds__(256, 4) k_hash_rows(HashArgs A) {
-    __shared__ uint8_t lut[256];
-    tip5::load_lut(lut);
+__global__ void __launch_bounds__(kHashThreads, 4) k_hash_rows(HashArgs A) {
+    __shared__ tip5::Tables T;
+    tip5::load_tables(T);
+    const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    hash_rows_body(A, blockIdx.x, lut);
+    hash_rows_body(A, blockIdx.x, W);
 }
 
-__global__ void __launch_bounds__(256, 4) k_hash_rows_multi(const HashArgs* __restrict__ args,
-                                                         const u32* __restrict__ start, u32 nseg) {
-    __shared__ uint8_t lut[256];
-    tip5::load_lut(lut);
+__global__ void __launch_bounds__(kHashThreads, 4) k_hash_rows_multi(
+    const HashArgs* __restrict__ args, const u32* __restrict__ start, u32 nseg) {
+    __shared__ tip5::Tables T;
+    tip5::load_tables(T);
+    const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
     u32 seg = find_seg(start, nseg, blockIdx.x);
     HashArgs A = args[seg];
-    hash_rows_body(A, blockIdx.x - start[seg], lut);
+    hash_rows_body(A, blockIdx.x - start[seg], W);
 }
 
 // Column-chunk absorption for the streaming ("frugal") commit: each row's
@@ -94,216 +122,180 @@ __global__ void __launch_bounds__(256, 4) k_hash_rows_multi(const HashArgs* __re
 // [rest, 1, 0...] and writes the canonical digest (tip5.cpp:246-282).  The
 // carried state is in Montgomery form, the carried elements are canonical.
 template <bool FINAL>
-__global__ void __launch_bounds__(256) k_absorb_chunk(const u64* __restrict__ chunk, u64 rows,
-                                                      u32 ccols, u64* __restrict__ state,
-                                                      u64* __restrict__ pend, u32 npend,
-                                                      int first, u64* __restrict__ dig) {
-    __shared__ uint8_t lut[256];
-    tip5::load_lut(lut);
+__global__ void __launch_bounds__(kHashThreads, 4)
+    k_absorb_chunk(const u64* __restrict__ chunk, u64 rows, u32 ccols, u64* __restrict__ state,
+                   u64* __restrict__ pend, u32 npend, int first, u64* __restrict__ dig) {
+    __shared__ tip5::Tables T;
+    tip5::load_tables(T);
+    const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    u64 row = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= rows) return;
-    u64 s[tip5::STATE];
+    const u64 row = wave_first(blockIdx.x) + W.n;
+    const u64 r = row < rows ? row : rows - 1;  // lanes past the end repeat the last row
+    u64 s[tip5::WORDS];
 #pragma unroll
-    for (int i = 0; i < tip5::STATE; i++) s[i] = first ? 0ull : state[(u64)i * rows + row];
+    for (int v = 0; v < tip5::WORDS; v++) s[v] = first ? 0ull : state[(u64)(4 * v + W.g) * rows + r];
     auto elem = [&](u32 j) -> u64 {
-        return j < npend ? pend[(u64)j * rows + row] : chunk[(u64)(j - npend) * rows + row];
+        return j < npend ? pend[(u64)j * rows + r] : chunk[(u64)(j - npend) * rows + r];
     };
     const u32 total = npend + ccols;
     u32 used = 0;
     for (; used + tip5::RATE <= total; used += tip5::RATE) {
-#pragma unroll
-        for (int i = 0; i < tip5::RATE; i++) s[i] = tip5::to_m(elem(used + i));
-        tip5::permutation_m(s, lut);
+        absorb(s, W, [&](u32 i) { return elem(used + i); });
+        tip5::permutation_m(s, W);
     }
     const u32 rest = total - used;
     if (FINAL) {
+        absorb_last(s, W, rest, [&](u32 i) { return elem(used + i); });
+        tip5::permutation_m(s, W);
+        if (row < rows) store_digest(dig + row * tip5::DIGEST, s, W);
+    } else if (row < rows) {
+        // carried elements: position i is read and written by the same lane
 #pragma unroll
-        for (int i = 0; i < tip5::RATE; i++) {
-            u32 ui = (u32)i;
-            s[i] = ui < rest ? tip5::to_m(elem(used + ui)) : (ui == rest ? tip5::kOneM : 0ull);
+        for (int v = 0; v < 3; v++) {
+            const u32 i = 4 * v + W.g;
+            if (i < rest) pend[(u64)i * rows + row] = elem(used + i);
         }
-        tip5::permutation_m(s, lut);
-        store_digest(dig + row * tip5::DIGEST, s);
-    } else {
-        // carried elements first (they may be read from pend itself: read all, then write)
-        u64 carry[tip5::RATE];
 #pragma unroll
-        for (int i = 0; i < tip5::RATE; i++) carry[i] = (u32)i < rest ? elem(used + i) : 0ull;
-#pragma unroll
-        for (int i = 0; i < tip5::RATE; i++)
-            if ((u32)i < rest) pend[(u64)i * rows + row] = carry[i];
-#pragma unroll
-        for (int i = 0; i < tip5::STATE; i++) state[(u64)i * rows + row] = s[i];
+        for (int v = 0; v < tip5::WORDS; v++) state[(u64)(4 * v + W.g) * rows + row] = s[v];
     }
 }
 
 // Tip5 permutation of num states (16 u64 each, in place); outputs canonical.
-__global__ void __launch_bounds__(256) k_permutation(u64* __restrict__ st, u64 num) {
-    __shared__ uint8_t lut[256];
-    tip5::load_lut(lut);
+__global__ void __launch_bounds__(kHashThreads, 4) k_permutation(u64* __restrict__ st, u64 num) {
+    __shared__ tip5::Tables T;
+    tip5::load_tables(T);
+    const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    const u64 i = wave_first(blockIdx.x) + W.n;
+    const u64* in = st + (i < num ? i : num - 1) * tip5::STATE + W.g;
+    u64 s[tip5::WORDS];
+#pragma unroll
+    for (int v = 0; v < tip5::WORDS; v++) s[v] = tip5::to_m(in[4 * v]);
+    tip5::permutation_m(s, W);
     if (i >= num) return;
-    u64 s[tip5::STATE];
 #pragma unroll
-    for (int k = 0; k < tip5::STATE; k++) s[k] = tip5::to_m(st[i * tip5::STATE + k]);
-    tip5::permutation_m(s, lut);
-#pragma unroll
-    for (int k = 0; k < tip5::STATE; k++) st[i * tip5::STATE + k] = tip5::from_m(s[k]);
+    for (int v = 0; v < tip5::WORDS; v++) st[i * tip5::STATE + W.g + 4 * v] = tip5::from_m(s[v]);
 }
 
 // Rounds [first, first + count) of the permutation on num states (in place).
 // trace (may be null) receives, per state, the input and the state after each
 // of those rounds: trace[(i * (count + 1) + j) * 16 + k].  Outputs canonical.
-__global__ void __launch_bounds__(256) k_permutation_rounds(u64* __restrict__ st, u64 num,
-                                                            u32 first, u32 count,
-                                                            u64* __restrict__ trace) {
-    __shared__ uint8_t lut[256];
-    tip5::load_lut(lut);
+__global__ void __launch_bounds__(kHashThreads) k_permutation_rounds(u64* __restrict__ st, u64 num,
+                                                                     u32 first, u32 count,
+                                                                     u64* __restrict__ trace) {
+    __shared__ tip5::Tables T;
+    tip5::load_tables(T);
+    const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= num) return;
-    u64 s[tip5::STATE];
+    const u64 i = wave_first(blockIdx.x) + W.n;
+    const bool live = i < num;
+    const u64* in = st + (live ? i : num - 1) * tip5::STATE + W.g;
+    u64* tr = trace && live ? trace + i * (count + 1) * tip5::STATE + W.g : nullptr;
+    u64 s[tip5::WORDS];
 #pragma unroll
-    for (int k = 0; k < tip5::STATE; k++) s[k] = tip5::to_m(st[i * tip5::STATE + k]);
-    u64* tr = trace ? trace + i * (count + 1) * tip5::STATE : nullptr;
-    if (tr) {
-#pragma unroll
-        for (int k = 0; k < tip5::STATE; k++) tr[k] = st[i * tip5::STATE + k];
+    for (int v = 0; v < tip5::WORDS; v++) {
+        const u64 x = in[4 * v];
+        if (tr) tr[4 * v] = x;
+        s[v] = tip5::to_m(x);
     }
     for (u32 r = 0; r < count; r++) {
-        tip5::round_m(s, (int)(first + r), lut);
+        tip5::round_m(s, (int)(first + r), W);
         if (tr) {
 #pragma unroll
-            for (int k = 0; k < tip5::STATE; k++) tr[(r + 1) * tip5::STATE + k] = tip5::from_m(s[k]);
+            for (int v = 0; v < tip5::WORDS; v++)
+                tr[(r + 1) * tip5::STATE + 4 * v] = tip5::from_m(s[v]);
         }
     }
+    if (!live) return;
 #pragma unroll
-    for (int k = 0; k < tip5::STATE; k++) st[i * tip5::STATE + k] = tip5::from_m(s[k]);
+    for (int v = 0; v < tip5::WORDS; v++) st[i * tip5::STATE + W.g + 4 * v] = tip5::from_m(s[v]);
 }
 
-__device__ __forceinline__ void hash_pair(const u64* l, const u64* r, u64 s[tip5::STATE],
-                                          const uint8_t* lut) {
-#pragma unroll
-    for (int k = 0; k < 5; k++) {
-        s[k] = tip5::to_m(l[k]);
-        s[5 + k] = tip5::to_m(r[k]);
-    }
-#pragma unroll
-    for (int k = 10; k < tip5::STATE; k++) s[k] = tip5::kOneM;
-    tip5::permutation_m(s, lut);
+// hash_pair: the two digests are words 0..9 (elem), the capacity is ones.
+template <class F>
+__device__ __forceinline__ void hash_pair(u64 s[tip5::WORDS], const tip5::Wave& W, const F& elem) {
+    s[2] = s[3] = tip5::kOneM;
+    absorb(s, W, elem);
+    tip5::permutation_m(s, W);
 }
 
 // out[i] = hash_pair(left[i], right[i])  (Backend::hash_pairs, backend.hpp:110-115)
-__global__ void __launch_bounds__(256) k_hash_pairs(const u64* __restrict__ left,
-                                                    const u64* __restrict__ right,
-                                                    u64* __restrict__ out, u64 count) {
-    __shared__ uint8_t lut[256];
-    tip5::load_lut(lut);
+__global__ void __launch_bounds__(kHashThreads, 4) k_hash_pairs(const u64* __restrict__ left,
+                                                                const u64* __restrict__ right,
+                                                                u64* __restrict__ out, u64 count) {
+    __shared__ tip5::Tables T;
+    tip5::load_tables(T);
+    const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    u64 s[tip5::STATE];
-    hash_pair(left + 5 * i, right + 5 * i, s, lut);
-    store_digest(out + 5 * i, s);
+    const u64 i = wave_first(blockIdx.x) + W.n;
+    const u64 r = i < count ? i : count - 1;
+    u64 s[tip5::WORDS];
+    hash_pair(s, W, [&](u32 k) { return k < 5 ? left[5 * r + k] : right[5 * r + k - 5]; });
+    if (i < count) store_digest(out + 5 * i, s, W);
 }
 
 // One launch of the Merkle build: children are the nodes of one level; each
-// block hashes 2T children into T parents (T active threads, T <= blockDim)
-// and continues for `levels` levels inside LDS.  Level j (1-based) parents go
-// to dst[j-1] + index.
-__device__ __forceinline__ void merkle_body(const MerkleArgs& A, u64 blk, const uint8_t* lut,
+// block hashes 2T children into T parents (16 per wave, T <= 16 waves) and
+// continues for `levels` levels inside LDS.  Level j (1-based) parents go to
+// dst[j-1] + index.
+__device__ __forceinline__ void merkle_body(const MerkleArgs& A, u64 blk, const tip5::Wave& W,
                                             u64* buf) {
-    const u32 T = A.T;
-    const u32 t = threadIdx.x;
-    u64 s[tip5::STATE];
-    if (t < T) {
-        u64 parent = blk * T + t;
-        hash_pair(A.src + 10 * parent, A.src + 10 * parent + 5, s, lut);
-        u64 d[5];
-#pragma unroll
-        for (int k = 0; k < 5; k++) d[k] = tip5::from_m(s[k]);
-#pragma unroll
-        for (int k = 0; k < 5; k++) {
-            A.dst[0][5 * parent + k] = d[k];
-            buf[5 * t + k] = d[k];
-        }
+    const u32 first = (threadIdx.x >> 6) * tip5::GROUP;  // the wave's first parent
+    const u32 t = first + W.n;
+    u32 width = A.T;
+    u64 s[tip5::WORDS];
+    if (first < width) {  // (whole waves)
+        const u64* c = A.src + 10 * (blk * width + (t < width ? t : 0));
+        hash_pair(s, W, [&](u32 k) { return c[k]; });
     }
-    u32 width = T;
-    for (u32 j = 1; j < A.levels; j++) {
-        __syncthreads();
-        width >>= 1;
-        u64 d[5];
+    for (u32 j = 0;; j++) {
+        const bool last = j + 1 == A.levels;
         if (t < width) {
-            hash_pair(buf + 10 * t, buf + 10 * t + 5, s, lut);
-#pragma unroll
-            for (int k = 0; k < 5; k++) d[k] = tip5::from_m(s[k]);
-        }
-        __syncthreads();
-        if (t < width) {
-            u64 parent = blk * width + t;
-#pragma unroll
-            for (int k = 0; k < 5; k++) {
-                A.dst[j][5 * parent + k] = d[k];
-                buf[5 * t + k] = d[k];
+            u64* d = A.dst[j] + 5 * (blk * width + t);
+            const u64 x = tip5::from_m(s[0]);
+            d[W.g] = x;
+            if (!last) buf[5 * t + W.g] = x;
+            if (W.g == 0) {
+                const u64 z = tip5::from_m(s[1]);
+                d[4] = z;
+                if (!last) buf[5 * t + 4] = z;
             }
         }
-    }
-}
-
-// The same levels with each hash on a group of 16 lanes (tip5::permutation_group16):
-// a 256-thread block holds 16 groups, hashes T <= 16 parents of its first level
-// and continues in LDS to their subtree root.  Group g, lane w: state word w of
-// parent g is child word w (the two children are adjacent: words 0..9), then
-// capacity ones.
-__device__ __forceinline__ void merkle_body_group16(const MerkleArgs& A, u64 blk,
-                                                    const uint8_t* lut, u64* buf) {
-    const u32 g = threadIdx.x >> 4, w = threadIdx.x & 15;
-    u32 width = A.T;
-    u64 s = tip5::kOneM;
-    if (g < width && w < 10) s = tip5::to_m(A.src[10 * (blk * width + g) + w]);
-    s = tip5::permutation_group16(s, w, lut);
-    if (g < width && w < tip5::DIGEST) {
-        const u64 d = tip5::from_m(s);
-        A.dst[0][5 * (blk * width + g) + w] = d;
-        buf[5 * g + w] = d;
-    }
-    for (u32 j = 1; j < A.levels; j++) {
-        __syncthreads();  // the previous level's digests are in buf
+        if (last) break;
+        __syncthreads();  // this level's digests are in buf
         width >>= 1;
-        s = tip5::kOneM;
-        if (g < width && w < 10) s = tip5::to_m(buf[10 * g + w]);
-        __syncthreads();  // every read of buf precedes this level's writes
-        s = tip5::permutation_group16(s, w, lut);
-        if (g < width && w < tip5::DIGEST) {
-            const u64 d = tip5::from_m(s);
-            A.dst[j][5 * (blk * width + g) + w] = d;
-            buf[5 * g + w] = d;
+        u64 in[3] = {0, 0, 0};
+        if (first < width) {
+            const u64* c = buf + 10 * (t < width ? t : 0);
+            in[0] = c[W.g];
+            in[1] = c[4 + W.g];
+            if (W.g < 2) in[2] = c[8 + W.g];
         }
+        __syncthreads();  // every read of buf precedes the next level's writes
+        if (first < width) hash_pair(s, W, [&](u32 k) { return in[k >> 2]; });
     }
 }
 
-__global__ void __launch_bounds__(256) k_merkle_subtrees(MerkleArgs A) {
-    __shared__ uint8_t lut[256];
-    __shared__ u64 buf[256 * 5];
-    tip5::load_lut(lut);
+template <int THREADS>
+__global__ void __launch_bounds__(THREADS) k_merkle_subtrees(MerkleArgs A) {
+    __shared__ tip5::Tables T;
+    __shared__ u64 buf[THREADS / 64 * tip5::GROUP * 5];
+    tip5::load_tables(T);
+    const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    if (A.group16) merkle_body_group16(A, blockIdx.x, lut, buf);
-    else merkle_body(A, blockIdx.x, lut, buf);
+    merkle_body(A, blockIdx.x, W, buf);
 }
 
-__global__ void __launch_bounds__(256) k_merkle_subtrees_multi(const MerkleArgs* __restrict__ args,
-                                                               const u32* __restrict__ start,
-                                                               u32 nseg) {
-    __shared__ uint8_t lut[256];
-    __shared__ u64 buf[256 * 5];
-    tip5::load_lut(lut);
+__global__ void __launch_bounds__(kMerkleThreads) k_merkle_subtrees_multi(
+    const MerkleArgs* __restrict__ args, const u32* __restrict__ start, u32 nseg) {
+    __shared__ tip5::Tables T;
+    __shared__ u64 buf[kMerkleThreads / 64 * tip5::GROUP * 5];
+    tip5::load_tables(T);
+    const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
     u32 seg = find_seg(start, nseg, blockIdx.x);
     const MerkleArgs& A = args[seg];  // read in place: a private copy would spill dst[]
-    if (A.group16) merkle_body_group16(A, blockIdx.x - start[seg], lut, buf);
-    else merkle_body(A, blockIdx.x - start[seg], lut, buf);
+    merkle_body(A, blockIdx.x - start[seg], W, buf);
 }
 
 // Gather: out[q] = node with heap index idx[q] (1 <= idx < 2n) of a tree in
@@ -332,30 +324,29 @@ __global__ void k_gather_heap(const u64* __restrict__ tree, u64 n, u32 logn, int
 int launch_hash_rows(const u64* tab, u64 rows, u64 cols, u64* dig, hipStream_t st) {
     if (rows == 0) return TVH_OK;
     if (cols > 0xFFFFFFFFull) return TVH_ERR_INVALID_ARG;
-    u32 blocks = (u32)((rows + 255) / 256);
-    hipLaunchKernelGGL(k_hash_rows, dim3(blocks), dim3(256), 0, st, HashArgs{tab, rows, (u32)cols, dig});
+    hipLaunchKernelGGL(k_hash_rows, dim3(sponge_blocks(rows)), dim3(kHashThreads), 0, st,
+                       HashArgs{tab, rows, (u32)cols, dig});
     return check_launch();
 }
 
 int launch_absorb_chunk(const u64* chunk, u64 rows, u64 ccols, u64* state, u64* pend, u32 npend,
                         bool first, bool final_chunk, u64* dig, hipStream_t st) {
     if (rows == 0) return TVH_OK;
-    u32 blocks = (u32)((rows + 255) / 256);
+    const dim3 blocks(sponge_blocks(rows)), tpb(kHashThreads);
     if (final_chunk)
-        hipLaunchKernelGGL(k_absorb_chunk<true>, dim3(blocks), dim3(256), 0, st, chunk, rows,
-                           (u32)ccols, state, pend, npend, (int)first, dig);
+        hipLaunchKernelGGL(k_absorb_chunk<true>, blocks, tpb, 0, st, chunk, rows, (u32)ccols, state,
+                           pend, npend, (int)first, dig);
     else
-        hipLaunchKernelGGL(k_absorb_chunk<false>, dim3(blocks), dim3(256), 0, st, chunk, rows,
-                           (u32)ccols, state, pend, npend, (int)first, dig);
+        hipLaunchKernelGGL(k_absorb_chunk<false>, blocks, tpb, 0, st, chunk, rows, (u32)ccols, state,
+                           pend, npend, (int)first, dig);
     return check_launch();
 }
 
 // Fiat-Shamir sponge on a device-resident state (16 canonical u64), following
 // the reference's device transcript (fiat_shamir_kernel.cu: fs_absorb_device_gpu
 // pads [data..., 1, 0...] to a multiple of 10 and overwrites the rate before
-// each permutation; squeeze reads the rate, then permutes).  One lane runs the
-// whole absorption in one launch; the other 63 lanes of the wave only help
-// load the S-box table.
+// each permutation; squeeze reads the rate, then permutes).  One wave runs the
+// whole absorption in one launch; its 16 sponges are the same one.
 // mode 0 absorb, 1 squeeze, 2 init (zeros; a kernel rather than a memset so
 // that the call can be captured in a graph).
 __global__ void __launch_bounds__(64) k_sponge(u64* __restrict__ state,
@@ -365,31 +356,31 @@ __global__ void __launch_bounds__(64) k_sponge(u64* __restrict__ state,
         if (threadIdx.x < tip5::STATE) state[threadIdx.x] = 0;
         return;
     }
-    const bool squeeze = mode == 1;
-    __shared__ uint8_t lut[256];
-    tip5::load_lut(lut);
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    u64 s[tip5::STATE];
+    __shared__ tip5::Tables T;
+    tip5::load_tables(T);
+    const tip5::Wave W = tip5::make_wave(T);
+    u64 s[tip5::WORDS];
 #pragma unroll
-    for (int i = 0; i < tip5::STATE; i++) s[i] = tip5::to_m(state[i]);
-    if (squeeze) {
+    for (int v = 0; v < tip5::WORDS; v++) s[v] = tip5::to_m(state[4 * v + W.g]);
+    __syncthreads();  // (also: every lane has read the state before lanes n = 0 write it)
+    if (mode == 1) {
 #pragma unroll
-        for (int i = 0; i < tip5::RATE; i++) out[i] = tip5::from_m(s[i]);
-        tip5::permutation_m(s, lut);
+        for (int v = 0; v < 3; v++)
+            if (W.n == 0 && 4 * v + W.g < (u32)tip5::RATE) out[4 * v + W.g] = tip5::from_m(s[v]);
+        tip5::permutation_m(s, W);
     } else {
-        u64 padded = (len + 1 + tip5::RATE - 1) / tip5::RATE * tip5::RATE;
-        for (u64 base = 0; base < padded; base += tip5::RATE) {
-#pragma unroll
-            for (int i = 0; i < tip5::RATE; i++) {
-                u64 pos = base + i;
-                s[i] = pos < len ? tip5::to_m(data[pos]) : (pos == len ? tip5::kOneM : 0ull);
-            }
-            tip5::permutation_m(s, lut);
+        u64 base = 0;
+        for (; base + tip5::RATE <= len; base += tip5::RATE) {
+            absorb(s, W, [&](u32 i) { return data[base + i]; });
+            tip5::permutation_m(s, W);
         }
+        absorb_last(s, W, (u32)(len - base), [&](u32 i) { return data[base + i]; });
+        tip5::permutation_m(s, W);
     }
+    if (W.n == 0) {
 #pragma unroll
-    for (int i = 0; i < tip5::STATE; i++) state[i] = tip5::from_m(s[i]);
+        for (int v = 0; v < tip5::WORDS; v++) state[4 * v + W.g] = tip5::from_m(s[v]);
+    }
 }
 
 int launch_sponge(u64* state, const u64* data, u64 len, u64* out, int mode, hipStream_t st) {
@@ -419,7 +410,7 @@ int launch_xfe_leaves(const u64* xfe, u64 n, u64* leaves, hipStream_t st) {
 
 int launch_permutation(u64* states, u64 num, hipStream_t st) {
     if (num == 0) return TVH_OK;
-    hipLaunchKernelGGL(k_permutation, dim3((u32)((num + 255) / 256)), dim3(256), 0, st, states,
+    hipLaunchKernelGGL(k_permutation, dim3(sponge_blocks(num)), dim3(kHashThreads), 0, st, states,
                        num);
     return check_launch();
 }
@@ -427,15 +418,15 @@ int launch_permutation(u64* states, u64 num, hipStream_t st) {
 int launch_permutation_rounds(u64* states, u64 num, u32 first, u32 count, u64* trace,
                               hipStream_t st) {
     if (num == 0) return TVH_OK;
-    hipLaunchKernelGGL(k_permutation_rounds, dim3((u32)((num + 255) / 256)), dim3(256), 0, st,
+    hipLaunchKernelGGL(k_permutation_rounds, dim3(sponge_blocks(num)), dim3(kHashThreads), 0, st,
                        states, num, first, count, trace);
     return check_launch();
 }
 
 int launch_hash_pairs(const u64* l, const u64* r, u64* out, u64 count, hipStream_t st) {
     if (count == 0) return TVH_OK;
-    hipLaunchKernelGGL(k_hash_pairs, dim3((u32)((count + 255) / 256)), dim3(256), 0, st, l, r,
-                       out, count);
+    hipLaunchKernelGGL(k_hash_pairs, dim3(sponge_blocks(count)), dim3(kHashThreads), 0, st, l, r, out,
+                       count);
     return check_launch();
 }
 
@@ -444,31 +435,21 @@ u64 merkle_level_base(u64 n, u32 level, int layout) {
 }
 
 // Launch groups of the Merkle build of an n-leaf tree whose leaves are already
-// at level 0: group g covers up to 9 levels; T active threads per block.
-int merkle_groups(u64* tree, u64 n, int layout, std::vector<MerkleGroup>& groups) {
+// at level 0: group g covers up to 9 levels; T parents per block at its first.
+// A launch over many tables (multi) has one block size for all of them.
+int merkle_groups(u64* tree, u64 n, int layout, bool multi, std::vector<MerkleGroup>& groups) {
     groups.clear();
     u32 logn = log2u(n);
     u32 lvl = 0;
     while (lvl < logn) {
         u64 nchild = n >> lvl;
         u64 parents = nchild / 2;
-        // Levels of more than 2^15 parents take a launch each with one hash
-        // per thread (continuing inside a block would halve the active threads
-        // per level).  Above them one hash on one lane is a latency of ~21 us
-        // per level, so each hash runs on 16 lanes (permutation_group16, ~6 us):
-        // a 256-thread block hashes up to 16 parents and, once all blocks fit
-        // on the GPU at once (<= 2^14 parents), continues to their subtree root,
-        // up to 5 levels per launch.  Measured at 2^22 leaves: levels 2^16..1
-        // in 387 us with one lane per hash, 152 us in this form.
-        const bool group16 = parents <= (1u << 15);
-        u32 T = group16 ? (parents >= 16 ? 16 : (u32)parents)
-                        : (parents >= 256 ? 256 : (u32)parents);  // parents is a power of two
-        u32 maxlev = 0;
-        while ((1u << maxlev) <= T) maxlev++;  // T = 16 -> 5 levels
-        if (!group16 || parents > (1u << 14)) maxlev = 1;
+        const bool wide = parents > kMerkleSubtreeParents;
+        const u64 most = wide && !multi ? kSpongesPerBlock : kMerkleSponges;
+        u32 T = (u32)(parents < most ? parents : most);  // parents is a power of two
+        u32 maxlev = wide ? 1 : log2u(T) + 1;            // T = 256 -> 9 levels
         u32 levels = logn - lvl < maxlev ? logn - lvl : maxlev;
         MerkleGroup g;
-        g.args.group16 = group16 ? 1u : 0u;
         g.args.src = tree + 5 * merkle_level_base(n, lvl, layout);
         for (u32 j = 0; j < 9; j++)
             g.args.dst[j] = j < levels ? tree + 5 * merkle_level_base(n, lvl + j + 1, layout) : nullptr;
@@ -484,10 +465,14 @@ int merkle_groups(u64* tree, u64 n, int layout, std::vector<MerkleGroup>& groups
 // Build levels 1..log2(n) of a tree whose leaves are already at level 0.
 int launch_merkle_levels(u64* tree, u64 n, int layout, hipStream_t st) {
     std::vector<MerkleGroup> groups;
-    merkle_groups(tree, n, layout, groups);
+    merkle_groups(tree, n, layout, false, groups);
     for (const MerkleGroup& g : groups) {
-        hipLaunchKernelGGL(k_merkle_subtrees, dim3(g.blocks), dim3(g.args.group16 ? 256 : g.args.T),
-                           0, st, g.args);
+        if (g.args.T <= kSpongesPerBlock)
+            hipLaunchKernelGGL(k_merkle_subtrees<kHashThreads>, dim3(g.blocks), dim3(kHashThreads), 0,
+                               st, g.args);
+        else
+            hipLaunchKernelGGL(k_merkle_subtrees<kMerkleThreads>, dim3(g.blocks),
+                               dim3(kMerkleThreads), 0, st, g.args);
         int rc = check_launch();
         if (rc) return rc;
     }
@@ -497,15 +482,16 @@ int launch_merkle_levels(u64* tree, u64 n, int layout, hipStream_t st) {
 int launch_hash_rows_multi(const HashArgs* d_args, const u32* d_start, u32 nseg, u32 blocks,
                            hipStream_t st) {
     if (!blocks) return TVH_OK;
-    hipLaunchKernelGGL(k_hash_rows_multi, dim3(blocks), dim3(256), 0, st, d_args, d_start, nseg);
+    hipLaunchKernelGGL(k_hash_rows_multi, dim3(blocks), dim3(kHashThreads), 0, st, d_args, d_start,
+                       nseg);
     return check_launch();
 }
 
 int launch_merkle_multi(const MerkleArgs* d_args, const u32* d_start, u32 nseg, u32 blocks,
                         hipStream_t st) {
     if (!blocks) return TVH_OK;
-    hipLaunchKernelGGL(k_merkle_subtrees_multi, dim3(blocks), dim3(256), 0, st, d_args, d_start,
-                       nseg);
+    hipLaunchKernelGGL(k_merkle_subtrees_multi, dim3(blocks), dim3(kMerkleThreads), 0, st, d_args,
+                       d_start, nseg);
     return check_launch();
 }
 

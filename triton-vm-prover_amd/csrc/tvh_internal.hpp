@@ -243,6 +243,13 @@ int launch_fill_table(u64* d, u64 rows, u64 cols, u64 seed, u64* rej, hipStream_
 u64 fill_table_scratch_elems();
 
 // ---- Tip5 launchers (tip5_kernels.hip) ----
+// 16 sponges per wave: a block of the hashing kernels takes 64 of them.
+constexpr u32 kHashThreads = 256, kSpongesPerBlock = kHashThreads / 64 * tip5::GROUP;
+inline u32 sponge_blocks(u64 count) { return (u32)((count + kSpongesPerBlock - 1) / kSpongesPerBlock); }
+// Merkle levels of at most kMerkleSubtreeParents parents run several levels to
+// a launch, in blocks of up to kMerkleSponges parents.
+constexpr u32 kMerkleThreads = 1024, kMerkleSponges = kMerkleThreads / 64 * tip5::GROUP;
+constexpr u64 kMerkleSubtreeParents = 1u << 15;
 struct HashArgs {
     const u64* tab;
     u64 rows;
@@ -253,15 +260,13 @@ struct MerkleArgs {
     const u64* src;  // children level
     u64* dst[9];     // parents of the next `levels` levels
     u32 levels;
-    u32 T;           // parents per block at the first level (one thread each, or one
-                     // 16-lane group each when group16)
-    u32 group16;     // 1: each hash runs on 16 lanes (permutation_group16), 256-thread blocks
+    u32 T;           // parents per block at the first level
 };
 struct MerkleGroup {
     MerkleArgs args;
     u32 blocks;
 };
-int merkle_groups(u64* tree, u64 n, int layout, std::vector<MerkleGroup>& groups);
+int merkle_groups(u64* tree, u64 n, int layout, bool multi, std::vector<MerkleGroup>& groups);
 int launch_hash_rows_multi(const HashArgs* d_args, const u32* d_start, u32 nseg, u32 blocks,
                            hipStream_t st);
 int launch_merkle_multi(const MerkleArgs* d_args, const u32* d_start, u32 nseg, u32 blocks,

@@ -142,13 +142,7 @@ def autotune(lib, shapes, tvh, force=0, skip=False):
 def lde_kernels(lib, n, m, w) -> str:
     v = lib.lde_get_variant(n.bit_length() - 1, (m // n).bit_length() - 1, cols=w)
     tile = 14 - ((v >> 2) & 3)
-    if v & 3 == 1:
-        row = "k_lde_step2"
-    else:
-        rt = 13 if v & 16 else 12 if v & 64 else 14
-        it = 13 if v & 32 else rt
-        row = f"k_lde_rowinv<{it}> + k_lde_expand<{rt}>"
-    return f"LDE passes (k_step1<{tile}> + {row} + k_lde_step3<{tile}>)"
+    return f"LDE passes (k_step1<{tile}> + k_lde_rows or k_lde_cosets + k_lde_step3<{tile}>)"
 
 
 def run_main(args, tvh, lib, hip_rt):

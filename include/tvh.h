@@ -163,28 +163,22 @@ int tvh_lde_release_constants(void);
 /* ---- LDE kernel forms and autotuning -------------------------------------- */
 
 /* Kernel variants of the LDE, all with identical results.  A variant code is
- * form | (tile << 2).  The form is the kernel shape of the fused row step
- * (inverse row DFT, coset scaling, forward row DFT): TVH_LDE_WIDE runs it as
- * one kernel with all cosets of a row in one 1024-thread LDS tile;
- * TVH_LDE_SPLIT runs the inverse row DFTs as a kernel of their own (one more
- * read and write of the trace-sized data, every thread busy) before the
- * expansion.  Tile 0/1/2 gives the column steps LDS tiles of 2^14/2^13/2^12
- * elements (1024/512/256 threads).  TVH_LDE_ROW_HALF (with TVH_LDE_SPLIT only)
- * gives the two row kernels 2^13-element tiles (512 threads, two blocks per CU)
- * instead of 2^14, with the row length halved where E * row length would not
- * fit; TVH_LDE_INV_HALF (with TVH_LDE_SPLIT only, not with TVH_LDE_ROW_HALF)
- * gives only the inverse row kernel the 2^13 tile; TVH_LDE_ROW_QUARTER (with
- * TVH_LDE_SPLIT only, alone) gives both row kernels 2^12-element tiles (256
- * threads, four blocks per CU).  The variant is chosen per
- * (log2 trace_len, log2 expansion, width band), the width bands being
- * tables of fewer than 64 columns, 64..255 and 256 or more;
- * tvh_lde_set_variant sets every width band, tvh_lde_autotune the band of
- * its num_cols.  TVH_LDE_AUTO restores the default
- * (TVH_LDE_SPLIT with column tile 2 and TVH_LDE_ROW_QUARTER for 2^13..2^16
- * rows, TVH_LDE_ROW_HALF for 2^17..2^18, column tile 1 and TVH_LDE_ROW_HALF
- * from 2^19; TVH_LDE_SPLIT | TVH_LDE_INV_HALF with tile 1 at 2^12;
- * TVH_LDE_WIDE with tile 2 below).  Batch plans use each table's form with
- * column tile 1 and 2^13-element row tiles.
+ * form | (tile << 2) | flag.  Form and flag bound the tile of the row step
+ * (inverse row DFT, coset scaling, forward row DFTs in one kernel), which all
+ * cosets of a row share, and with it the row length: 2^14 elements with
+ * TVH_LDE_WIDE or TVH_LDE_SPLIT, 2^13 with TVH_LDE_SPLIT | TVH_LDE_ROW_HALF,
+ * 2^12 with TVH_LDE_SPLIT | TVH_LDE_ROW_QUARTER; TVH_LDE_INV_HALF (with
+ * TVH_LDE_SPLIT only, alone) is accepted and changes nothing.  Within that the
+ * library takes the shortest tile that holds the rows it chose.  Tile 0/1/2
+ * gives the column steps LDS tiles of 2^14/2^13/2^12 elements (1024/512/256
+ * threads).  The variant is chosen per (log2 trace_len, log2 expansion, width
+ * band), the width bands being tables of fewer than 64 columns, 64..255 and
+ * 256 or more; tvh_lde_set_variant sets every width band, tvh_lde_autotune the
+ * band of its num_cols.  TVH_LDE_AUTO restores the default: TVH_LDE_SPLIT with
+ * the shortest row tile that holds the whole transform's cosets (up to 2^14
+ * codeword elements) or leaves columns of 2^8, and column tile 1 (2 for tables
+ * of fewer than 2^23 elements).  Batch plans use each table's row tile and
+ * column tile 1.
  * No reference counterpart (the reference has one fixed kernel schedule per
  * size, src/gpu/kernels/ntt_kernel.cu). */
 enum {

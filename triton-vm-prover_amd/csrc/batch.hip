@@ -66,10 +66,10 @@ int tvh_batch_plan_create(const tvh_table_desc* tables, size_t count, tvh_batch_
     DeviceState* ds = current_device();
     if (!ds) return TVH_ERR_DEVICE;
     std::vector<Step1Args> s1;
-    std::vector<LdeArgs> s2w, s2i, s2e;  // wide row step; split form: inverse rows, expansion
+    std::vector<LdeArgs> s2[3];  // by row tile: 2^12, 2^13, 2^14
     std::vector<Step3Args> s3;
-    std::vector<u32> b1, b2w, b2i, b2e, b3;
-    std::vector<size_t> l1, l2w, l2i, l2e, l3;
+    std::vector<u32> b1, b2[3], b3;
+    std::vector<size_t> l1, l2[3], l3;
     std::vector<HashArgs> h;
     std::vector<u32> hb;
     std::vector<std::vector<MerkleArgs>> ma;
@@ -93,25 +93,17 @@ int tvh_batch_plan_create(const tvh_table_desc* tables, size_t count, tvh_batch_
         if (t.num_cols) {
             if (P.k1) {
                 s1.push_back(P.s1);
-                b1.push_back(P.s1_blocks);
-                l1.push_back(P.s1_lds);
+                b1.push_back(P.g1.blocks);
+                l1.push_back(P.g1.lds);
             }
-            if (P.split) {
-                s2i.push_back(P.s2inv);
-                b2i.push_back(P.inv_blocks);
-                l2i.push_back(P.inv_lds);
-                s2e.push_back(P.s2);
-                b2e.push_back(P.s2_blocks);
-                l2e.push_back(P.s2_lds);
-            } else {
-                s2w.push_back(P.s2);
-                b2w.push_back(P.s2_blocks);
-                l2w.push_back(P.s2_lds);
-            }
+            const u32 t2 = P.row_lt - 12;
+            s2[t2].push_back(P.s2);
+            b2[t2].push_back(P.g2.blocks);
+            l2[t2].push_back(P.g2.lds);
             if (P.k3) {
                 s3.push_back(P.s3);
-                b3.push_back(P.s3_blocks);
-                l3.push_back(P.s3_lds);
+                b3.push_back(P.g3.blocks);
+                l3.push_back(P.g3.lds);
             }
         }
         u64 m = t.target_len;
@@ -133,9 +125,7 @@ int tvh_batch_plan_create(const tvh_table_desc* tables, size_t count, tvh_batch_
     plan->device = ds->device;
     std::vector<uint8_t> blob;
     add_phase(blob, plan->lde[LDE_PHASE_STEP1], s1, b1, l1);
-    add_phase(blob, plan->lde[LDE_PHASE_ROWINV], s2i, b2i, l2i);
-    add_phase(blob, plan->lde[LDE_PHASE_STEP2], s2w, b2w, l2w);
-    add_phase(blob, plan->lde[LDE_PHASE_EXPAND], s2e, b2e, l2e);
+    for (int q = 0; q < 3; q++) add_phase(blob, plan->lde[LDE_PHASE_ROWS + q], s2[q], b2[q], l2[q]);
     add_phase(blob, plan->lde[LDE_PHASE_STEP3], s3, b3, l3);
     add_phase(blob, plan->hash, h, hb, {});
     plan->merkle.resize(ma.size());

@@ -35,22 +35,22 @@ static std::mutex g_dev_mu;
 static DeviceState g_devs[64];
 
 static int build_tables(DeviceState& ds) {
-    // 6 tables of 4096 entries: r4096 fwd/inv, lo fwd/inv, hi fwd/inv
-    std::vector<u64> h(6 * 4096);
+    // 6 tables of 4096 entries: r4096 fwd/inv, lo fwd/inv, hi fwd/inv; then the
+    // matrix sets of the small DFTs, fwd/inv
+    const size_t dft_words = dft_matrices_words();
+    std::vector<u64> h(6 * 4096 + dft_words);  // two directions of dft_words u32
     u64 w24 = gl::root_of_unity(kMaxLogN);
     u64 w24i = gl::inv(w24);
     u64 w4096 = gl::root_of_unity(12), w4096i = gl::inv(w4096);
     u64 w24_4096 = gl::pow(w24, 4096), w24i_4096 = gl::pow(w24i, 4096);
     u64 a = 1, ai = 1, b = 1, bi = 1, c = 1, ci = 1;
-    // stored in Montgomery form (w * 2^64 mod p): the kernels apply them with gl::mont_mul
-    auto m = [](u64 x) { return gl::canon(gl::to_mont(x)); };
     for (int e = 0; e < 4096; e++) {
-        h[0 * 4096 + e] = m(a);
-        h[1 * 4096 + e] = m(ai);
-        h[2 * 4096 + e] = m(b);
-        h[3 * 4096 + e] = m(bi);
-        h[4 * 4096 + e] = m(c);
-        h[5 * 4096 + e] = m(ci);
+        h[0 * 4096 + e] = a;
+        h[1 * 4096 + e] = ai;
+        h[2 * 4096 + e] = b;
+        h[3 * 4096 + e] = bi;
+        h[4 * 4096 + e] = c;
+        h[5 * 4096 + e] = ci;
         a = gl::mul(a, w4096);
         ai = gl::mul(ai, w4096i);
         b = gl::mul(b, w24);
@@ -58,6 +58,8 @@ static int build_tables(DeviceState& ds) {
         c = gl::mul(c, w24_4096);
         ci = gl::mul(ci, w24i_4096);
     }
+    for (int dir = 0; dir < 2; dir++)
+        build_dft_matrices(dir == 1, (u32*)(h.data() + 6 * 4096) + dir * dft_words);
     u64* d = nullptr;
     if (hipMalloc(&d, h.size() * sizeof(u64)) != hipSuccess)
         return set_error(TVH_ERR_OOM, "twiddle tables");
@@ -70,6 +72,7 @@ static int build_tables(DeviceState& ds) {
         ds.roots.r4096[dir] = d + (0 + dir) * 4096;
         ds.roots.lo[dir] = d + (2 + dir) * 4096;
         ds.roots.hi[dir] = d + (4 + dir) * 4096;
+        ds.roots.dft[dir] = (const u32*)(d + 6 * 4096) + dir * dft_words;
     }
     return TVH_OK;
 }

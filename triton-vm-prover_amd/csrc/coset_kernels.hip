@@ -16,18 +16,18 @@ namespace tvh {
 
 namespace {
 
-// t[i] = base^i in Montgomery form (base^i * 2^64 mod p), i < count: one
+// t[i] = base^i, i < count: one
 // square-and-multiply per entry (a table of at most 4096 entries per call).
 __global__ void k_pow_table(u64* __restrict__ t, u64 base, u32 count) {
     u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) t[i] = gl::canon(gl::to_mont(gl::pow(base, i)));
+    if (i < count) t[i] = gl::pow(base, i);
 }
 
 constexpr int kTabTpb = 256;
 constexpr int kTabPer = 4;  // elements per thread, kTabTpb apart (coalesced)
 
 // y[c*n + i] = (x[c*n + i] + [i < k] rand[c*k + i] * delta) * base^i with
-// base^i = tlo[i mod 4096] * thi[i / 4096] (Montgomery-form tables): two
+// base^i = tlo[i mod 4096] * thi[i / 4096]: two
 // cached loads and two products per element.  x may equal y.
 __global__ void __launch_bounds__(kTabTpb) k_scale_table(const u64* x, u64* y, u64 n, u32 log_n,
                                                          u64 total, const u64* __restrict__ tlo,
@@ -42,8 +42,7 @@ __global__ void __launch_bounds__(kTabTpb) k_scale_table(const u64* x, u64* y, u
         u64 i = e & (n - 1);
         u64 v = x[e];
         if (i < k) v = gl::add(v, gl::mul(rand[(e >> log_n) * k + i], delta));
-        u64 f = gl::mont_mul(tlo[i & 4095], thi[i >> 12]);  // base^i in Montgomery form
-        y[e] = gl::mont_mul(v, f);
+        y[e] = gl::mul(v, gl::mul(tlo[i & 4095], thi[i >> 12]));
     }
 }
 

@@ -267,19 +267,27 @@ __device__ __forceinline__ bool in_mask(mask m) { return __builtin_amdgcn_invers
     asm volatile("v_subb_co_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(ko) : "v"(a), "v"(b), "s"(k))
 #define GL_SUBB_0(r, ko, a, k) \
     asm volatile("v_subb_co_u32 %0, %1, %2, 0, %3" : "=v"(r), "=s"(ko) : "v"(a), "s"(k))
-// bad |= k & ~c (k is overwritten); kept on the scalar unit
-#define GL_NOTE(bad, k, c) \
-    asm volatile("s_andn2_b64 %1, %1, %2\n\ts_or_b64 %0, %0, %1" : "+s"(bad), "+s"(k) : "s"(c) : "scc")
 // r = a * b + c (64 bits) and the carry out; the second form has b = 2^32 - 1
 #define GL_MAD_CO(r, k, a, b, c) \
     asm volatile("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(k) : "v"(a), "v"(b), "v"(c))
 #define GL_MAD_EPS_CO(r, k, a, c) \
     asm volatile("v_mad_u64_u32 %0, %1, %2, -1, %3" : "=v"(r), "=s"(k) : "v"(a), "v"(c))
 
-// l + (h1:h0) * 2^64 -> lazy u64, or bad
+// Lanes of value i with k & ~c (k is overwritten), kept on the scalar unit: in a
+// mask of its own, or joined to one mask for all values.
 template <int N>
+__device__ __forceinline__ void note_rare(mask (&bad)[N], int i, mask& k, mask c) {
+    asm volatile("s_andn2_b64 %0, %1, %2" : "=s"(bad[i]) : "s"(k), "s"(c) : "scc");
+}
+__device__ __forceinline__ void note_rare(mask& bad, int, mask& k, mask c) {
+    asm volatile("s_andn2_b64 %1, %1, %2\n\ts_or_b64 %0, %0, %1" : "+s"(bad), "+s"(k) : "s"(c) : "scc");
+}
+
+// l + (h1:h0) * 2^64 -> lazy u64, or bad: r then has to be lowered by 2^32 - 1
+// (u - h1 wrapped to at least 2^64 - 2^32).  Bad: mask[N] or mask.
+template <int N, class Bad>
 __device__ __forceinline__ void fold128_rare(u64 (&r)[N], const u64 (&l)[N], const u32 (&h0)[N],
-                                             const u32 (&h1)[N], mask& bad) {
+                                             const u32 (&h1)[N], Bad& bad) {
     static_assert(N >= 3, "wait states");
     u64 u[N];
     u32 r0[N], r1[N];
@@ -291,18 +299,17 @@ __device__ __forceinline__ void fold128_rare(u64 (&r)[N], const u64 (&l)[N], con
 #pragma unroll
     for (int i = 0; i < N; i++) GL_SUBB_0(r1[i], k[i], (u32)(u[i] >> 32), k[i]);
 #pragma unroll
-    for (int i = 0; i < N; i++) GL_ADDC_0(r1[i], none, r1[i], c[i]);              // + c * 2^32
+    for (int i = 0; i < N; i++) GL_ADDC_0(r1[i], none, r1[i], c[i]);                // + c * 2^32
 #pragma unroll
     for (int i = 0; i < N; i++) {
-        GL_NOTE(bad, k[i], c[i]);
+        note_rare(bad, i, k[i], c[i]);
         r[i] = mk64(r0[i], r1[i]);
     }
 }
 
 // r = a * b, any u64 -> lazy u64, or bad
-template <int N>
-__device__ __forceinline__ void mul_rare(u64 (&r)[N], const u64 (&a)[N], const u64 (&b)[N],
-                                         mask& bad) {
+template <int N, class Bad>
+__device__ __forceinline__ void mul_rare(u64 (&r)[N], const u64 (&a)[N], const u64 (&b)[N], Bad& bad) {
     static_assert(N >= 3, "wait states");
     u64 p[N], q[N], y[N], l[N];
     u32 l1[N], h0[N], h1[N];
@@ -328,8 +335,8 @@ __device__ __forceinline__ void mul_rare(u64 (&r)[N], const u64 (&a)[N], const u
 }
 
 // r = a * a, any u64 -> lazy u64, or bad
-template <int N>
-__device__ __forceinline__ void sqr_rare(u64 (&r)[N], const u64 (&a)[N], mask& bad) {
+template <int N, class Bad>
+__device__ __forceinline__ void sqr_rare(u64 (&r)[N], const u64 (&a)[N], Bad& bad) {
     static_assert(N >= 3, "wait states");
     u64 p[N], q[N], x[N], l[N];
     u32 l1[N], h0[N], h1[N];
@@ -362,6 +369,33 @@ __device__ __forceinline__ void sqr_rare(u64 (&r)[N], const u64 (&a)[N], mask& b
     fold128_rare(r, l, h0, h1, bad);
 }
 
+// r = a * b, any u64 -> lazy u64 (exact; the unlikely borrow in a branch)
+template <int N>
+__device__ __forceinline__ void mul_n(u64 (&r)[N], const u64 (&a)[N], const u64 (&b)[N]) {
+    mask bad[N], any = 0;
+    mul_rare(r, a, b, bad);
+#pragma unroll
+    for (int i = 0; i < N; i++) asm volatile("s_or_b64 %0, %0, %1" : "+s"(any) : "s"(bad[i]) : "scc");
+    if (__builtin_expect(in_mask(any), 0)) {
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            if (in_mask(bad[i])) r[i] -= EPS;
+    }
+}
+
+// lazy -> canonical: p <= x < 2^64 only with a high word of ones
+template <int N>
+__device__ __forceinline__ void canon_n(u64 (&x)[N]) {
+    bool big = false;
+#pragma unroll
+    for (int i = 0; i < N; i++) big |= (u32)(x[i] >> 32) == 0xFFFFFFFFu;
+    if (__builtin_expect(big, 0)) {
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            if (x[i] >= P) x[i] -= P;
+    }
+}
+
 // x * 2^64 (into Montgomery form), any u64 -> lazy u64, or bad (only when the
 // low word of x is 0 and the high one is not)
 template <int N>
@@ -383,7 +417,7 @@ __device__ __forceinline__ void to_mont_rare(u64 (&r)[N], const u64 (&x)[N], mas
     }
 }
 
-// Constants of join_bytes that the compiler must not see through (it would
+// Constants of the joins that the compiler must not see through (it would
 // replace the multiply-adds by shifts and carries).
 struct JoinConsts {
     u32 two16, eps;
@@ -395,21 +429,23 @@ __device__ __forceinline__ JoinConsts join_consts() {
 }
 
 // Sum of d[t] * 256^t over eight byte places whose pair sums A = d[0] + 256 d[1],
-// B, C, D lie in [0, 2^31): A + B 2^16 + C 2^32 + D 2^48 -> u64 congruent to it.
-// With H = C + D 2^16 < 2^48 the value is (A + B 2^16) + H0 2^32 + H1 (2^32 - 1),
-// whose 64-bit sum carries only when H0 is within 2^17 of 2^32 (once in 2^15):
-// `carry` then says that 2^32 - 1 has to be added.  Three multiply-adds and one
-// add with carry after the four shift-adds.
-__device__ __forceinline__ u64 join_bytes_rare(const JoinConsts& J, u32 d0, u32 d1, u32 d2, u32 d3,
-                                               u32 d4, u32 d5, u32 d6, u32 d7, bool& carry) {
-    const u32 A = d0 + (d1 << 8), B = d2 + (d3 << 8), C = d4 + (d5 << 8), D = d6 + (d7 << 8);
-    const u64 L = (u64)B * J.two16 + A, H = (u64)D * J.two16 + C;
+// B, C, D lie in [0, 2^31): L + H 2^32 with the halves L = A + B 2^16 and
+// H = C + D 2^16, each below 2^48.
+__device__ __forceinline__ u64 join_half(const JoinConsts& J, u32 d0, u32 d1, u32 d2, u32 d3) {
+    const u32 A = d0 + (d1 << 8), B = d2 + (d3 << 8);
+    return (u64)B * J.two16 + A;
+}
+// L + H 2^32 -> u64 congruent to it: L + H0 2^32 + H1 (2^32 - 1), whose 64-bit
+// sum carries only when H0 is within 2^17 of 2^32 (once in 2^15 and less):
+// `carry` then says that 2^32 - 1 has to be added.
+__device__ __forceinline__ u64 join_rare(const JoinConsts& J, u64 L, u64 H, bool& carry) {
     const u64 L2 = (u64)(u32)(H >> 32) * J.eps + L;
     u32 k;
     const u32 r1 = __builtin_addc((u32)(L2 >> 32), (u32)H, 0u, &k);
     carry = k != 0;
     return mk64((u32)L2, r1);
 }
+
 // 2^e mod p for 0 <= e < 192 (compile-time usable)
 __host__ __device__ constexpr u64 pow2_mod_p(int e) {
     u64 r = 1;

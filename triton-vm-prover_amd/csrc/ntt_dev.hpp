@@ -10,339 +10,467 @@
 // Each size-N transform is a four-step split N = N1 * N2 (N1 = 2^a):
 //   step 1: N1-point DFTs down the columns of the N1 x N2 view, twiddle w_N^(n2 k1)
 //   step 2: N2-point DFTs along rows (k1 fixed)
-// The LDE fuses INTT step 2, the coset scaling of all E cosets and forward
-// step 1 into one kernel (k_lde_step2), so a column is read from HBM three
-// times and written three times, with d_out as the only working memory:
+// The LDE runs INTT step 2, the coset scaling of all E cosets and forward step 1
+// on whole rows in one kernel, with d_out as the only working memory:
 //   K1  trace            -> Y   at out[E*N2*k1 + n2]
 //   K2  Y (rows k1)      -> Z_s at out[E*(u1 + N2*k1) + s]   (in place per row)
 //   K3  Z (u1-tile, all s) -> codewords at out[E*(u1 + N2*u2) + s] (in place)
-// Sub-DFTs of length L <= 4096 run in LDS as Stockham radix-16 passes: each
-// thread holds R values, applies w_(Ns*R)^(k*r) from a table and an R-point
-// DFT whose twiddles are powers of two (w_64 = 2^39), natural order in/out.
+//
+// Sub-DFTs of length L <= 4096 run in LDS as radix-16 passes whose 16-point
+// DFTs are matrix products (see Matrix).  Values between the kernels and inside
+// them are lazy (any u64 congruent mod p); a kernel whose output leaves the
+// library makes it canonical.
 //
 // This header holds the device code shared by the translation units that
-// instantiate the kernels (ntt_step1.hip, lde_rows.hip, lde_expand.hip,
+// instantiate the kernels (ntt_step1.hip, ntt_step2.hip, lde_rows.hip,
 // lde_step3.hip); the host side (plans, constant tables, launches) is
 // ntt_kernels.hip.
+//
+// Measured on a 2^20 x 379 table to four cosets (3.2 GB in, 12.7 GB out), with
+// radix-16 butterflies on the VALU before: K1 1.67 ms (2.2), K2 12.3 (12.2 in two
+// kernels, which wrote and read the coefficients in between), K3 5.3 (7.1).  K1 and
+// K3 move 3.8 and 4.8 TB/s, near what the memory gives a kernel that reads and
+// writes the same amount; K2 is bound by VALU issue: per output two products for
+// the twiddles between passes, one for the coset, two for the twiddle on the way
+// out, and 12 operations in each of three DFT passes.
 #pragma once
 
-#include <utility>
+#include <type_traits>
 
 #include "tvh_internal.hpp"
 
 namespace tvh {
 
-constexpr int TPB = 1024;    // threads per block of every NTT kernel (16 waves)
-constexpr int TILE = 16384;  // u64 elements per block: 16 per thread, 128 KB before padding
-constexpr int LOG_TILE = 14;
-
-__device__ __forceinline__ int pidx(int t, int i, int Lp) { return t * Lp + i + (i >> 4); }
-__host__ __device__ inline int padded_len(int L) { return L + (L >> 4) + 1; }
-
-template <int LOGR>
-__device__ __forceinline__ constexpr int brev(int i) {
-    int r = 0;
-    for (int b = 0; b < LOGR; b++)
-        if (i & (1 << b)) r |= 1 << (LOGR - 1 - b);
-    return r;
-}
-
-// R-point DFT in registers, natural order in and out: radix-2 DIT on the
-// bit-reversed input.  The butterflies of stage LEN use w_LEN^j =
-// 2^(39*(64/LEN)*j mod 192) (w_64 = 2^39); a twiddle 2^e with e >= 96 is
-// -2^(e-96), folded into the butterfly by swapping add and sub; 2^e itself is
-// applied by word shifts (gl::mul_pow2).  Every index and exponent is a
-// template constant (index sequences), so the whole DFT is straight-line code.
-template <bool INV, int LEN, int J>
-__device__ __forceinline__ void dft_bfly(u64& x, u64& y) {
-    constexpr int e0 = (39 * (64 / LEN) * J) % 192;
-    constexpr int e = INV ? (192 - e0) % 192 : e0;
-    constexpr bool negw = e >= 96;
-    constexpr int ep = negw ? e - 96 : e;
-    u64 t = ep == 0 ? y : gl::mul_pow2<ep>(y);
-    u64 u = x;
-    if (negw) {
-        x = gl::sub(u, t);
-        y = gl::add(u, t);
-    } else {
-        x = gl::add(u, t);
-        y = gl::sub(u, t);
-    }
-}
-
-template <bool INV, int LEN, size_t... K>
-__device__ __forceinline__ void dft_stage(u64* a, std::index_sequence<K...>) {
-    // butterfly K: group K / (LEN/2), offset j = K % (LEN/2)
-    (dft_bfly<INV, LEN, (int)(K % (LEN / 2))>(a[(K / (LEN / 2)) * LEN + K % (LEN / 2)],
-                                             a[(K / (LEN / 2)) * LEN + K % (LEN / 2) + LEN / 2]),
-     ...);
-}
-
-template <int LOGR, bool INV, size_t... S>
-__device__ __forceinline__ void dft_stages(u64* a, std::index_sequence<S...>) {
-    (dft_stage<INV, (2 << S)>(a, std::make_index_sequence<(1 << LOGR) / 2>{}), ...);
-}
-
-template <int LOGR, bool INV>
-__device__ __forceinline__ void dft_reg(u64* v) {
-    constexpr int R = 1 << LOGR;
-    u64 a[R];
-#pragma unroll
-    for (int i = 0; i < R; i++) a[i] = v[brev<LOGR>(i)];
-    dft_stages<LOGR, INV>(a, std::make_index_sequence<LOGR>{});
-#pragma unroll
-    for (int i = 0; i < R; i++) v[i] = a[i];
-}
-
-template <int LOGR, bool INV, int NTPB = TPB, int NTILE = TILE>
-__device__ __forceinline__ void stockham_pass(u64* buf, int logL, int Lp, int NT, int Ns,
-                                              const u64* __restrict__ r4096) {
-    constexpr int R = 1 << LOGR;
-    constexpr int MAXIT = NTILE / (R * NTPB);
-    const int per = 1 << (logL - LOGR);
-    const int total = NT << (logL - LOGR);
-    const int step = 4096 / (Ns * R);
-    static_assert(MAXIT >= 1, "radix larger than the per-thread element count");
-    u64 v[MAXIT][R];
-#pragma unroll
-    for (int it = 0; it < MAXIT; it++) {
-        int w = threadIdx.x + it * NTPB;
-        if (w < total) {
-            int t = w >> (logL - LOGR);
-            int j = w & (per - 1);
-            int k = j & (Ns - 1);
-#pragma unroll
-            for (int r = 0; r < R; r++) v[it][r] = buf[pidx(t, j + r * per, Lp)];
-            if (Ns > 1) {
-#pragma unroll
-                for (int r = 1; r < R; r++) v[it][r] = gl::mont_mul(v[it][r], r4096[k * r * step]);
-            }
-            dft_reg<LOGR, INV>(v[it]);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < MAXIT; it++) {
-        int w = threadIdx.x + it * NTPB;
-        if (w < total) {
-            int j = (w) & (per - 1);
-            int t = w >> (logL - LOGR);
-            int k = j & (Ns - 1);
-            int base = (j - k) * R + k;
-#pragma unroll
-            for (int r = 0; r < R; r++) buf[pidx(t, base + r * Ns, Lp)] = v[it][r];
-        }
-    }
-    __syncthreads();
-}
-
-// NT transforms of length 2^logL (<= 4096) in LDS; NT * L <= NTILE; NTPB
-// threads hold NTILE / NTPB values each.
-template <bool INV, int NTPB = TPB, int NTILE = TILE>
-__device__ __forceinline__ void lds_dft(u64* buf, int logL, int NT, const u64* __restrict__ r4096) {
-    const int Lp = padded_len(1 << logL);
-    int Ns = 1;
-    int rem = logL;
-    while (rem >= 4) {
-        stockham_pass<4, INV, NTPB, NTILE>(buf, logL, Lp, NT, Ns, r4096);
-        Ns <<= 4;
-        rem -= 4;
-    }
-    if (rem == 3) stockham_pass<3, INV, NTPB, NTILE>(buf, logL, Lp, NT, Ns, r4096);
-    else if (rem == 2) stockham_pass<2, INV, NTPB, NTILE>(buf, logL, Lp, NT, Ns, r4096);
-    else if (rem == 1) stockham_pass<1, INV, NTPB, NTILE>(buf, logL, Lp, NT, Ns, r4096);
-}
-
-// ---------------------------------------------------------------- fused-endpoint DFT
-// The same Stockham passes as lds_dft, but the first pass takes its inputs
-// straight from global memory (a Load functor) and the last pass writes its
-// outputs straight to global memory (a Store functor): per transform one LDS
-// write and read per middle pass instead of a global->LDS copy before and an
-// LDS->global copy after, and 2 barriers per middle pass only.  A one-pass
-// transform (L <= 16) never touches LDS.
+// ---------------------------------------------------------------- 16-point DFT
+// A wave transforms 16 groups of 16 elements at once: lane 16g + n holds
+// elements e = 4v + g (v = 0..3) of group n, before and after (natural order),
+// the operand and result layout of v_mfma_i32_16x16x64_i8.
 //
-// Work item (t, j) of a radix-R pass: v[r] = x_t[j + r*per] (times the
-// Stockham twiddle when Ns > 1), R-point DFT, y_t[(j - k)*R + k + r*Ns] = v[r]
-// with k = j mod Ns.  Functors: load(t, j, per, v) fills v[0..R); store(t, j,
-// Ns, v) writes it.  TF (transform-fastest): adjacent threads take adjacent
-// transforms (column kernels, whose transforms are adjacent in memory);
-// otherwise adjacent elements of one transform (row kernels).
-struct LdsIO {
-    u64* buf;
-    int Lp;
-    template <int R>
-    __device__ __forceinline__ void load(int t, int j, int per, u64 (&v)[R]) const {
+// w_64 = 2^39, so a 16-point DFT (and the 2-, 4- and 8-point ones, 2^(4-r) of
+// them side by side) has coefficients +-2^x.  With an element split into bytes,
+// x = lo + 2^32 hi and 2^64 = 2^32 - 1, every output is a sum of eight byte
+// places, s and 4 + s for s < 4, of fixed signed bytes +-2^(x mod 8):
+//   place s: P_s lo - Q_s hi,  place 4 + s: Q_s lo + S_s hi,  S_s = P_s + Q_s.
+// Bytes are made signed by flipping their top bits; -Q_s hi is taken as Q_s * ~hi.
+// The constants this leaves and a bias that keeps the sums positive start the
+// accumulators.  16 products on the matrix cores and about 12 VALU operations
+// per element for the bytes and the join replace the 39 of the butterflies on
+// the VALU, which is what bounded the kernels.  256 elements take 360 cycles of
+// a SIMD with four waves on it (a product costs the VALU about 7 of its 16
+// cycles); with S_s hi as two products, which saves 16 registers, 440; with 2:4
+// sparse products, whose accumulators the VALU has to fill, 370.
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+constexpr u32 LOG_TILE = 14;  // log2 elements of the largest tile (128 KB before padding)
+
+// kDftWords u32 per matrix set (direction, r): P, Q, S for s = 0..3, each 64 lanes
+// x 4 words; then the accumulator starts of the even places, [4][g][v].
+constexpr u32 kDftStarts = 12 * 64 * 4;
+constexpr u32 kDftWords = kDftStarts + 64;
+constexpr u32 kDftBias = 1u << 25;
+constexpr u32 kSignBits = 0x80808080u;
+
+// The matrices stay in registers; the starts are read for each product, into the
+// registers of its result.
+struct Matrix {
+    v4i p[4], q[4], s[4];
+    const v4i* start;  // LDS (or global); the lane's first
+};
+__device__ __forceinline__ Matrix load_matrix(const u32* __restrict__ set, const u32* starts) {
+    Matrix M;
+    const u32 lane = threadIdx.x & 63;
+    const v4i* w = (const v4i*)set;
 #pragma unroll
-        for (int r = 0; r < R; r++) v[r] = buf[pidx(t, j + r * per, Lp)];
+    for (int i = 0; i < 4; i++) {
+        M.p[i] = w[i * 64 + lane];
+        M.q[i] = w[(4 + i) * 64 + lane];
+        M.s[i] = w[(8 + i) * 64 + lane];
     }
-    template <int R>
-    __device__ __forceinline__ void store(int t, int j, int Ns, const u64 (&v)[R]) const {
-        int k = j & (Ns - 1);
-        int base = (j - k) * R + k;
+    M.start = (const v4i*)starts + (lane >> 4);
+    return M;
+}
+
+// x any u64 -> lazy.  (The barriers keep other code's asm, whose registers the
+// compiler's hazard checks do not see, out of the matrix products; the one in
+// the middle halves the accumulators held at a time.)
+__device__ __forceinline__ void dft16(const Matrix& M, const gl::JoinConsts& J, u64 (&x)[4]) {
+    __builtin_amdgcn_sched_barrier(0);
+    v4i lo, hi, nh;
 #pragma unroll
-        for (int r = 0; r < R; r++) buf[pidx(t, base + r * Ns, Lp)] = v[r];
+    for (int v = 0; v < 4; v++) {
+        lo[v] = (int)((u32)x[v] ^ kSignBits);
+        hi[v] = (int)((u32)(x[v] >> 32) ^ kSignBits);
+        nh[v] = (int)((u32)(x[v] >> 32) ^ ~kSignBits);
+    }
+    const v4i zero = {0, 0, 0, 0};
+    v4i y[4];
+    u64 H[4];
+#define TVH_MFMA(a, b, c) __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0)
+#pragma unroll
+    for (int s = 0; s < 4; s++) y[s] = TVH_MFMA(M.q[s], lo, s & 1 ? zero : M.start[8 + 2 * s]);
+#pragma unroll
+    for (int s = 0; s < 4; s++) y[s] = TVH_MFMA(M.s[s], hi, y[s]);
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+        H[v] = gl::join_half(J, (u32)y[0][v], (u32)y[1][v], (u32)y[2][v], (u32)y[3][v]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < 4; s++) y[s] = TVH_MFMA(M.p[s], lo, s & 1 ? zero : M.start[2 * s]);
+#pragma unroll
+    for (int s = 0; s < 4; s++) y[s] = TVH_MFMA(M.q[s], nh, y[s]);
+#undef TVH_MFMA
+    bool carry[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const u64 L = gl::join_half(J, (u32)y[0][v], (u32)y[1][v], (u32)y[2][v], (u32)y[3][v]);
+        x[v] = gl::join_rare(J, L, H[v], carry[v]);
+    }
+    if (__builtin_expect(carry[0] | carry[1] | carry[2] | carry[3], 0)) {
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (carry[v]) x[v] += gl::EPS;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// ---------------------------------------------------------------- DFTs of a block
+// NT transforms of length L = 2^logL (16 < L <= 4096), NT * L <= 2^LT, in LDS by
+// decimation in frequency.  L = 2^rA * 2^rB * 16 with rB = min(4, logL - 4):
+//   pass A (L > 256): 2^rA-point DFTs over the top index bits, over the block;
+//   passes B, C: the 256-element (or shorter) pieces that remain, each by one
+//   wave on its own: no barrier lies between, and the twiddles between B and C
+//   are the lane's for the whole kernel.
+// A pass takes 16 elements i0 + e*S, S a sixteenth of the sub-transform; for
+// r < 4 the low 4 - r bits of e are left alone.  After pass A the result is
+// multiplied by w^(rest * digit) and goes back where it came from; pass C leaves
+// its piece in natural order.  So result k of the transform is at place
+// (k mod 2^rA) * 256 + k / 2^rA (result_place).
+//
+// A block has 2^(LT-4) threads, 16 elements each: all global loads are in flight
+// together, before the matrices take their registers, and the results are
+// stored from LDS in the order of global memory.  Tile and length are
+// compile-time constants, so that LDS accesses take immediate offsets; global
+// ones take a wave-uniform base and a byte offset that the lane keeps
+// throughout.  (With both at run time the same code took 1.6 times the VALU
+// instructions and spilled registers.)
+template <int LT, int LOGL, int LOGQ = 4>
+struct Shape {
+    static constexpr u32 kThreads = 1u << (LT - LOGQ), kWaves = kThreads / 64;
+    static constexpr u32 kPer = 1u << LOGQ;  // elements of a thread
+    static constexpr u32 L = 1u << LOGL, logNT = LT - LOGL, NT = 1u << logNT;
+    static constexpr u32 rA = LOGL > 8 ? LOGL - 8 : 0;
+    static constexpr u32 logP = LOGL < 8 ? LOGL : 8;  // length of a transform's piece
+    static constexpr u32 rB = logP - 4;
+    // LDS pitch of a transform.  Adjacent lanes take min(NT, 16) transforms and
+    // then adjacent elements: the pitch is an odd multiple of 16 / min(NT, 16),
+    // which spreads them over the banks.
+    static constexpr u32 unit = logNT >= 4 ? 1 : 16u >> logNT;
+    static constexpr u32 pitch = unit * (((L + (L >> 4) + (L >> 8) + unit) / unit) | 1);
+    static constexpr u32 kStarts = pitch * NT;  // two sets of accumulator starts follow
+};
+
+// Element i of transform t: base[(t >> sh) * ts + (t mod 2^sh) * ts2 + i * is].
+// (base: the block's first transform.)
+template <class T>
+struct Place {
+    T* base;
+    u32 sh, ts, ts2, is;
+    __device__ __forceinline__ u32 off(u32 t, u32 i) const {
+        return (t >> sh) * ts + (t & ((1u << sh) - 1)) * ts2 + i * is;
     }
 };
 
+// Access at a wave-uniform base plus the lane's byte offset (below 2^32: one
+// instruction, no address arithmetic).
+__device__ __forceinline__ u64 load_at(const u64* base, u32 bytes) {
+    return *(const u64*)((const char*)base + bytes);
+}
+__device__ __forceinline__ void store_at(u64* base, u32 bytes, u64 x) {
+    *(u64*)((char*)base + bytes) = x;
+}
+
+// LDS place of element i.  (Additive over index parts that share no bit.)
+__host__ __device__ constexpr u32 lds_index(u32 i) { return i + (i >> 4) + (i >> 8); }
+// Where result k lies.
+__host__ __device__ constexpr u32 result_place(u32 k, u32 rA) {
+    return ((k & ((1u << rA) - 1)) << 8) | (k >> rA);
+}
+
 // Workgroup barrier for LDS hand-offs only: waits for this wave's LDS
-// operations, not for its global loads (the __syncthreads fence also drains
-// the vector-memory counter, which would expose the latency of twiddle loads
-// issued ahead of the barrier).  No thread of these kernels reads global
+// operations, not for its global ones.  No thread of these kernels reads global
 // memory that another thread of the block writes before the barrier.
 __device__ __forceinline__ void lds_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
+// LDS hand-off between lanes of one wave: its LDS operations execute in order,
+// so only the compiler has to keep theirs.
+__device__ __forceinline__ void wave_handoff() { asm volatile("" ::: "memory"); }
 
-// Stockham twiddles of one pass for the thread's work items, loaded ahead of
-// the pass: tw.t[it][r] = r4096[k * r * step] (r >= 1) for work item it.
-template <int LOGR, int NTPB, int NTILE>
-struct PassTw {
-    static constexpr int R = 1 << LOGR;
-    static constexpr int MAXIT = NTILE / (R * NTPB);
-    u64 t[MAXIT][R];
+__device__ __forceinline__ u32 wave_index() {
+    return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+}
+
+template <u32 LOGS>
+__device__ __forceinline__ void lds_put(u64* p, const u64 (&x)[4]) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) p[lds_index((u32)(4 * v) << LOGS)] = x[v];
+}
+template <u32 LOGS>
+__device__ __forceinline__ void lds_get(const u64* p, u64 (&x)[4]) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) x[v] = p[lds_index((u32)(4 * v) << LOGS)];
+}
+
+// Twiddles w_(16 S)^(rest * digit), rest = (e mod 2^(4-R)) S + jl, digit = e >> (4-R),
+// of the elements e = 4v + g of a group with offset jl < S in a pass of digit bits
+// R and stride S = 2^LOGS.
+template <u32 R, u32 LOGS>
+__device__ __forceinline__ void pass_twiddles(u64 (&f)[4], u32 jl, u32 g, const u64* __restrict__ r4096) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const u32 e = 4 * v + g;
+        f[v] = load_at(r4096, (((e & ((1u << (4 - R)) - 1)) << LOGS) + jl) * ((e >> (4 - R)) << (11 - LOGS)));
+    }
+}
+
+// Pass A on the first 2^log_t transforms: groups j of stride S = L / 16, lanes
+// transform-fastest.  The next group's elements and twiddles are loaded before
+// this one is transformed.
+template <class Z>
+__device__ __forceinline__ void dft_pass_a(u64* buf, u32 log_t, const Matrix& M,
+                                           const gl::JoinConsts& J, const u64* __restrict__ r4096) {
+    constexpr u32 kStep = 16 * Z::kWaves, kLogS = Z::logP + Z::rA - 4;
+    const u32 g = (threadIdx.x & 63) >> 4, n = threadIdx.x & 15;
+    const u32 total = 1u << (log_t + kLogS);  // (at least 16: L > 256)
+    const u32 mask = (1u << log_t) - 1;
+    const u32 jn = n >> log_t;
+    u64* const lane_p = buf + (n & mask) * Z::pitch + lds_index(jn) + lds_index(g << kLogS);
+    u64 x[4], f[4];
+    auto get = [&](u32 w0, u64 (&x)[4], u64 (&f)[4]) -> u64* {
+        w0 = w0 < total ? w0 : 0;
+        const u32 j = w0 >> log_t;
+        u64* p = lane_p + ((w0 & mask) * Z::pitch + lds_index(j));
+        lds_get<kLogS>(p, x);
+        pass_twiddles<Z::rA, kLogS>(f, j + jn, g, r4096);
+        return p;
+    };
+    u32 w0 = wave_index() * 16;
+    if (w0 >= total) return;
+    u64* p = get(w0, x, f);
+#pragma unroll 1
+    for (; w0 < total; w0 += kStep) {
+        u64 x2[4], f2[4];
+        u64* p2 = get(w0 + kStep, x2, f2);
+        dft16(M, J, x);
+        gl::mul_n(x, x, f);
+        lds_put<kLogS>(p, x);
+        p = p2;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            x[v] = x2[v];
+            f[v] = f2[v];
+        }
+    }
+}
+
+// Passes B and C of the pieces of the first 2^log_t transforms: M is the matrix
+// of rB bits, at first.  From L = 256 on that is the one of pass C too; shorter
+// transforms, several to a piece of 256, take the passes one after the other (a
+// wave keeps its pieces).  Where 2^log_t transforms do not fill a piece, lanes
+// repeat its first groups (equal values go to equal places).
+template <class Z>
+__device__ __forceinline__ void dft_pieces(u64* buf, u32 log_t, Matrix& M, const u32* mats,
+                                           const u32* starts4, const gl::JoinConsts& J,
+                                           const u64* __restrict__ r4096) {
+    constexpr u32 kLogS = Z::rB, kShare = 8 - Z::logP, kPer = Z::rA;  // log2 transforms, pieces
+    const u32 g = (threadIdx.x & 63) >> 4, n = threadIdx.x & 15;
+    u32 tl = n >> kLogS;
+    const u32 j = n & ((1u << kLogS) - 1);
+    if (kShare) tl &= (1u << log_t) - 1;
+    u64* const lane_b = buf + tl * Z::pitch + lds_index(j) + lds_index(g << kLogS);  // element j + e * S
+    u64* const lane_c = buf + tl * Z::pitch + lds_index(j << 4) + g;  // group kk = j: (kk << 4) + e
+    const u32 pieces = log_t + kPer > kShare ? 1u << (log_t + kPer - kShare) : 1;
+    auto at = [&](u32 q) -> u32 {  // piece q: its first transform, its place in it
+        q = q < pieces ? q : 0;
+        return ((q >> kPer) << kShare) * Z::pitch + lds_index((q & ((1u << kPer) - 1)) << 8);
+    };
+    const u32 q0 = wave_index();
+    u64 f[4];
+    pass_twiddles<Z::rB, kLogS>(f, j, g, r4096);
+    if constexpr (Z::rB == 4) {
+        u64 x[4];
+        if (q0 < pieces) lds_get<4>(lane_b + at(q0), x);
+#pragma unroll 1
+        for (u32 q = q0; q < pieces; q += Z::kWaves) {
+            const u32 o = at(q);
+            u64 x2[4];
+            dft16(M, J, x);
+            gl::mul_n(x, x, f);
+            lds_put<4>(lane_b + o, x);
+            wave_handoff();
+            lds_get<0>(lane_c + o, x);
+            lds_get<4>(lane_b + at(q + Z::kWaves), x2);
+            dft16(M, J, x);
+            wave_handoff();
+            lds_put<4>(lane_b + o, x);  // result kk + 16 e, kk = j
+#pragma unroll
+            for (int v = 0; v < 4; v++) x[v] = x2[v];
+        }
+    } else {
+#pragma unroll 1
+        for (u32 q = q0; q < pieces; q += Z::kWaves) {
+            u64* p = lane_b + at(q);
+            u64 x[4];
+            lds_get<kLogS>(p, x);
+            dft16(M, J, x);
+            gl::mul_n(x, x, f);
+            lds_put<kLogS>(p, x);
+        }
+        M = load_matrix(mats + 3 * kDftWords, starts4);
+        wave_handoff();
+#pragma unroll 1
+        for (u32 q = q0; q < pieces; q += Z::kWaves) {
+            u64 x[4];
+            lds_get<0>(lane_c + at(q), x);
+            dft16(M, J, x);
+            wave_handoff();
+            lds_put<kLogS>(lane_b + at(q), x);  // result kk + S * e, kk = j
+        }
+    }
+}
+
+// The accumulator starts to LDS, the matrix of the first pass to registers.
+template <class Z>
+__device__ __forceinline__ Matrix dft_start(u64* buf, const u32* mats) {
+    constexpr u32 r1 = Z::rA ? Z::rA : Z::rB;
+    u32* const starts = (u32*)(buf + Z::kStarts);  // of r1 bits, of 4 bits
+    if (threadIdx.x < 128)
+        starts[threadIdx.x] = (mats + (threadIdx.x < 64 ? r1 - 1 : 3) * kDftWords + kDftStarts)[threadIdx.x & 63];
+    return load_matrix(mats + (r1 - 1) * kDftWords, starts);
+}
+// The first 2^log_t transforms of the block's LDS (elements at lds_index(i), in
+// natural order).  M as dft_start left it; it is the same
+// afterwards where all passes have 4 bits.  Starts with a barrier, ends without one.
+template <class Z>
+__device__ __forceinline__ void dft_passes(u64* buf, u32 log_t, Matrix& M, const u32* mats,
+                                           const u64* __restrict__ r4096) {
+    const gl::JoinConsts J = gl::join_consts();
+    const u32* const starts4 = (const u32*)(buf + Z::kStarts) + 64;
+    lds_barrier();
+    if constexpr (Z::rA != 0) {
+        dft_pass_a<Z>(buf, log_t, M, J, r4096);
+        if constexpr (Z::rA != 4) M = load_matrix(mats + 3 * kDftWords, starts4);
+        lds_barrier();
+    }
+    dft_pieces<Z>(buf, log_t, M, mats, starts4, J, r4096);
+}
+template <class Z>
+__device__ __forceinline__ void dft_block(u64* buf, u32 log_t, const u32* mats,
+                                          const u64* __restrict__ r4096) {
+    Matrix M = dft_start<Z>(buf, mats);
+    dft_passes<Z>(buf, log_t, M, mats, r4096);
+}
+
+// Elements tid + q * kThreads of the tile (q < 16): transform and index, the
+// thread's part (t, i) and the part of q (tq, iq), which share no bit.  TF
+// (transform-fastest): adjacent threads take adjacent transforms.
+template <class Z, bool TF>
+struct Tile {
+    u32 t, i;
+    __device__ __forceinline__ Tile()
+        : t(TF ? threadIdx.x & (Z::NT - 1) : threadIdx.x >> (LOGL())),
+          i(TF ? threadIdx.x >> Z::logNT : threadIdx.x & (Z::L - 1)) {}
+    static constexpr u32 LOGL() { return Z::logP + Z::rA; }
+    static constexpr u32 tq(u32 q) { return TF ? 0 : (q * Z::kThreads) >> LOGL(); }
+    static constexpr u32 iq(u32 q) {
+        return TF ? (q * Z::kThreads) >> Z::logNT : (q * Z::kThreads) & (Z::L - 1);
+    }
 };
 
-template <int LOGR, int NTPB, int NTILE, bool TF>
-__device__ __forceinline__ void prefetch_tw(PassTw<LOGR, NTPB, NTILE>& tw, int logL, int NT,
-                                            int logNT, int Ns, const u64* __restrict__ r4096) {
-    constexpr int R = 1 << LOGR;
-    constexpr int MAXIT = NTILE / (R * NTPB);
-    const int lp = logL - LOGR;
-    const int per = 1 << lp;
-    const int total = NT << lp;
-    const int step = 4096 / (Ns * R);
+// Global to LDS; scale(t, i, iq, x) changes four elements i + iq[v] of transform
+// t (TF) on the way.  valid: transforms of the tile that exist.
+// log_e: transforms e*C + u of each run of C * 2^log_e, C = 2^log_c, change places
+// to u * 2^log_e + e (TF).
+template <class Z, bool TF, class Scale>
+__device__ __forceinline__ void load_tile(u64* buf, const Place<const u64>& from, u32 valid,
+                                          const Scale& scale, u32 log_c = 0, u32 log_e = 0) {
+    typedef Tile<Z, TF> Ti;
+    const Ti T;
+    const u32 lane_o = 8 * from.off(T.t, T.i);
+    u64 x[Z::kPer];
+    if (valid == Z::NT) {
 #pragma unroll
-    for (int it = 0; it < MAXIT; it++) {
-        int w = threadIdx.x + it * NTPB;
-        if (w < total) {
-            int j = TF ? (w >> logNT) : (w & (per - 1));
-            int k = j & (Ns - 1);
+        for (u32 q = 0; q < Z::kPer; q++)
+            x[q] = load_at(from.base + from.off(Ti::tq(q), Ti::iq(q)), lane_o);
+    } else {
 #pragma unroll
-            for (int r = 1; r < R; r++) tw.t[it][r] = r4096[k * r * step];
+        for (u32 q = 0; q < Z::kPer; q++) {
+            x[q] = 0;
+            if (T.t + Ti::tq(q) < valid)
+                x[q] = load_at(from.base + from.off(Ti::tq(q), Ti::iq(q)), lane_o);
         }
     }
-}
-
-template <int LOGR, bool INV, int NTPB, int NTILE, bool TF, bool FROM_LDS, bool TO_LDS, class Ld,
-          class St>
-__device__ __forceinline__ void fused_pass(const LdsIO& io, int logL, int NT, int logNT, int Ns,
-                                           const PassTw<LOGR, NTPB, NTILE>& tw, const Ld& ld,
-                                           const St& st) {
-    constexpr int R = 1 << LOGR;
-    constexpr int MAXIT = NTILE / (R * NTPB);
-    static_assert(MAXIT >= 1, "radix larger than the per-thread element count");
-    const int lp = logL - LOGR;
-    const int per = 1 << lp;
-    const int total = NT << lp;
-    u64 v[MAXIT][R];
+    const u32 c1 = (1u << log_c) - 1, e1 = (1u << log_e) - 1;
+    const u32 t = (T.t & ~((1u << (log_c + log_e)) - 1)) | ((T.t & c1) << log_e) | ((T.t >> log_c) & e1);
+    u64* const lane_p = buf + t * Z::pitch + lds_index(T.i);
 #pragma unroll
-    for (int it = 0; it < MAXIT; it++) {
-        int w = threadIdx.x + it * NTPB;
-        if (w < total) {
-            int t = TF ? (w & (NT - 1)) : (w >> lp);
-            int j = TF ? (w >> logNT) : (w & (per - 1));
-            if (FROM_LDS) io.load<R>(t, j, per, v[it]);
-            else ld.template load<R>(t, j, per, v[it]);
-            if (Ns > 1) {
+    for (u32 q = 0; q < Z::kPer; q += 4) {
+        u64 y[4] = {x[q], x[q + 1], x[q + 2], x[q + 3]};
+        const u32 iq[4] = {Ti::iq(q), Ti::iq(q + 1), Ti::iq(q + 2), Ti::iq(q + 3)};
+        scale(T.t, T.i, iq, y);
 #pragma unroll
-                for (int r = 1; r < R; r++) v[it][r] = gl::mont_mul(v[it][r], tw.t[it][r]);
-            }
-            dft_reg<LOGR, INV>(v[it]);
-        }
+        for (u32 v = 0; v < 4; v++) lane_p[Ti::tq(q + v) * Z::pitch + lds_index(iq[v])] = y[v];
     }
-    if (FROM_LDS && TO_LDS) lds_barrier();  // in place: every read of the pass before any write
+}
+
+// LDS results to global; apply(x) changes four results of the thread (elements
+// 4j .. 4j + 3 in the j-th call) on the way.  Starts with the barrier after the
+// last pass.
+template <class Z, bool TF, class To, class Apply>
+__device__ __forceinline__ void store_tile(const u64* buf, const To& to, u32 valid,
+                                           const Apply& apply) {
+    typedef Tile<Z, TF> Ti;
+    const Ti T;
+    const u32 lane_o = 8 * to.off(T.t, T.i);
+    const u64* const lane_p = buf + T.t * Z::pitch + lds_index(result_place(T.i, Z::rA));
+    const bool full = valid == Z::NT;
+    lds_barrier();
 #pragma unroll
-    for (int it = 0; it < MAXIT; it++) {
-        int w = threadIdx.x + it * NTPB;
-        if (w < total) {
-            int t = TF ? (w & (NT - 1)) : (w >> lp);
-            int j = TF ? (w >> logNT) : (w & (per - 1));
-            if (TO_LDS) io.store<R>(t, j, Ns, v[it]);
-            else st.template store<R>(t, j, Ns, v[it]);
-        }
+    for (u32 q = 0; q < Z::kPer; q += 4) {
+        u64 x[4];
+#pragma unroll
+        for (u32 v = 0; v < 4; v++)
+            x[v] = lane_p[Ti::tq(q + v) * Z::pitch + lds_index(result_place(Ti::iq(q + v), Z::rA))];
+        apply(x);
+#pragma unroll
+        for (u32 v = 0; v < 4; v++)
+            if (full || T.t + Ti::tq(q + v) < valid)
+                store_at(to.base + to.off(Ti::tq(q + v), Ti::iq(q + v)), lane_o, x[v]);
     }
 }
 
-// Straight-line pass sequence for L = 2^(4Q + REM): Q radix-16 passes, then a
-// radix-2^REM pass (a radix-1 copy when L = 1).  Every radix, stride and
-// first/last role is a compile-time constant, which keeps register pressure
-// at one pass's worth.  The twiddles of pass P + 1 are loaded before the
-// barrier that ends pass P, so their latency overlaps the barrier wait.
-// The last pass maps threads by TFL, the others by TF: a row transform whose
-// output is stored transposed (adjacent rows adjacent in memory) loads its
-// rows element-fastest and stores them transform-fastest, both coalesced.
-template <int P, int NP, int Q, int REM, bool INV, int NTPB, int NTILE, bool TF, bool TFL,
-          class Ld, class St>
-__device__ __forceinline__ void fused_chain(const LdsIO& io, int NT, int logNT,
-                                            const u64* __restrict__ r4096, const Ld& ld,
-                                            const St& st,
-                                            const PassTw<(P < Q ? 4 : REM), NTPB, NTILE>& tw) {
-    constexpr int logL = 4 * Q + REM;
-    constexpr bool tf = P + 1 == NP ? TFL : TF;
-    fused_pass<(P < Q ? 4 : REM), INV, NTPB, NTILE, tf, (P > 0), (P + 1 < NP)>(
-        io, logL, NT, logNT, 1 << (4 * P), tw, ld, st);
-    if constexpr (P + 1 < NP) {
-        constexpr bool tf_next = P + 2 == NP ? TFL : TF;
-        PassTw<(P + 1 < Q ? 4 : REM), NTPB, NTILE> next;
-        prefetch_tw<(P + 1 < Q ? 4 : REM), NTPB, NTILE, tf_next>(next, logL, NT, logNT,
-                                                                1 << (4 * (P + 1)), r4096);
-        lds_barrier();
-        fused_chain<P + 1, NP, Q, REM, INV, NTPB, NTILE, TF, TFL>(io, NT, logNT, r4096, ld, st,
-                                                                  next);
+// Factors f * s^q of the thread's elements q, four at a time.
+struct FactorChain {
+    u64 f[4], s4;
+    __device__ __forceinline__ FactorChain(u64 f0, u64 s) {
+        const u64 s2 = gl::mul_lazy(s, s);
+        s4 = gl::mul_lazy(s2, s2);
+        f[0] = f0;
+        f[1] = gl::mul_lazy(f0, s);
+        f[2] = gl::mul_lazy(f0, s2);
+        f[3] = gl::mul_lazy(f[1], s2);
     }
-}
-
-template <int Q, int REM, bool INV, int NTPB, int NTILE, bool TF, bool TFL, class Ld, class St>
-__device__ __forceinline__ void fused_passes(const LdsIO& io, int NT, int logNT,
-                                             const u64* __restrict__ r4096, const Ld& ld,
-                                             const St& st) {
-    constexpr int NP = Q + ((REM != 0 || Q == 0) ? 1 : 0);
-    PassTw<(0 < Q ? 4 : REM), NTPB, NTILE> none;  // the first pass has no twiddles
-    fused_chain<0, NP, Q, REM, INV, NTPB, NTILE, TF, TFL>(io, NT, logNT, r4096, ld, st, none);
-}
-
-// LDS row pitch of a transform for the fused DFT: L + L/16 + pad, with pad
-// chosen so that the lanes of a 16-lane LDS cycle hit distinct banks under the
-// transform-fastest mapping (lane = j * NT' + t, NT' = min(NT, 16)):
-// t * pitch + j is then distinct mod 16 for t < NT', j < 16 / NT'.
-__host__ __device__ inline int fused_pitch(int L, int NT, bool tf) {
-    int ntp = NT < 16 ? NT : 16;
-    return L + (L >> 4) + (tf ? 16 / ntp : 1);
-}
-
-// NT (power of two) transforms of length 2^logL (<= 4096), NT * L <= NTILE.
-// The block's LDS (buf, NT * fused_pitch(L, NT, TF || TFL) u64) must not be in
-// use by other threads on entry.  TFL: thread mapping of the last pass.
-template <bool INV, int NTPB, int NTILE, bool TF, bool TFL = TF, class Ld, class St>
-__device__ __forceinline__ void fused_dft(u64* buf, int logL, int NT, int logNT,
-                                          const u64* __restrict__ r4096, const Ld& ld,
-                                          const St& st) {
-    const LdsIO io{buf, fused_pitch(1 << logL, NT, TF || TFL)};
-#define TVH_FUSED(q, r) \
-    fused_passes<q, r, INV, NTPB, NTILE, TF, TFL>(io, NT, logNT, r4096, ld, st)
-    switch (logL) {
-        case 0: TVH_FUSED(0, 0); break;
-        case 1: TVH_FUSED(0, 1); break;
-        case 2: TVH_FUSED(0, 2); break;
-        case 3: TVH_FUSED(0, 3); break;
-        case 4: TVH_FUSED(1, 0); break;
-        case 5: TVH_FUSED(1, 1); break;
-        case 6: TVH_FUSED(1, 2); break;
-        case 7: TVH_FUSED(1, 3); break;
-        case 8: TVH_FUSED(2, 0); break;
-        case 9: TVH_FUSED(2, 1); break;
-        case 10: TVH_FUSED(2, 2); break;
-        case 11: TVH_FUSED(2, 3); break;
-        default: TVH_FUSED(3, 0); break;  // 12
+    __device__ __forceinline__ void apply(u64 (&x)[4]) {
+        const u64 s[4] = {s4, s4, s4, s4};
+        gl::mul_n(x, x, f);
+        gl::mul_n(f, f, s);
     }
-#undef TVH_FUSED
-}
+};
 
-// w_N^(+-x) for x < N via the two-level 2^24 tables, in Montgomery form (the
-// tables hold w * 2^64 mod p): apply with gl::mont_mul.
+// w_N^(+-x) from the two-level 2^24 tables
 __device__ __forceinline__ u64 twiddle(const Roots& rt, int dir, u32 x, u32 logN) {
-    u32 y = x << (kMaxLogN - logN);
-    return gl::mont_mul(rt.lo[dir][y & 4095], rt.hi[dir][y >> 12]);
+    const u32 y = (x << (kMaxLogN - logN)) & ((1u << kMaxLogN) - 1);
+    return gl::mul_lazy(load_at(rt.lo[dir], (y & 4095) * 8), load_at(rt.hi[dir], (y >> 12) * 8));
 }
 
 // Per-block segment lookup for multi-table launches: start[i] is the first
@@ -354,146 +482,149 @@ __device__ __forceinline__ u32 find_segment(const u32* __restrict__ start, u32 n
         if (start[mid] <= blk) lo = mid;
         else hi = mid;
     }
-    return lo;
+    return __builtin_amdgcn_readfirstlane(lo);
 }
 
-// Transforms s = (c, n2): element i at src[c*sstride + (i << b) + n2].
-// Addressing in the column and row functors: every access is a block-uniform
-// base (the first transform of the block) plus a 32-bit element offset, so the
-// loads and stores take a scalar base and a vector offset and no 64-bit
-// address arithmetic runs per element.  Offsets stay below 2^32 elements: a
-// block's transforms span at most its tile's worth of columns, and the
-// in-column offset is below M <= 2^27.
-struct Step1Load {
-    const u64* src;
-    u64 sstride, s0, ntr;
-    u32 b;
-    template <int R>
-    __device__ __forceinline__ void load(int t, int j, int per, u64 (&v)[R]) const {
-        u64 s = s0 + t;
-        if (s < ntr) {
-            const u64 mask = (1ull << b) - 1;
-            const u64* base = src + (s0 >> b) * sstride + (s0 & mask);
-            const u32 o = (u32)(((s >> b) - (s0 >> b)) * sstride + (s & mask) - (s0 & mask));
-#pragma unroll
-            for (int r = 0; r < R; r++) v[r] = base[o + ((u32)(j + r * per) << b)];
-        } else {
-#pragma unroll
-            for (int r = 0; r < R; r++) v[r] = 0;
-        }
-    }
+// Where a block's transforms are: transform t0 + t of column c, `valid` of them.
+// A column of 2^log_per transforms takes max(1, 2^log_per / NT) blocks, so blocks
+// never span columns; where every column is a single transform (log_per = 0,
+// `flat`), a block takes NT columns.  In-block offsets stay below 2^31 bytes.
+struct BlockPlace {
+    u64 c;
+    u32 t0, valid;
 };
-// Step1Load with the coset scaling of a forward NTT (NttScale): element
-// i = (n1 << b) + n2 of column c enters as (x + [i < k] rand[c*k + i] *
-// delta) * base^i, base^i = p1[n1] * p2[n2] (p2[n2] is the same for all of a
-// thread's elements).  The p1 entries are loaded with the elements, so all
-// loads are in flight together; two products per element replace a separate
-// read-and-write pass over the table.
-struct Step1ScaleLoad {
-    const u64* src;
-    u64 sstride, s0, ntr;
-    u32 b;
-    NttScaleDev S;  // rand already offset to the launch's first column
-    template <int R>
-    __device__ __forceinline__ void load(int t, int j, int per, u64 (&v)[R]) const {
-        u64 s = s0 + t;
-        if (s < ntr) {
-            const u64 mask = (1ull << b) - 1;
-            const u64* base = src + (s0 >> b) * sstride + (s0 & mask);
-            const u32 o = (u32)(((s >> b) - (s0 >> b)) * sstride + (s & mask) - (s0 & mask));
-            const u32 n2 = (u32)(s & mask);
-            const u64 f2 = S.p2[n2];
-            u64 f1[R];
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                v[r] = base[o + ((u32)(j + r * per) << b)];
-                f1[r] = S.p1[j + r * per];
-            }
-            if (n2 < S.k) {  // i >= n2: only such transforms hold randomized elements
-                const u64 c = s >> b;
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const u64 i = ((u64)(j + r * per) << b) + n2;
-                    if (i < S.k) v[r] = gl::add(v[r], gl::mul(S.rand[c * S.k + i], S.delta));
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) v[r] = gl::mont_mul(gl::mont_mul(v[r], f1[r]), f2);
-        } else {
-#pragma unroll
-            for (int r = 0; r < R; r++) v[r] = 0;
-        }
+__device__ __forceinline__ BlockPlace block_place(u64 blk, u32 log_nt, u32 log_per, u64 cols, bool flat) {
+    BlockPlace B;
+    if (flat) {
+        B.c = blk << log_nt;
+        B.t0 = 0;
+        B.valid = cols - B.c < (1ull << log_nt) ? (u32)(cols - B.c) : 1u << log_nt;
+        return B;
     }
-};
-// Output k1 of transform (c, n2), times w_N^(+-n2*k1), to dst[c*dstride + E*N2*k1 + n2].
-template <bool INV>
-struct Step1Store {
-    u64* dst;
-    u64 dstride, s0, ntr;
-    u32 b, E, logN;
-    Roots rt;
-    template <int R>
-    __device__ __forceinline__ void store(int t, int j, int Ns, const u64 (&v)[R]) const {
-        u64 s = s0 + t;
-        if (s >= ntr) return;
-        const u64 mask = (1ull << b) - 1;
-        u64 n2 = s & mask;
-        u64* p0 = dst + (s0 >> b) * dstride + (s0 & mask);
-        const u32 o = (u32)(((s >> b) - (s0 >> b)) * dstride + n2 - (s0 & mask));
-        int k = j & (Ns - 1), base = (j - k) * R + k;
-        // table entries first (index 0 holds 1, so n2 = 0 or k1 = 0 needs no
-        // branch), then the products: the loads are in flight together
-        const u32 sh = kMaxLogN - logN;
-        u64 tl[R], th[R];
+    const u32 lb = log_per > log_nt ? log_per - log_nt : 0;  // log2 blocks of a column
+    B.c = blk >> lb;
+    B.t0 = ((u32)blk & ((1u << lb) - 1)) << log_nt;
+    B.valid = 1u << (log_per < log_nt ? log_per : log_nt);
+    return B;
+}
+
+// Transforms of length 2^logL <= 16: one product, no LDS; 16 / L transforms make a
+// group of the matrix product (lanes past the end: the last group again).
+// body(t, i) handles elements (t[v], i[v]), v < 4, of the lane; results have the
+// same indices.  A block takes 2^kSmallLogNT transforms.
+constexpr u32 kSmallLogNT = 8, kSmallThreads = 256;
+template <class Body>
+__device__ __forceinline__ void small_groups(u32 logL, const Body& body) {
+    const u32 g = (threadIdx.x & 63) >> 4, n = threadIdx.x & 15, sub = 4 - logL;
+    const u32 total = (1u << kSmallLogNT) >> sub;  // (at least 16)
+#pragma unroll 1
+    for (u32 w0 = wave_index() * 16; w0 < total; w0 += blockDim.x / 4) {
+        u32 t[4], i[4];
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            u32 y = (u32)(n2 * (u32)(base + r * Ns)) << sh;
-            tl[r] = rt.lo[INV][y & 4095];
-            th[r] = rt.hi[INV][y >> 12];
+        for (int v = 0; v < 4; v++) {
+            const u32 e = 4 * v + g;
+            t[v] = ((w0 + n) << sub) + (e & ((1u << sub) - 1));
+            i[v] = e >> sub;
         }
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            u32 k1 = (u32)(base + r * Ns);
-            p0[o + ((E * k1) << b)] = gl::mont_mul(v[r], gl::mont_mul(tl[r], th[r]));
-        }
+        body(t, i);
     }
-};
+}
+// The small DFT of 2^logL points (none for one point).
+__device__ __forceinline__ void small_dft(u32 logL, const u32* mats, const gl::JoinConsts& J, u64 (&x)[4]) {
+    if (!logL) return;
+    const u32* set = mats + (logL - 1) * kDftWords;
+    const Matrix M = load_matrix(set, set + kDftStarts);
+    dft16(M, J, x);
+}
 
 // ---------------------------------------------------------------- step 1
-// Transforms s = (c, n2), element n1 at src[c*sstride + N2*n1 + n2]; DFT over n1
-// (inverse if INV) -> k1; times w_N^(+-n2*k1); to dst[c*dstride + E*N2*k1 + n2].
-// Adjacent threads take adjacent transforms (adjacent n2: contiguous in HBM).
-template <bool INV, int LT = LOG_TILE>
-__device__ __forceinline__ void step1_body(const Step1Args& A, u64 blk, const Roots& rt) {
+// Transforms n2 of column c, element n1 at src[c*sstride + N2*n1 + n2]; DFT over
+// n1 (inverse if INV) -> k1; times w_N^(+-n2*k1) and the constant A.factor; to
+// dst[c*dstride + E*N2*k1 + n2].  Adjacent lanes take adjacent transforms
+// (adjacent n2: contiguous in HBM).
+// SCALED (forward): element i = (n1 << b) + n2 of column c enters as
+// (x + [i < k] rand[c*k + i] * delta) * base^i, base^i = p1[n1] * p2[n2]: p1 on
+// the way in, p2 (the same for a whole transform) with the output factor, in
+// place of a separate read-and-write pass over the table.
+template <bool INV, bool SCALED>
+struct Step1 {
+    const Step1Args& A;
+    const NttScaleDev& S;
+    const Roots& rt;
+    BlockPlace B;
+    Place<const u64> in;
+    Place<u64> out;
+    __device__ __forceinline__ Step1(const Step1Args& A_, const NttScaleDev& S_, const Roots& rt_,
+                                     u64 blk, u32 log_nt)
+        : A(A_), S(S_), rt(rt_) {
+        const u32 b = A.logN - A.a;
+        B = block_place(blk, log_nt, b, 0, false);
+        in = {A.src + B.c * A.sstride + B.t0, 0, 1, 0, 1u << b};
+        out = {A.dst + B.c * A.dstride + B.t0, 0, 1, 0, A.E << b};
+    }
+    __device__ __forceinline__ void scale(u32 t, u32 i, const u32 (&iq)[4], u64 (&x)[4]) const {
+        u64 f[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) f[v] = load_at(S.p1 + iq[v], i * 8);
+        if (S.k) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const u64 pos = ((u64)(iq[v] + i) << (A.logN - A.a)) + B.t0 + t;
+                if (pos < S.k)
+                    x[v] = gl::add(x[v], gl::mul(S.rand[B.c * S.k + pos], S.delta));
+            }
+        }
+        gl::mul_n(x, x, f);
+    }
+    __device__ __forceinline__ u64 constant(u32 t) const {  // of transform t's results
+        u64 f = A.factor;
+        if (SCALED) f = gl::mul_lazy(f, S.p2[(B.t0 + t) & ((1u << (A.logN - A.a)) - 1)]);
+        return f;
+    }
+};
+template <bool INV, bool SCALED, int LT, int LOGL>
+__device__ __forceinline__ void step1_body(const Step1Args& A, const NttScaleDev& S, u64 blk,
+                                           const Roots& rt) {
     extern __shared__ u64 lds[];
-    constexpr int NTPB = 1 << (LT - 4);
-    const u32 b = A.logN - A.a;
-    const u64 s0 = blk << A.logNT;
-    const Step1Load ld{A.src, A.sstride, s0, A.ntr, b};
-    const Step1Store<INV> st{A.dst, A.dstride, s0, A.ntr, b, A.E, A.logN, rt};
-    fused_dft<INV, NTPB, 1 << LT, true>(lds, A.a, 1 << A.logNT, A.logNT, rt.r4096[INV], ld, st);
+    typedef Shape<LT, LOGL> Z;
+    const Step1<INV, SCALED> P(A, S, rt, blk, Z::logNT);
+    load_tile<Z, true>(lds, P.in, P.B.valid,
+                       [&](u32 t, u32 i, const u32 (&iq)[4], u64 (&x)[4]) {
+                           if constexpr (SCALED) P.scale(t, i, iq, x);
+                       });
+    dft_block<Z>(lds, Z::logNT, rt.dft[INV], rt.r4096[INV]);
+    // the thread's results are k = k0 + q * L/16 of one transform
+    const Tile<Z, true> T;
+    const u32 n2 = P.B.t0 + T.t;
+    FactorChain F(gl::mul_lazy(P.constant(T.t), twiddle(rt, INV, n2 * T.i, A.logN)),
+                  twiddle(rt, INV, n2 * (Z::L / 16), A.logN));
+    store_tile<Z, true>(lds, P.out, P.B.valid, [&](u64 (&x)[4]) { F.apply(x); });
 }
-
-// Forward step 1 with the input scaling (Step1ScaleLoad).
-template <int LT>
-__device__ __forceinline__ void step1_scaled_body(const Step1Args& A, const NttScaleDev& S,
-                                                  u64 blk, const Roots& rt) {
-    extern __shared__ u64 lds[];
-    constexpr int NTPB = 1 << (LT - 4);
-    const u32 b = A.logN - A.a;
-    const u64 s0 = blk << A.logNT;
-    const Step1ScaleLoad ld{A.src, A.sstride, s0, A.ntr, b, S};
-    const Step1Store<false> st{A.dst, A.dstride, s0, A.ntr, b, A.E, A.logN, rt};
-    fused_dft<false, NTPB, 1 << LT, true>(lds, A.a, 1 << A.logNT, A.logNT, rt.r4096[0], ld, st);
+__device__ __forceinline__ void step1_small(const Step1Args& A, const NttScaleDev& S, u64 blk,
+                                            const Roots& rt) {
+    const Step1<false, true> P(A, S, rt, blk, kSmallLogNT);
+    const gl::JoinConsts J = gl::join_consts();
+    small_groups(A.a, [&](const u32 (&t)[4], const u32 (&i)[4]) {
+        u64 x[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {  // (each in a transform of its own)
+            const u32 zero[4] = {0, 0, 0, 0};
+            x[v] = t[v] < P.B.valid ? P.in.base[P.in.off(t[v], i[v])] : 0;
+            u64 y[4] = {x[v], x[v], x[v], x[v]};
+            P.scale(t[v], i[v], zero, y);
+            x[v] = y[0];
+        }
+        small_dft(A.a, rt.dft[0], J, x);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const u64 f = gl::mul_lazy(P.constant(t[v]), twiddle(rt, 0, (P.B.t0 + t[v]) * i[v], A.logN));
+            if (t[v] < P.B.valid) P.out.base[P.out.off(t[v], i[v])] = gl::mul_lazy(x[v], f);
+        }
+    });
 }
-
-
-
-// ---------------------------------------------------------------- plain NTT step 2
-// Rows s = (c, k1): n2 at src[c*N + N2*k1 + n2]; DFT over n2 -> k2 (times N^-1
-// when INV); to dst[c*N + k1 + N1*k2].
 
 // ---------------------------------------------------------------- LDE step 2
+// Randomizer term of coefficient r of column c in coset s (canonical).
 __device__ __forceinline__ u64 rand_term(const LdeArgs& A, u64 c, u32 s, u64 r) {
     const RandSpec& rs = A.rs;
     u32 limb = (u32)(c % rs.group);
@@ -509,349 +640,281 @@ __device__ __forceinline__ u64 rand_term(const LdeArgs& A, u64 c, u32 s, u64 r) 
     return gl::mul(gl::mul(*p, d), gl::pow(A.toff, r));
 }
 
-// INTT = false: the rows already hold the inverse-transformed coefficients
-// (written by k_lde_rowinv), only the coset expansion runs here.
-template <bool INTT = true>
-__device__ __forceinline__ void lde_step2_body(const LdeArgs& A, u64 blk, const Roots& rt) {
-    extern __shared__ u64 lds[];
-    u64* out = A.out;
-    const u32 a = A.a, b = A.logN - A.a, E = A.E, logNT = A.logNT;
-    const int L = 1 << b;
-    const int Lp = padded_len(L);
-    const int NT = 1 << logNT;           // rows per block
-    const u64 nrows = A.cols << a;
-    const u64 s0 = blk << logNT;
-    // load Y rows into transforms 0..NT-1 (slot s = 0)
-    for (int e = threadIdx.x; e < NT * L; e += TPB) {
-        int t = e >> b, i = e & (L - 1);
-        u64 s = s0 + t;
-        if (s < nrows) {
-            u64 c = s >> a, k1 = s & ((1ull << a) - 1);
-            lds[pidx(t, i, Lp)] = A.src[c * A.src_col_stride + k1 * A.src_row_stride + i];
-        }
-    }
-    __syncthreads();
-    if (INTT) lds_dft<true>(lds, b, NT, rt.r4096[1]);
-    // expand: transform (sl*NT + t) <- f_sl for row t
-    for (int e = threadIdx.x; e < NT * L; e += TPB) {
-        int t = e >> b, k2 = e & (L - 1);
-        u64 s = s0 + t;
-        if (s < nrows) {
-            u64 c = s >> a, k1 = s & ((1ull << a) - 1);
-            u64 C = lds[pidx(t, k2, Lp)];
-            u64 r = k1 + ((u64)k2 << a);
-            for (u32 sl = 0; sl < E; sl++) {
-                u64 v = C;
-                if (r < A.rs.k) v = gl::add(v, rand_term(A, c, sl, r));
-                lds[pidx(sl * NT + t, k2, Lp)] = gl::mont_mul(v, A.pb[(sl << b) + k2]);
-            }
-        }
-    }
-    __syncthreads();
-    lds_dft<false>(lds, b, NT * E, rt.r4096[0]);
-    // write Z_s[u1][k1] to out[E*(u1 + N2*k1) + s], contiguous over (u1, s)
-    // Output factor pa[s][k1] * w_N^(k1*u1) (N^-1 beta_s^k1 and the four-step
-    // twiddle; pb was applied before the row DFT).
-    const int logRW = b + A.logE;  // row of all cosets: E * N2 elements
-    const int RW = 1 << logRW;
-    if (RW == TILE) {
-        // one row per block (k1 uniform): thread outputs q = tid + TPB*j have
-        // the fixed coset sl = tid mod E and u1 = tid/E + (TPB/E)*j, so the
-        // factor advances by w_N^(k1*TPB/E) per j
-        u64 s = s0;
-        if (s < nrows) {
-            u64 c = s >> a, k1 = s & ((1ull << a) - 1);
-            const int sl = threadIdx.x & (E - 1);
-            const u32 u0 = threadIdx.x >> A.logE;
-            u64 f = A.pa[(sl << a) + k1];
-            if (k1 && u0) f = gl::mont_mul(f, twiddle(rt, 0, (u32)(k1 * u0), A.logN));
-            const u64 step = twiddle(rt, 0, (u32)(k1 * (TPB >> A.logE)), A.logN);
-            u64* dst = out + c * A.M + (((u64)E * k1) << b);
-#pragma unroll
-            for (int j = 0; j < TILE / TPB; j++) {
-                int q = threadIdx.x + j * TPB;
-                int u1 = q >> A.logE;
-                dst[q] = gl::mont_mul(lds[pidx(sl, u1, Lp)], f);
-                if (j + 1 < TILE / TPB) f = gl::mont_mul(f, step);
-            }
-        }
-    } else {
-        for (int e = threadIdx.x; e < NT * RW; e += TPB) {
-            int t = e >> logRW, q = e & (RW - 1);
-            int u1 = q >> A.logE, sl = q & (E - 1);
-            u64 s = s0 + t;
-            if (s < nrows) {
-                u64 c = s >> a, k1 = s & ((1ull << a) - 1);
-                u64 f = A.pa[(sl << a) + k1];
-                if (u1 && k1) f = gl::mont_mul(f, twiddle(rt, 0, (u32)(k1 * u1), A.logN));
-                out[c * A.M + (((u64)E * k1) << b) + q] =
-                    gl::mont_mul(lds[pidx(sl * NT + t, u1, Lp)], f);
-            }
-        }
-    }
-}
-
-
-// Split form of the fused row step: k_lde_rowinv inverse-transforms TILE / N2
-// rows per block with every thread busy and writes the coefficients where the
-// row was (out[c*M + E*N2*k1 + n2]); k_lde_expand then runs the coset
-// expansion of k_lde_step2 on them.  One extra read and write of N elements
-// per column buys full occupancy for the inverse row DFT, which the fused
-// kernel runs with a quarter of its threads at E = 4.
-// Rows s = (c, k1) of N2 elements at src[c*scs + k1*srs + i].
-struct RowLoad {
-    const u64* src;
-    u64 scs, srs, s0, nrows;
-    u32 a;
-    template <int R>
-    __device__ __forceinline__ void load(int t, int j, int per, u64 (&v)[R]) const {
-        u64 s = s0 + t;
-        if (s < nrows) {
-            const u64 mask = (1ull << a) - 1;
-            const u64* p = src + (s0 >> a) * scs + (s0 & mask) * srs;
-            const u32 o = (u32)(((s >> a) - (s0 >> a)) * scs + ((s & mask) - (s0 & mask)) * srs);
-#pragma unroll
-            for (int r = 0; r < R; r++) v[r] = p[o + (u32)(j + r * per)];
-        } else {
-#pragma unroll
-            for (int r = 0; r < R; r++) v[r] = 0;
-        }
-    }
-};
-// Row (c, k1) to out[c*M + E*N2*k1 + i].
-struct RowStore {
-    u64* out;
-    u64 M, s0, nrows;
-    u32 a, b, E;
-    template <int R>
-    __device__ __forceinline__ void store(int t, int j, int Ns, const u64 (&v)[R]) const {
-        u64 s = s0 + t;
-        if (s >= nrows) return;
-        const u64 mask = (1ull << a) - 1;
-        u64* p = out + (s0 >> a) * M + (((u64)E * (s0 & mask)) << b);
-        const u32 o = (u32)(((s >> a) - (s0 >> a)) * M + (((u64)E * ((s & mask) - (s0 & mask))) << b));
-        int k = j & (Ns - 1), base = (j - k) * R + k;
-#pragma unroll
-        for (int r = 0; r < R; r++) p[o + (u32)(base + r * Ns)] = v[r];
-    }
-};
-
-// Row tiles of 2^LT elements, 16 per thread (LT = 14: 1024 threads, one block
-// per CU; LT = 13: 512 threads, two blocks per CU).
-template <int LT = LOG_TILE>
-__device__ __forceinline__ void lde_rowinv_body(const LdeArgs& A, u64 blk, const Roots& rt) {
-    extern __shared__ u64 lds[];
-    const u32 b = A.logN - A.a;
-    const u64 nrows = A.cols << A.a;
-    const u64 s0 = blk << A.logNT;  // rows per block of this kernel: 2^LT / N2
-    const RowLoad ld{A.src, A.src_col_stride, A.src_row_stride, s0, nrows, A.a};
-    const RowStore st{A.out, A.M, s0, nrows, A.a, b, A.E};
-    fused_dft<true, (1 << (LT - 4)), (1 << LT), false>(lds, b, 1 << A.logNT, A.logNT,
-                                                        rt.r4096[1], ld, st);
-}
-
-
-
-// Coset transforms T = t*E + sl of row t (coefficients at src rows, written
-// by k_lde_rowinv): element k2 = (C_k2 + randomizer term) * beta_sl^(N1*k2).
-// Cosets are the fastest index, so that with the transform-fastest thread
-// mapping the E cosets of one output position are written by adjacent lanes
-// (out[E*u1 + sl] contiguous).
-struct ExpandLoad {
+// A block takes NT rows (c, k1) (NT * E * N2 = 2^LT) of Y: inverse row DFT to
+// coefficients, which stay in LDS, then all E coset transforms of each row;
+// output u1 of coset sl, times N^-1 beta_sl^k1 w_N^(k1*u1), to
+// out[c*M + E*N2*k1 + E*u1 + sl].  Coefficient k2 enters coset sl as (C +
+// randomizer term) * beta_sl^(N1*k2).  Transforms T = t*E + sl: cosets are the
+// fastest index, so the E cosets of one output position are stored by adjacent
+// lanes.  The outputs overwrite the row in place (its reads all precede the
+// block's first barrier, its writes follow its last one).
+struct Rows {
     const LdeArgs& A;
-    u64 s0, nrows;
-    template <int R>
-    __device__ __forceinline__ void load(int T, int j, int per, u64 (&v)[R]) const {
-        const u32 a = A.a, b = A.logN - A.a;
-        u32 sl = (u32)T & (A.E - 1);
-        u64 s = s0 + ((u32)T >> A.logE);
-        if (s >= nrows) {
-#pragma unroll
-            for (int r = 0; r < R; r++) v[r] = 0;
-            return;
-        }
-        const u64 mask = (1ull << a) - 1;
-        u64 c = s >> a, k1 = s & mask;
-        const u64* p = A.src + (s0 >> a) * A.src_col_stride + (s0 & mask) * A.src_row_stride;
-        const u32 o = (u32)((c - (s0 >> a)) * A.src_col_stride + (k1 - (s0 & mask)) * A.src_row_stride);
-        const u32 ob = sl << b;
-        // every load first, with no branch in between, so that they are in
-        // flight together
-        u64 f[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            v[r] = p[o + (u32)(j + r * per)];
-            f[r] = A.pb[ob + (u32)(j + r * per)];
-        }
-        // randomizer terms: element k2 of row k1 is trace row k1 + k2 * N1,
-        // which carries one when below rand_len (possible only for k1 < rand_len)
-        if (k1 < A.rs.k) {
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                u64 rr = k1 + ((u64)(j + r * per) << a);
-                if (rr < A.rs.k) v[r] = gl::add(v[r], rand_term(A, c, sl, rr));
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < R; r++) v[r] = gl::mont_mul(v[r], f[r]);
+    BlockPlace B;
+    Place<const u64> in;
+    Place<u64> out;
+    __device__ __forceinline__ Rows(const LdeArgs& A_, u64 blk, u32 log_nt) : A(A_) {
+        const u32 a = A.a, row = A.E << (A.logN - a);  // (a = 0: M = E*N2)
+        B = block_place(blk, log_nt, a, A.cols, a == 0);
+        in = {A.src + B.c * A.src_col_stride + B.t0 * A.src_row_stride, 0,
+              (u32)(a ? A.src_row_stride : A.src_col_stride), 0, 1};
+        out = {A.out + B.c * A.M + (u64)B.t0 * row, A.logE, row, 1, A.E};
     }
-};
-// Output u1 of coset sl, row k1, times N^-1 beta_sl^k1 w_N^(k1*u1), to
-// out[c*M + E*N2*k1 + E*u1 + sl].  On the last radix-16 pass of a full row the
-// thread's outputs are u1 = j + Ns*r, so the factor advances by w_N^(k1*Ns).
-struct ExpandStore {
-    const LdeArgs& A;
-    Roots rt;
-    u64 s0, nrows;
-    template <int R>
-    __device__ __forceinline__ void store(int T, int j, int Ns, const u64 (&v)[R]) const {
-        const u32 a = A.a, b = A.logN - A.a, E = A.E;
-        u32 sl = (u32)T & (E - 1);
-        u64 s = s0 + ((u32)T >> A.logE);
-        if (s >= nrows) return;
-        u64 k1 = s & ((1ull << a) - 1);
-        // row s starts at out + s*E*N2 (c*M + k1*E*N2 with M = N1*E*N2)
-        u64* dst = A.out + ((s0 * E) << b);
-        const u32 o = (u32)(((s - s0) * E) << b) + sl;
-        // (twiddle index 0 holds 1: no branch for k1 = 0 or u1 = 0)
-        u64 f = A.pa[((u64)sl << a) + k1];
-        int k = j & (Ns - 1), base = (j - k) * R + k;
-        if (R * Ns == (1 << b)) {  // base = j: u1 = j + Ns*r
-            f = gl::mont_mul(f, twiddle(rt, 0, (u32)(k1 * j), A.logN));
-            const u64 step = twiddle(rt, 0, (u32)(k1 * Ns), A.logN);
-            // factors f * step^r as C interleaved chains step^C apart: a
-            // dependency depth of about R / C products instead of R - 1
-            constexpr int C = R >= 4 ? 4 : R;
-            u64 fr[C];
-            fr[0] = f;
-            u64 stride = step;
-            if constexpr (C == 4) {
-                const u64 step2 = gl::mont_sqr(step);
-                fr[1] = gl::mont_mul(f, step);
-                fr[2] = gl::mont_mul(f, step2);
-                fr[3] = gl::mont_mul(fr[1], step2);
-                stride = gl::mont_sqr(step2);
-            } else if constexpr (C == 2) {
-                fr[1] = gl::mont_mul(f, step);
-                stride = gl::mont_sqr(step);
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                dst[o + E * (u32)(j + r * Ns)] = gl::mont_mul(v[r], fr[r % C]);
-                if (r + C < R) fr[r % C] = gl::mont_mul(fr[r % C], stride);
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                u32 u1 = (u32)(base + r * Ns);
-                u64 g = gl::mont_mul(f, twiddle(rt, 0, (u32)(k1 * u1), A.logN));
-                dst[o + E * u1] = gl::mont_mul(v[r], g);
-            }
+    // k1 of row t (a column of its own: 0)
+    __device__ __forceinline__ u32 k1(u32 t) const { return A.a ? B.t0 + t : 0; }
+    // coefficient k2 of row t with its randomizer term: element k2 of row k1 is
+    // coefficient k1 + k2 * N1, which carries one when below rand_len
+    __device__ __forceinline__ u64 randomized(u32 t, u32 sl, u32 k2, u64 x) const {
+        const u64 r = k1(t) + ((u64)k2 << A.a);
+        if (r >= A.rs.k || t >= B.valid) return x;
+        return gl::add(gl::canon(x), rand_term(A, A.a ? B.c : B.c + t, sl, r));
+    }
+    // The randomizer terms of the scaled coefficients of 2^log_rows rows in cosets
+    // s0 .. s0 + 2^log_s - 1 in LDS (transform t * 2^log_s + s): the few elements
+    // that carry one, spread over the block (a term is ~20 dependent products, which
+    // would hold up the block in the one wave that has them: 2^16 x 156 with 98
+    // randomizers, 0.57 against 0.43 ms).
+    template <class Z>
+    __device__ __forceinline__ void add_randomizers(u64* lds, u32 logL, u32 log_rows, u32 s0, u32 log_s) const {
+        const u64 first = A.a ? B.t0 : 0;  // the smallest coefficient index
+        if (first >= A.rs.k) return;
+        lds_barrier();
+        const u64 per = ((A.rs.k - 1 - first) >> A.a) + 1;
+        const u32 n = per < Z::L ? (u32)per : Z::L;
+#pragma unroll 1
+        for (u32 e = threadIdx.x; e < n << (log_rows + log_s); e += Z::kThreads) {
+            const u32 s = e & ((1u << log_s) - 1), t = (e >> log_s) & ((1u << log_rows) - 1);
+            const u32 k2 = e >> (log_s + log_rows);
+            u64* const p = lds + ((t << log_s) + s) * Z::pitch + lds_index(k2);
+            *p = gl::add(gl::canon(*p),
+                         gl::mul(randomized(t, s0 + s, k2, 0), A.pb[((s0 + s) << logL) + k2]));
         }
     }
 };
-
-// Split form, second kernel: for NT rows per block (NT * E * N2 = 2^LT), the E
-// coset transforms straight from the coefficient rows to the codewords.  The
-// outputs overwrite the coefficient row in place, so every coset of a row
-// must be computed by the block that reads the row (its reads all precede its
-// first barrier, its writes follow its last one).
-template <int LT = LOG_TILE>
-__device__ __forceinline__ void lde_expand_body(const LdeArgs& A, u64 blk, const Roots& rt) {
+template <int LT, int LOGL>
+__device__ __forceinline__ void lde_rows_body(const LdeArgs& A, u64 blk, const Roots& rt) {
     extern __shared__ u64 lds[];
-    const u32 b = A.logN - A.a;
-    const u64 nrows = A.cols << A.a;
-    const u64 s0 = blk << A.logNT;
-    const ExpandLoad ld{A, s0, nrows};
-    const ExpandStore st{A, rt, s0, nrows};
-    fused_dft<false, (1 << (LT - 4)), (1 << LT), true>(
-        lds, b, (int)(A.E << A.logNT), (int)(A.logE + A.logNT), rt.r4096[0], ld, st);
+    typedef Shape<LT, LOGL> Z;  // the E * NT coset transforms
+    typedef Tile<Z, false> Ti;  // of the rows: elements q < 16 / E
+    const Rows P(A, blk, Z::logNT - A.logE);
+    const Ti T;
+    {
+        const u32 lane_o = 8 * P.in.off(T.t, T.i);
+        u64 x[16];
+#pragma unroll
+        for (u32 q = 0; q < 16; q++)
+            if ((q << A.logE) < 16) {
+                x[q] = 0;
+                if (T.t + Ti::tq(q) < P.B.valid)
+                    x[q] = load_at(P.in.base + P.in.off(Ti::tq(q), Ti::iq(q)), lane_o);
+            }
+        u64* const lane_p = lds + T.t * Z::pitch + lds_index(T.i);
+#pragma unroll
+        for (u32 q = 0; q < 16; q++)
+            if ((q << A.logE) < 16 && T.t + Ti::tq(q) < Z::NT >> A.logE)
+                lane_p[Ti::tq(q) * Z::pitch + lds_index(Ti::iq(q))] = x[q];
+    }
+    dft_block<Z>(lds, Z::logNT - A.logE, rt.dft[1], rt.r4096[1]);
+    // coefficients to registers, then to every coset's transform: product j of
+    // the thread is element q = j / E in coset j mod E
+    {
+        u64 f[16], x[16];
+#pragma unroll
+        for (u32 j = 0; j < 16; j++) {
+            const u32 q = j >> A.logE, sl = j & (A.E - 1);
+            f[j] = load_at(A.pb + (sl << LOGL) + Ti::iq(q), T.i * 8);
+        }
+        lds_barrier();
+        const u64* const lane_p = lds + T.t * Z::pitch + lds_index(result_place(T.i, Z::rA));
+#pragma unroll
+        for (u32 j = 0; j < 16; j++) {
+            const u32 q = j >> A.logE;
+            x[j] = lane_p[Ti::tq(q) * Z::pitch + lds_index(result_place(Ti::iq(q), Z::rA))];
+        }
+        lds_barrier();
+        u64* const to = lds + (T.t << A.logE) * Z::pitch + lds_index(T.i);
+#pragma unroll
+        for (u32 j = 0; j < 16; j += 4) {
+            u64 y[4] = {x[j], x[j + 1], x[j + 2], x[j + 3]};
+            const u64 fj[4] = {f[j], f[j + 1], f[j + 2], f[j + 3]};
+            gl::mul_n(y, y, fj);
+#pragma unroll
+            for (u32 v = 0; v < 4; v++) {
+                const u32 q = (j + v) >> A.logE, sl = (j + v) & (A.E - 1);
+                to[((Ti::tq(q) << A.logE) + sl) * Z::pitch + lds_index(Ti::iq(q))] = y[v];
+            }
+        }
+    }
+    P.template add_randomizers<Z>(lds, LOGL, Z::logNT - A.logE, 0, A.logE);
+    dft_block<Z>(lds, Z::logNT, rt.dft[0], rt.r4096[0]);
+    // the thread's results are u1 = u0 + q * N2/16 of transform T: the factor
+    // advances by w_N^(k1 * N2/16)
+    const Tile<Z, true> U;
+    const u32 k1 = P.k1(U.t >> A.logE);
+    const u32 valid = P.B.valid << A.logE;
+    u64 f0 = A.pa[((U.t & (A.E - 1)) << A.a) + (k1 & ((1u << A.a) - 1))];
+    if (A.a) {
+        FactorChain F(gl::mul_lazy(f0, twiddle(rt, 0, k1 * U.i, A.logN)),
+                      twiddle(rt, 0, k1 * (Z::L / 16), A.logN));
+        store_tile<Z, true>(lds, P.out, valid, [&](u64 (&x)[4]) { F.apply(x); });
+    } else {  // a whole transform per row: no step-1 twiddle, and the codewords
+        const u64 f[4] = {f0, f0, f0, f0};
+        store_tile<Z, true>(lds, P.out, valid, [&](u64 (&x)[4]) {
+            gl::mul_n(x, x, f);
+            gl::canon_n(x);
+        });
+    }
 }
-
-
-
+// Rows of 2^12 elements: the E coset transforms one after the other, in a tile of
+// one transform, from coefficients that wait in LDS.  A block is 8 waves and 70 KB,
+// so a CU has two, each at a different place of its work (one tile of 2^14 for four
+// cosets is one block of 16 waves, which all meet at every barrier and load
+// together).  Output u1 of coset s goes to place (u1 / C) * C*E + s*C + u1 mod C of
+// its row, C = 2^log_c: runs of C elements where E*u1 + s would leave gaps of E;
+// step 3 puts them in order.
+struct CosetPlace {
+    u64* base;
+    u32 row, log_c, log_e;
+    __device__ __forceinline__ u32 off(u32 t, u32 i) const {
+        return t * row + ((i >> log_c) << (log_c + log_e)) + (i & ((1u << log_c) - 1));
+    }
+};
+constexpr u32 kCosetsLt = 12, kCosetsThreads = 512;
+__device__ __forceinline__ void lde_cosets_body(const LdeArgs& A, u64 blk, const Roots& rt) {
+    extern __shared__ u64 lds[];
+    typedef Shape<kCosetsLt, kCosetsLt, 3> Z;
+    typedef Tile<Z, false> Ti;
+    const Rows P(A, blk, Z::logNT);
+    const Ti T;
+    load_tile<Z, false>(lds, P.in, Z::NT, [](u32, u32, const u32 (&)[4], u64 (&)[4]) {});
+    dft_block<Z>(lds, Z::logNT, rt.dft[1], rt.r4096[1]);
+    u64 f[Z::kPer];
+    auto factors = [&](u32 s) {
+#pragma unroll
+        for (u32 q = 0; q < Z::kPer; q++) f[q] = load_at(A.pb + (s << kCosetsLt) + Ti::iq(q), T.i * 8);
+    };
+    factors(0);
+    lds_barrier();
+    const u64* const from = lds + T.t * Z::pitch + lds_index(result_place(T.i, Z::rA));
+    u64* const coef = lds + Z::kStarts + 64 + threadIdx.x;  // the thread's own
+    u64* const to = lds + T.t * Z::pitch + lds_index(T.i);
+#pragma unroll
+    for (u32 q = 0; q < Z::kPer; q++)
+        coef[q * Z::kThreads] = from[Ti::tq(q) * Z::pitch + lds_index(result_place(Ti::iq(q), Z::rA))];
+    const Tile<Z, true> U;
+    const u32 k1 = P.k1(U.t);
+    const u64 w0 = twiddle(rt, 0, k1 * U.i, A.logN), ws = twiddle(rt, 0, k1 * (Z::kThreads >> Z::logNT), A.logN);
+    CosetPlace out{P.out.base, P.out.ts, A.log_c, A.logE};
+    Matrix M = dft_start<Z>(lds, rt.dft[0]);
+#pragma unroll 1
+    for (u32 s = 0; s < A.E; s++) {
+        lds_barrier();
+#pragma unroll
+        for (u32 q = 0; q < Z::kPer; q += 4) {
+            u64 y[4];
+#pragma unroll
+            for (u32 v = 0; v < 4; v++) y[v] = coef[(q + v) * Z::kThreads];
+            const u64 fq[4] = {f[q], f[q + 1], f[q + 2], f[q + 3]};
+            gl::mul_n(y, y, fq);
+#pragma unroll
+            for (u32 v = 0; v < 4; v++) to[Ti::tq(q + v) * Z::pitch + lds_index(Ti::iq(q + v))] = y[v];
+        }
+        P.template add_randomizers<Z>(lds, kCosetsLt, Z::logNT, s, 0);
+        // (opaque: no twiddle is kept in registers from one coset to the next)
+        const u64* r4096 = rt.r4096[0];
+        asm("" : "+s"(r4096) : "s"(s));
+        dft_passes<Z>(lds, Z::logNT, M, rt.dft[0], r4096);
+        factors(s + 1 < A.E ? s + 1 : 0);
+        FactorChain F(gl::mul_lazy(A.pa[(s << A.a) + k1], w0), ws);
+        store_tile<Z, true>(lds, out, Z::NT, [&](u64 (&v)[4]) { F.apply(v); });
+        out.base += 1u << A.log_c;
+    }
+}
+// Rows of at most 16 elements: a group's rows stay with their lanes, every coset
+// is computed from registers (a row is read before it is overwritten).
+__device__ __forceinline__ void lde_rows_small(const LdeArgs& A, u64 blk, const Roots& rt) {
+    const u32 a = A.a, b = A.logN - a;
+    const Rows P(A, blk, kSmallLogNT);
+    const gl::JoinConsts J = gl::join_consts();
+    small_groups(b, [&](const u32 (&t)[4], const u32 (&i)[4]) {
+        u64 x[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) x[v] = t[v] < P.B.valid ? P.in.base[P.in.off(t[v], i[v])] : 0;
+        small_dft(b, rt.dft[1], J, x);
+        for (u32 sl = 0; sl < A.E; sl++) {
+            u64 y[4];
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                y[v] = gl::mul_lazy(P.randomized(t[v], sl, i[v], x[v]), A.pb[(sl << b) + i[v]]);
+            small_dft(b, rt.dft[0], J, y);
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                if (t[v] >= P.B.valid) continue;
+                u64 f = A.pa[((u64)sl << a) + P.k1(t[v])];
+                if (a) f = gl::mul_lazy(f, twiddle(rt, 0, P.k1(t[v]) * i[v], A.logN));
+                P.out.base[P.out.off((t[v] << A.logE) + sl, i[v])] = gl::canon(gl::mul_lazy(y[v], f));
+            }
+        }
+    });
+}
 
 // ---------------------------------------------------------------- LDE step 3
-// Transforms (c, q = u1*E + s), element k1 at out[c*M + E*N2*k1 + q]; forward
-// DFT over k1 -> u2, written back to out[c*M + E*N2*u2 + q].
-// Transforms (c, q) of one column: element i at out[c*M + (i << logQ) + q], in place.
-struct Step3IO {
-    u64* out;
-    u64 M, s0, ntr;
-    u32 logQ;
-    __device__ __forceinline__ u64* base() const {
-        return out + (s0 >> logQ) * M + (s0 & ((1ull << logQ) - 1));
-    }
-    __device__ __forceinline__ u32 off(u64 s) const {
-        const u64 mask = (1ull << logQ) - 1;
-        return (u32)(((s >> logQ) - (s0 >> logQ)) * M + (s & mask) - (s0 & mask));
-    }
-    template <int R>
-    __device__ __forceinline__ void load(int t, int j, int per, u64 (&v)[R]) const {
-        u64 s = s0 + t;
-        if (s < ntr) {
-            const u64* p = base();
-            const u32 o = off(s);
-#pragma unroll
-            for (int r = 0; r < R; r++) v[r] = p[o + ((u32)(j + r * per) << logQ)];
-        } else {
-#pragma unroll
-            for (int r = 0; r < R; r++) v[r] = 0;
-        }
-    }
-    template <int R>
-    __device__ __forceinline__ void store(int t, int j, int Ns, const u64 (&v)[R]) const {
-        u64 s = s0 + t;
-        if (s >= ntr) return;
-        u64* p = base();
-        const u32 o = off(s);
-        int k = j & (Ns - 1), base = (j - k) * R + k;
-#pragma unroll
-        for (int r = 0; r < R; r++) p[o + ((u32)(base + r * Ns) << logQ)] = v[r];
-    }
-};
-
-template <int LT = LOG_TILE>
+// Transforms q = u1*E + s of column c, element k1 at out[c*M + E*N2*k1 + q];
+// forward DFT over k1 -> u2, written back to out[c*M + E*N2*u2 + q] (codewords).
+template <int LT, int LOGL>
 __device__ __forceinline__ void lde_step3_body(const Step3Args& A, u64 blk, const Roots& rt) {
     extern __shared__ u64 lds[];
-    constexpr int NTPB = 1 << (LT - 4);
-    const u32 b = A.logN - A.a;
-    const u32 logQ = b + A.logE;  // transforms per column = E*N2
-    const Step3IO io{A.out, A.M, blk << A.logNT, A.cols << logQ, logQ};
-    // every input of the block is read in the first pass, before any output is
-    // written: in place is safe
-    fused_dft<false, NTPB, 1 << LT, true>(lds, A.a, 1 << A.logNT, A.logNT, rt.r4096[0], io, io);
+    typedef Shape<LT, LOGL> Z;
+    const u32 logQ = A.logN - A.a + A.logE;  // transforms per column = E*N2
+    const BlockPlace B = block_place(blk, Z::logNT, logQ, 0, false);
+    u64* col = A.out + B.c * A.M + B.t0;
+    // every input of the block is read before any output is written
+    load_tile<Z, true>(lds, Place<const u64>{col, 0, 1, 0, 1u << logQ}, B.valid,
+                       [](u32, u32, const u32 (&)[4], u64 (&)[4]) {}, A.log_c, A.log_c ? A.logE : 0);
+    dft_block<Z>(lds, Z::logNT, rt.dft[0], rt.r4096[0]);
+    store_tile<Z, true>(lds, Place<u64>{col, 0, 1, 0, 1u << logQ}, B.valid,
+                        [](u64 (&x)[4]) { gl::canon_n(x); });
 }
+// Lengths 2^5..2^12 by a compile-time constant: f(std::integral_constant<int, LOGL>).
+template <class F>
+__host__ __device__ __forceinline__ void with_length(u32 logL, const F& f) {
+    switch (logL) {
+        case 5: f(std::integral_constant<int, 5>{}); break;
+        case 6: f(std::integral_constant<int, 6>{}); break;
+        case 7: f(std::integral_constant<int, 7>{}); break;
+        case 8: f(std::integral_constant<int, 8>{}); break;
+        case 9: f(std::integral_constant<int, 9>{}); break;
+        case 10: f(std::integral_constant<int, 10>{}); break;
+        case 11: f(std::integral_constant<int, 11>{}); break;
+        default: f(std::integral_constant<int, 12>{}); break;
+    }
+}
+// A launch of `cols` columns of 2^log_per transforms (flat: one each, as
+// block_place) of length 2^logL in tiles of 2^lt elements; 2^log_e transforms of the
+// tile belong to one of a column's.
+LaunchShape launch_shape(u32 lt, u32 logL, u32 log_per, u64 cols, bool flat, u32 log_e = 0);
 
 // ---- host launchers of the kernels (one translation unit each) ----
+// lt: log2 tile (12..14); blocks, threads and LDS follow from launch_shape.
 // ntt_step1.hip
-int launch_k_step1(bool inv, u32 lt, u32 blocks, size_t lds, hipStream_t st, const Step1Args& A,
+int launch_k_step1(bool inv, u32 lt, const LaunchShape& g, hipStream_t st, const Step1Args& A,
                    const Roots& rt);
 int launch_k_step1_multi(const Step1Args* args, const u32* start, u32 nseg, u32 blocks, size_t lds,
                          hipStream_t st, const Roots& rt);
-int launch_k_step1_scaled(u32 lt, u32 blocks, size_t lds, hipStream_t st, const Step1Args& A,
+int launch_k_step1_scaled(u32 lt, const LaunchShape& g, hipStream_t st, const Step1Args& A,
                           const NttScaleDev& S, const Roots& rt);
-int launch_k_ntt_step2(bool inv, u32 lt, u32 blocks, size_t lds, hipStream_t st, const u64* src,
-                       u64* dst, u32 logN, u32 a, u64 nrows, u32 logNT, u64 ninv_m,
-                       const Roots& rt);
 int set_attributes_step1(int lds_bytes);
+// ntt_step2.hip
+int launch_k_ntt_step2(bool inv, u32 lt, const LaunchShape& g, hipStream_t st, const u64* src,
+                       u64* dst, u32 logN, u32 a, u64 cols, u64 ninv, const Roots& rt);
+int set_attributes_step2(int lds_bytes);
 // lde_rows.hip
-int launch_k_lde_rowinv(u32 lt, u32 blocks, size_t lds, hipStream_t st, const LdeArgs& A,
-                        const Roots& rt);
-int launch_k_lde_rowinv_multi(const LdeArgs* args, const u32* start, u32 nseg, u32 blocks,
-                              size_t lds, hipStream_t st, const Roots& rt);
-int launch_k_lde_step2(u32 blocks, size_t lds, hipStream_t st, const LdeArgs& A, const Roots& rt);
-int launch_k_lde_step2_multi(const LdeArgs* args, const u32* start, u32 nseg, u32 blocks,
-                             size_t lds, hipStream_t st, const Roots& rt);
+int launch_k_lde_rows(u32 lt, const LaunchShape& g, hipStream_t st, const LdeArgs& A, const Roots& rt);
+int launch_k_lde_rows_multi(u32 lt, const LdeArgs* args, const u32* start, u32 nseg, u32 blocks,
+                            size_t lds, hipStream_t st, const Roots& rt);
 int set_attributes_rows(int lds_bytes);
-// lde_expand.hip
-int launch_k_lde_expand(u32 lt, u32 blocks, size_t lds, hipStream_t st, const LdeArgs& A,
-                        const Roots& rt);
-int launch_k_lde_expand_multi(const LdeArgs* args, const u32* start, u32 nseg, u32 blocks,
-                              size_t lds, hipStream_t st, const Roots& rt);
-int set_attributes_expand(int lds_bytes);
 // lde_step3.hip
-int launch_k_lde_step3(u32 lt, u32 blocks, size_t lds, hipStream_t st, const Step3Args& A,
+int launch_k_lde_step3(u32 lt, const LaunchShape& g, hipStream_t st, const Step3Args& A,
                        const Roots& rt);
 int launch_k_lde_step3_multi(const Step3Args* args, const u32* start, u32 nseg, u32 blocks,
                              size_t lds, hipStream_t st, const Roots& rt);

@@ -1,8 +1,7 @@
 // Host side of the batched Goldilocks NTT and the coset low-degree extension:
 // kernel variants and plans, the per-shape coset tables, launches, the
 // synthetic fill and the XFE relayout.  The kernels themselves are in
-// ntt_dev.hpp (device code) and ntt_step1.hip, lde_rows.hip, lde_expand.hip,
-// lde_step3.hip (instantiations and launchers).
+// ntt_dev.hpp (device code) and ntt_step1.hip, lde_rows.hip, lde_step3.hip (instantiations and launchers).
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -17,14 +16,13 @@ namespace tvh {
 __global__ void k_lde_consts(u64* pa, u64* pb, u32 a, u32 b, u32 E, const u64* beta, u64 ninv) {
     u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
     u64 n1 = 1ull << a, n2 = 1ull << b;
-    // stored in Montgomery form (x * 2^64 mod p) for gl::mont_mul
     if (i < E * n1) {
         u64 s = i >> a, k1 = i & (n1 - 1);
-        pa[i] = gl::canon(gl::to_mont(gl::mul(ninv, gl::pow(beta[s], k1))));
+        pa[i] = gl::mul(ninv, gl::pow(beta[s], k1));
     } else if (i < E * (n1 + n2)) {
         u64 j = i - E * n1;
         u64 s = j >> b, k2 = j & (n2 - 1);
-        pb[j] = gl::canon(gl::to_mont(gl::pow(gl::pow(beta[s], n1), k2)));
+        pb[j] = gl::pow(gl::pow(beta[s], n1), k2);
     }
 }
 
@@ -66,15 +64,19 @@ static std::atomic<int> g_variant[kMaxLogN + 1][5][kWidthClasses];
 int lde_variant(u32 logN, u32 logE, u64 cols) {
     int v = (logN <= kMaxLogN && logE <= 4) ? g_variant[logN][logE][width_class(cols)].load() : 0;
     if (v) return v;
-    // default (measured on MI355X at widths 156..379, 2^12..2^21 rows): the split
-    // form with 2^12-element row tiles for 2^13..2^16 rows, 2^13-element row
-    // tiles above (column tiles 2^12, 2^13 from 2^19 rows), 2^13 for the inverse
-    // rows only at 2^12 rows, the single fused kernel below
-    if (logN >= 19) return LDE_SPLIT | (1 << 2) | LDE_ROW_HALF;
-    if (logN >= 17) return LDE_SPLIT | (2 << 2) | LDE_ROW_HALF;
-    if (logN >= 13) return LDE_SPLIT | (2 << 2) | LDE_ROW_QUARTER;
-    if (logN == 12) return LDE_SPLIT | (1 << 2) | LDE_INV_HALF;
-    return LDE_WIDE | (2 << 2);
+    // default (measured at 16, 88 and 379 columns, 2^8..2^21 rows, E = 1..16): up to
+    // 2^14 codeword elements the whole transform in the shortest tile (2^12 x 379,
+    // E = 4: 62 us, split 113; 2^10 x 379: 21 in 2^12 tiles, 31 in 2^14); above, the
+    // shortest row tile with columns of 2^8, two passes (2^18 x 379: 4.32 ms, 4.66
+    // and 4.72 in 2^13 and 2^14; 2^20 x 140: 6.3 in 2^14, 7.2 and 7.5 shorter).
+    // Column tiles of 2^13, but 2^12 where those make fewer than four blocks a CU
+    // (2^16 x 88: 197 against 204 us; 2^16 x 379: 983 against 916).
+    const u32 all = logN + logE;
+    if (all >= 26) return LDE_SPLIT | 1 << 2 | LDE_ROW_HALF;  // (refused, as these shapes ask for a = 13)
+    const u32 b = logN < 20 ? logN - 8 : 12;
+    const u32 row = all <= LOG_TILE ? all : b + logE;
+    const int col = (cols << logN) < (1ull << 23) ? 2 : 1;
+    return LDE_SPLIT | col << 2 | (row <= 12 ? LDE_ROW_QUARTER : row == 13 ? LDE_ROW_HALF : 0);
 }
 
 bool lde_variant_valid(int v) {
@@ -92,27 +94,50 @@ int set_lde_variant(u32 logN, u32 logE, int v, int wc) {
     return TVH_OK;
 }
 
+// Passes over LDS (or one product) of a transform of length 2^l.
+static u32 passes(u32 l) { return l <= 4 ? 1 : l <= 8 ? 2 : 3; }
+
+// N = N1 * N2, N1 = 2^a.  A row's E coset transforms share one tile (E * N2 <=
+// 2^row_lt, N2 <= 4096: the row step overwrites its input row in place, so a
+// row's cosets cannot be split over blocks).  Within that the split with the
+// fewest passes, then the longest rows (more contiguous bytes, fewer columns of
+// the strided step).  A column step has at least 2^5 points (shorter ones leave
+// part of the matrices idle) and, if it can, at most 2^9: longer ones leave less
+// than a cache line of adjacent columns in a 2^13 tile (2^20 x 140, E = 4, in
+// 2^13 row tiles: 7.2 ms with 2^9, 13.5 with 2^12).  Above 2^12 columns the shape
+// is refused (a > 12).
 static u32 choose_split(u32 logN, u32 E, u32 row_lt) {
-    // N2 (the contiguous row step) as long as one row tile holds all E cosets
-    // of a row (E * N2 <= 2^row_lt, N2 <= 4096: the expansion overwrites its
-    // input row in place, so a row's cosets cannot be split over blocks);
-    // N1 = N / N2 takes the strided step, whose HBM segments are (column
-    // tile) / N1 elements wide.
-    u32 logE = log2u(E);
-    u32 bmax = row_lt - logE;
+    u32 bmax = row_lt - log2u(E);
     if (bmax > 12) bmax = 12;
-    u32 b = logN < bmax ? logN : bmax;
-    return logN - b;
+    if (logN <= bmax) return 0;
+    if (logN - bmax > 12) return logN - bmax;
+    u32 best = 0, cost = ~0u;
+    for (u32 a = logN - bmax > 5 ? logN - bmax : 5; a <= 9 && a < logN; a++) {
+        const u32 c = passes(a) + passes(logN - a);
+        if (c < cost) {
+            cost = c;
+            best = a;
+        }
+    }
+    return best ? best : logN - bmax;
 }
 
-static u32 tile_log_nt(u32 logL, u32 lt = LOG_TILE) {
-    // transforms per block of a 2^lt tile: 2^lt / max(L, 32)
-    u32 l = logL < 5 ? 5 : logL;
-    return lt - l;
-}
-
-static size_t lds_bytes(u32 logL, u32 logNT) {
-    return ((size_t)padded_len(1 << logL) << logNT) * sizeof(u64);
+LaunchShape launch_shape(u32 lt, u32 logL, u32 log_per, u64 cols, bool flat, u32 log_e) {
+    LaunchShape g;
+    u32 log_nt = kSmallLogNT;
+    g.threads = kSmallThreads;
+    if (logL > 4) {
+        log_nt = lt - logL - log_e;
+        g.threads = 1u << (lt - 4);
+        // (the pitch of Shape<LT, LOGL>, then two sets of accumulator starts)
+        const u32 L = 1u << logL, lnt = lt - logL, unit = lnt >= 4 ? 1 : 16u >> lnt;
+        const size_t pitch = unit * (((L + (L >> 4) + (L >> 8) + unit) / unit) | 1);
+        g.lds = (pitch << lnt) * sizeof(u64) + 2 * 64 * sizeof(u32);
+    }
+    const u64 blocks = flat ? (cols + (1ull << log_nt) - 1) >> log_nt
+                            : cols << (log_per > log_nt ? log_per - log_nt : 0);
+    g.blocks = (u32)blocks;
+    return g;
 }
 
 struct ConstKey {
@@ -228,20 +253,13 @@ int lde_release_consts() {
 
 int prepare_lde(const u64* trace, u64 cols, u64 n, const RandSpec& rs, u64 toff, u64 goff,
                 u64 m, bool truncate, u64* out, LdePlan* P, bool batch) {
-    P->k1 = P->k3 = P->split = false;
+    P->k1 = P->k3 = false;
     P->k2_variant = lde_variant(log2u(n), log2u(m / (n ? n : 1)), cols);
-    // multi-table launches run the column and row kernels with one tile each
-    // (kBatchColLt, kBatchRowLt) for every table of the launch
     P->col_lt = batch ? kBatchColLt : LOG_TILE - ((P->k2_variant >> 2) & 3);
-    P->row_lt = batch                                  ? kBatchRowLt
-                : (P->k2_variant & LDE_ROW_QUARTER) ? LOG_TILE - 2
-                : (P->k2_variant & LDE_ROW_HALF)    ? LOG_TILE - 1
-                                                     : LOG_TILE;
-    P->inv_lt = P->row_lt < LOG_TILE                 ? P->row_lt
-                : (P->k2_variant & LDE_INV_HALF)    ? LOG_TILE - 1
-                                                     : LOG_TILE;
-    if ((P->k2_variant & 3) != LDE_SPLIT) P->row_lt = LOG_TILE;  // the wide kernel's tile
-    P->s1_blocks = P->s2_blocks = P->s3_blocks = 0;
+    P->row_lt = (P->k2_variant & LDE_ROW_QUARTER) ? LOG_TILE - 2
+                : (P->k2_variant & LDE_ROW_HALF)  ? LOG_TILE - 1
+                                                  : LOG_TILE;
+    P->g1 = P->g2 = P->g3 = LaunchShape{};
     if (cols == 0) return TVH_OK;
     if (!is_pow2(n) || !is_pow2(m)) return set_error(TVH_ERR_NOT_POW2, "lde lengths");
     if (m < n) return set_error(TVH_ERR_INVALID_ARG, "target_len < trace_len");
@@ -255,6 +273,10 @@ int prepare_lde(const u64* trace, u64 cols, u64 n, const RandSpec& rs, u64 toff,
     DeviceState* ds = current_device();
     if (!ds) return TVH_ERR_DEVICE;
     u32 a = choose_split(logN, E, P->row_lt);
+    if (batch) {  // the shapes that row tiles of 2^13 (wide form: 2^14) can take
+        const u32 bound = (P->k2_variant & 3) == LDE_SPLIT ? LOG_TILE - 1 : LOG_TILE;
+        if (a > 12 || choose_split(logN, E, bound) > 12) a = choose_split(logN, E, bound);
+    }
     u32 b = logN - a;
     if (a > 12) return set_error(TVH_ERR_UNSUPPORTED, "split");
     ConstVal cv;
@@ -265,11 +287,8 @@ int prepare_lde(const u64* trace, u64 cols, u64 n, const RandSpec& rs, u64 toff,
     // map trace -> Y, so K2 then reads the trace itself.
     P->k1 = a > 0;
     if (P->k1) {
-        u32 logNT = tile_log_nt(a, P->col_lt);
-        u64 ntr = cols << b;
-        P->s1 = Step1Args{trace, n, out, m, logN, a, E, ntr, logNT};
-        P->s1_blocks = (u32)((ntr + (1ull << logNT) - 1) >> logNT);
-        P->s1_lds = (size_t)fused_pitch(1 << a, 1 << logNT, true) * (1u << logNT) * sizeof(u64);
+        P->s1 = Step1Args{trace, n, out, m, logN, a, E, 1};
+        P->g1 = launch_shape(P->col_lt, a, b, cols, false);
     }
     // K2: INTT step 2 + coset scaling + forward step 1
     {
@@ -293,40 +312,31 @@ int prepare_lde(const u64* trace, u64 cols, u64 n, const RandSpec& rs, u64 toff,
             A.delta_n[s] = gl::mul(d, nmod);
             ws = gl::mul(ws, wE);
         }
-        u32 logNT = P->row_lt - (b + logE);  // NT * E * N2 = 2^row_lt
-        if (b < 5) logNT = P->row_lt - 5 - logE;
-        u64 nrows = cols << a;
-        if ((1ull << logNT) > nrows) logNT = log2u(nrows);
-        A.logNT = logNT;
         A.src = P->k1 ? out : trace;
         A.src_col_stride = P->k1 ? m : n;
         A.src_row_stride = P->k1 ? ((u64)E << b) : 0;
-        P->s2_blocks = (u32)((nrows + (1ull << logNT) - 1) >> logNT);
-        P->s2_lds = lds_bytes(b, logNT + logE);
-        if ((P->k2_variant & 3) == LDE_SPLIT)  // k_lde_expand: transform-fastest pitch
-            P->s2_lds = (size_t)fused_pitch(1 << b, (int)(E << logNT), true) * (E << logNT) * sizeof(u64);
-        P->split = (P->k2_variant & 3) == LDE_SPLIT;
-        if (P->split) {  // inverse rows first (TILE / N2 rows per block), then expansion from out
-            u32 li = tile_log_nt(b, P->inv_lt);
-            if ((1ull << li) > nrows) li = log2u(nrows);
-            P->inv_logNT = li;
-            P->inv_blocks = (u32)((nrows + (1ull << li) - 1) >> li);
-            P->inv_lds = lds_bytes(b, li);
-            P->s2inv = A;
-            P->s2inv.logNT = li;
-            A.src = out;
-            A.src_col_stride = m;
-            A.src_row_stride = (u64)E << b;
+        // Rows of 2^12 in four cosets: one after the other in a 2^12 tile (2^20 x 379:
+        // 12.3 ms, 12.8 in one tile of 2^14).  Shorter rows in more cosets share a
+        // tile: with two matrices to reload for each coset they are slower one by one
+        // (2^18 x 379, E = 8: LDE 10.1 against 8.4 ms; 2^19 x 264, E = 4: 7.6, 6.7).
+        A.cosets = a > 0 && b == kCosetsLt && logE >= 2 && !batch;
+        A.log_c = 0;
+        if (A.cosets) {  // whole runs to a block of step 3; 16 elements are a cache line
+            const u32 log_nt = P->col_lt - a;
+            A.log_c = log_nt > logE ? std::min(log_nt - logE, 4u) : 0;
+            P->g2 = launch_shape(kCosetsLt, b, a, cols, false);
+            P->g2.threads = kCosetsThreads;
+            P->g2.lds += sizeof(u64) << kCosetsLt;
+        } else {
+            P->row_lt = std::max(b + logE, 12u);  // the shortest tile that holds a row's cosets
+            P->g2 = launch_shape(P->row_lt, b, a, cols, a == 0, b > 4 ? logE : 0);
         }
     }
     // K3: forward step 2 for all cosets (identity when N1 = 1)
     P->k3 = a > 0;
     if (P->k3) {
-        u32 logNT = tile_log_nt(a, P->col_lt);
-        u64 ntr = cols << (b + logE);
-        P->s3 = Step3Args{out, logN, a, logE, cols, m, logNT};
-        P->s3_blocks = (u32)((ntr + (1ull << logNT) - 1) >> logNT);
-        P->s3_lds = (size_t)fused_pitch(1 << a, 1 << logNT, true) * (1u << logNT) * sizeof(u64);
+        P->s3 = Step3Args{out, logN, a, logE, P->s2.log_c, m};
+        P->g3 = launch_shape(P->col_lt, a, b + logE, cols, false);
     }
     return TVH_OK;
 }
@@ -337,16 +347,10 @@ int launch_lde(const u64* trace, u64 cols, u64 n, const RandSpec& rs, u64 toff, 
     int rc = prepare_lde(trace, cols, n, rs, toff, goff, m, truncate, out, &P, false);
     if (rc || cols == 0) return rc;
     DeviceState* ds = current_device();
-    if (P.k1 && (rc = launch_k_step1(true, P.col_lt, P.s1_blocks, P.s1_lds, st, P.s1, ds->roots)))
+    if (P.k1 && (rc = launch_k_step1(true, P.col_lt, P.g1, st, P.s1, ds->roots)))
         return rc;
-    if (P.split) {
-        if ((rc = launch_k_lde_rowinv(P.inv_lt, P.inv_blocks, P.inv_lds, st, P.s2inv, ds->roots)))
-            return rc;
-        if ((rc = launch_k_lde_expand(P.row_lt, P.s2_blocks, P.s2_lds, st, P.s2, ds->roots))) return rc;
-    } else if ((rc = launch_k_lde_step2(P.s2_blocks, P.s2_lds, st, P.s2, ds->roots))) {
-        return rc;
-    }
-    if (P.k3 && (rc = launch_k_lde_step3(P.col_lt, P.s3_blocks, P.s3_lds, st, P.s3, ds->roots)))
+    if ((rc = launch_k_lde_rows(P.row_lt, P.g2, st, P.s2, ds->roots))) return rc;
+    if (P.k3 && (rc = launch_k_lde_step3(P.col_lt, P.g3, st, P.s3, ds->roots)))
         return rc;
     return TVH_OK;
 }
@@ -360,18 +364,12 @@ int launch_lde_multi(int phase, const void* d_args, const u32* d_start, u32 nseg
         case LDE_PHASE_STEP1:
             return launch_k_step1_multi((const Step1Args*)d_args, d_start, nseg, blocks, lds, st,
                                         ds->roots);
-        case LDE_PHASE_ROWINV:
-            return launch_k_lde_rowinv_multi((const LdeArgs*)d_args, d_start, nseg, blocks, lds, st,
-                                             ds->roots);
-        case LDE_PHASE_STEP2:
-            return launch_k_lde_step2_multi((const LdeArgs*)d_args, d_start, nseg, blocks, lds, st,
-                                            ds->roots);
-        case LDE_PHASE_EXPAND:
-            return launch_k_lde_expand_multi((const LdeArgs*)d_args, d_start, nseg, blocks, lds, st,
-                                             ds->roots);
-        default:
+        case LDE_PHASE_STEP3:
             return launch_k_lde_step3_multi((const Step3Args*)d_args, d_start, nseg, blocks, lds, st,
                                             ds->roots);
+        default:
+            return launch_k_lde_rows_multi(12 + phase - LDE_PHASE_ROWS, (const LdeArgs*)d_args, d_start,
+                                           nseg, blocks, lds, st, ds->roots);
     }
 }
 
@@ -413,19 +411,21 @@ int launch_ntt_batched(const u64* src, u64* dst, u64 n, u64 cols, bool inverse, 
     if (logN > kMaxLogN) return set_error(TVH_ERR_UNSUPPORTED, "NTT size > 2^24");
     DeviceState* ds = current_device();
     if (!ds) return TVH_ERR_DEVICE;
-    // Split N = N1 * N2 and column tile, measured on MI355X: for 2^18..2^22 rows
-    // the column step takes N1 = 2^(logN/2 - 1) points in 2^13-element tiles
-    // (two 512-thread blocks per CU), 3-13 % faster than N1 = 2^(logN/2) in
-    // 2^14 tiles (2^20 x 379 forward: 5.43 against 5.80 ms).  Above 2^22 the
-    // row length is capped at 2^12, and 2^13 tiles would hold only 4 or 2
-    // columns' transforms (32 or 16 B segments), so the 2^14 tiles stay.
-    const bool big = logN >= 18 && logN <= 22;
-    u32 a = logN / 2 - (big ? 1 : 0), b = logN - a;
-    if (b > 12) {
-        b = 12;
-        a = logN - b;
-    }
-    const u32 col_lt = big ? LOG_TILE - 1 : LOG_TILE;
+    // Split N = N1 * N2 and tiles, measured on MI355X over 2^13..2^24 rows and 4 to
+    // 1000 columns.  Two passes in each step where both lengths can be at most 2^8
+    // to 2^10 (2^16 x 379: N1 = 2^8 190 us, 2^7 218), rows of 2^12 above 2^20.
+    // Column tiles of 2^13 elements (2^12 while those are fewer than four blocks a
+    // CU: 2^14 x 60 21 us, 25 in 2^13 tiles, 35 in 2^14; 2^14 beyond 2^22 rows, where
+    // 2^13 would hold 4 or 2 columns' transforms, 32 or 16 B segments).  The row
+    // step stores each block's rows transposed, in runs as long as its row count:
+    // the shortest tile that holds 8 rows (2^17 x 251: 276 us in 2^12, 296 in 2^13;
+    // 2^18 x 379: 0.98 ms in 2^14, 0.88 in 2^13, 0.92 with 4 rows in 2^12).
+    u32 a = logN <= 14 ? logN / 2 : logN <= 19 ? 8 : logN == 20 ? 10 : logN - 12;
+    // up to 2^12 rows the row step alone (2^10 x 100: 9.4 us in 2^12 tiles, 19.6 in 2^14)
+    if (logN <= 12 && !scale) a = 0;
+    const u32 b = logN - a;
+    const u32 col_lt = logN > 22 ? LOG_TILE : (cols << logN) < (1ull << 23) && a < 10 ? 12 : 13;
+    const u32 row_lt = a == 0 ? 12 : std::min(std::max(b + 3, 12u), (u32)LOG_TILE);
     NttScaleDev S{};
     if (scale) {  // p1[n1] = base^(N2 n1), p2[n2] = base^n2
         if (!scale->tables) return set_error(TVH_ERR_INVALID_ARG, "no tables for the NTT scaling");
@@ -436,59 +436,105 @@ int launch_ntt_batched(const u64* src, u64* dst, u64 n, u64 cols, bool inverse, 
             (rc = launch_pow_table(scale->tables + (1ull << a), scale->base, 1ull << b, st)))
             return rc;
     }
-    // The row step stores each block's rows transposed, in runs as long as its
-    // row count: 2^13 tiles (512 threads) win while they still hold 8 rows
-    // (N2 <= 2^10: 2^18 x 379 inverse 1.09 against 1.26 ms) and lose when
-    // they hold fewer (2^22 x 64, N2 = 2^12: 6.3 against 4.0 ms).
-    const u32 row_lt = (big && b <= 10) ? LOG_TILE - 1 : LOG_TILE;
     // step 1 writes each group of columns to the scratch, step 2 writes it back
     u64 group = scratch_elems / n;
     if (!scratch || group == 0)
         return set_error(TVH_ERR_INVALID_ARG, "NTT scratch of %llu elements < n = %llu",
                          (unsigned long long)scratch_elems, (unsigned long long)n);
     if (group > cols) group = cols;
-    u64 ninv_m = gl::mul(gl::inv(n % gl::P), gl::EPS);  // N^-1 in Montgomery form
+    u64 ninv = gl::inv(n % gl::P);
     int rc;
     for (u64 c0 = 0; c0 < cols; c0 += group) {
         u64 g = cols - c0 < group ? cols - c0 : group;
         const u64* sg = src + c0 * n;  // step 1 reads the group from src
         u64* d = dst + c0 * n;         // step 2 writes it to dst
-        {
-            u32 logNT = tile_log_nt(a, col_lt);
-            u64 ntr = g << b;
-            u64 blocks = (ntr + (1ull << logNT) - 1) >> logNT;
-            Step1Args A{sg, n, scratch, n, logN, a, 1u, ntr, logNT};
-            const size_t s1_lds =
-                (size_t)fused_pitch(1 << a, 1 << logNT, true) * (1u << logNT) * sizeof(u64);
+        const bool one_step = a == 0 && !scale;
+        if (!one_step) {
+            const LaunchShape s1 = launch_shape(col_lt, a, b, g, false);
+            Step1Args A{sg, n, scratch, n, logN, a, 1u, inverse ? ninv : 1};
             if (scale) {
                 NttScaleDev Sg = S;
                 if (Sg.rand) Sg.rand += c0 * Sg.k;  // the group's first column
-                rc = launch_k_step1_scaled(col_lt, (u32)blocks, s1_lds, st, A, Sg, ds->roots);
+                rc = launch_k_step1_scaled(col_lt, s1, st, A, Sg, ds->roots);
             } else {
-                rc = launch_k_step1(inverse, col_lt, (u32)blocks, s1_lds, st, A, ds->roots);
+                rc = launch_k_step1(inverse, col_lt, s1, st, A, ds->roots);
             }
             if (rc) return rc;
         }
-        {
-            u32 logNT = tile_log_nt(b, row_lt);
-            u64 nrows = g << a;
-            if ((1ull << logNT) > nrows) logNT = log2u(nrows);
-            u64 blocks = (nrows + (1ull << logNT) - 1) >> logNT;
-            const size_t s2_lds =
-                (size_t)fused_pitch(1 << b, 1 << logNT, true) * (1u << logNT) * sizeof(u64);
-            if ((rc = launch_k_ntt_step2(inverse, row_lt, (u32)blocks, s2_lds, st, scratch, d,
-                                         logN, a, nrows, logNT, ninv_m, ds->roots)))
-                return rc;
+        const LaunchShape s2 = launch_shape(row_lt, b, a, g, a == 0);
+        if ((rc = launch_k_ntt_step2(inverse, row_lt, s2, st, one_step ? sg : scratch, d, logN, a, g,
+                                     ninv, ds->roots)))
+            return rc;
+    }
+    return TVH_OK;
+}
+
+// ---------------------------------------------------------------- DFT matrices
+u32 dft_matrices_words() { return 4 * kDftWords; }
+
+// Coefficient 2^x (0 <= x < 192, 2^96 = -1) of byte `b` of an element's low word
+// in byte place pos < 12 (2^(8 pos), 2^96 = -1): +-2^(x mod 8) or 0.
+static int unfolded(u32 x, u32 b, u32 pos) {
+    u32 e = (x + 8 * b) % 192;
+    const int sign = e >= 96 ? -1 : 1;
+    if (e >= 96) e -= 96;
+    return e / 8 == pos ? sign * (1 << (e % 8)) : 0;
+}
+
+void build_dft_matrices(bool inverse, u32* out) {
+    typedef unsigned __int128 u128;
+    for (u32 r = 1; r <= 4; r++, out += kDftWords) {
+        const u32 sub = (1u << (4 - r)) - 1;
+        for (u32 i = 0; i < kDftWords; i++) out[i] = 0;
+        // output k from input j: w_(2^r)^(digit product) when their low bits agree
+        auto power = [&](u32 k, u32 j) -> u32 {
+            const u32 kj = ((k >> (4 - r)) * (j >> (4 - r))) % (1u << r);
+            const u32 x = (39 * (64 >> r) * kj) % 192;  // w_64 = 2^39
+            return inverse ? (192 - x) % 192 : x;
+        };
+        for (u32 k = 0; k < 16; k++) {
+            // what the products leave out of output k: sum over j, b of
+            // coefficient * 128 per byte, and of Q_s for -x = ~x + 1
+            u64 total = 0, q_sum[4] = {0, 0, 0, 0};
+            for (u32 j = 0; j < 16; j++) {
+                if ((k & sub) != (j & sub)) continue;
+                const u32 x = power(k, j);
+                total = gl::add(total, gl::mul(gl::pow2_mod_p(x), kSignBits * 0x100000001ull));
+                // lane 16 (j mod 4) + row of k (k = 4 (row mod 4) + row / 4), register j / 4
+                const u32 at = (16 * (j & 3) + 4 * (k & 3) + (k >> 2)) * 4 + (j >> 2);
+                for (u32 s = 0; s < 4; s++)
+                    for (u32 b = 0; b < 4; b++) {
+                        const int u0 = unfolded(x, b, s), u4 = unfolded(x, b, s + 4),
+                                  u8 = unfolded(x, b, s + 8);
+                        const int p = u0 - u8, q = u4 + u8, pq = u0 + u4;
+                        out[s * 256 + at] |= (u32)(p & 255) << (8 * b);
+                        out[(4 + s) * 256 + at] |= (u32)(q & 255) << (8 * b);
+                        out[(8 + s) * 256 + at] |= (u32)(pq & 255) << (8 * b);
+                        q_sum[s] = gl::add(q_sum[s], q < 0 ? gl::P - (u64)-q : (u64)q);
+                    }
+            }
+            for (u32 s = 0; s < 4; s++) total = gl::add(total, gl::mul(q_sum[s], 1ull << (8 * s)));
+            const u128 bias = (u128)kDftBias * (1 + (1ull << 16) + (1ull << 32) + (1ull << 48));
+            const u64 c = gl::sub(total, (u64)(bias % gl::P));
+            for (u32 q = 0; q < 4; q++)  // start[q][g = k mod 4][v = k / 4]
+                out[kDftStarts + (q * 4 + (k & 3)) * 4 + (k >> 2)] =
+                    kDftBias + (u32)((c >> (16 * q)) & 0xFFFF);
         }
     }
+}
+
+int set_lds_attribute(const std::vector<const void*>& kernels, int bytes) {
+    for (const void* f : kernels)
+        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)
+            return set_error(TVH_ERR_DEVICE, "LDS attribute");
     return TVH_OK;
 }
 
 int ntt_set_attributes() {
     const int bytes = 150 * 1024;
     int rc;
-    if ((rc = set_attributes_step1(bytes)) || (rc = set_attributes_rows(bytes)) ||
-        (rc = set_attributes_expand(bytes)) || (rc = set_attributes_step3(bytes)))
+    if ((rc = set_attributes_step1(bytes)) || (rc = set_attributes_step2(bytes)) ||
+        (rc = set_attributes_rows(bytes)) || (rc = set_attributes_step3(bytes)))
         return rc;
     return TVH_OK;
 }

@@ -1,0 +1,115 @@
+// Row step of the batched NTT: kernels and their launchers.
+#include "ntt_dev.hpp"
+
+namespace tvh {
+
+// Rows k1 of column c, N2 = 2^b elements at src[c*N + N2*k1 + n2] (the column
+// step's output); DFT over n2 -> k2; element k2 to dst[c*N + k1 + N1*k2].  The
+// rows are read element-fastest and stored transform-fastest, so adjacent lanes
+// write adjacent k1 (runs as long as the block's row count).  COLS: without a
+// column step (a = 0) the rows are the columns, read and written alike, in place
+// too, and take the factor N^-1 of an inverse transform here.
+template <bool INV, bool COLS>
+struct RowStep {
+    BlockPlace B;
+    Place<const u64> in;
+    Place<u64> out;
+    u64 ninv;
+    __device__ __forceinline__ RowStep(const u64* src, u64* dst, u32 logN, u32 a, u64 cols, u64 ninv_,
+                                       u64 blk, u32 log_nt)
+        : ninv(ninv_) {
+        const u32 b = logN - a;
+        B = block_place(blk, log_nt, a, cols, COLS);
+        in = {src + (B.c << logN) + ((u64)B.t0 << b), 0, 1u << b, 0, 1};
+        out = {dst + (B.c << logN) + B.t0, 0, COLS ? 1u << logN : 1u, 0, 1u << a};
+    }
+    __device__ __forceinline__ void finish(u64 (&x)[4]) const {
+        if (INV && COLS) {
+            const u64 f[4] = {ninv, ninv, ninv, ninv};
+            gl::mul_n(x, x, f);
+        }
+        gl::canon_n(x);
+    }
+};
+
+template <bool INV, bool COLS, int LT, int LOGL>
+__global__ void __launch_bounds__(1 << (LT - 4), 4) k_ntt_step2(const u64* src, u64* dst, u32 logN,
+                                                                u32 a, u64 cols, u64 ninv, Roots rt) {
+    extern __shared__ u64 lds[];
+    typedef Shape<LT, LOGL> Z;
+    const RowStep<INV, COLS> P(src, dst, logN, a, cols, ninv, blockIdx.x, Z::logNT);
+    load_tile<Z, false>(lds, P.in, P.B.valid, [](u32, u32, const u32 (&)[4], u64 (&)[4]) {});
+    dft_block<Z>(lds, Z::logNT, rt.dft[INV], rt.r4096[INV]);
+    store_tile<Z, !COLS>(lds, P.out, P.B.valid, [&](u64 (&x)[4]) { P.finish(x); });
+}
+// rows of at most 16 elements
+template <bool INV, bool COLS>
+__global__ void __launch_bounds__(kSmallThreads) k_ntt_step2_small(const u64* src, u64* dst, u32 logN,
+                                                                   u32 a, u64 cols, u64 ninv, Roots rt) {
+    const RowStep<INV, COLS> P(src, dst, logN, a, cols, ninv, blockIdx.x, kSmallLogNT);
+    const gl::JoinConsts J = gl::join_consts();
+    small_groups(logN - a, [&](const u32 (&t)[4], const u32 (&i)[4]) {
+        u64 x[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) x[v] = t[v] < P.B.valid ? P.in.base[P.in.off(t[v], i[v])] : 0;
+        small_dft(logN - a, rt.dft[INV], J, x);
+        P.finish(x);
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (t[v] < P.B.valid) P.out.base[P.out.off(t[v], i[v])] = x[v];
+    });
+}
+
+template <bool INV, bool COLS>
+static void launch_step2(u32 lt, const LaunchShape& g, hipStream_t st, const u64* src, u64* dst,
+                         u32 logN, u32 a, u64 cols, u64 ninv, const Roots& rt) {
+    const dim3 blocks(g.blocks), tpb(g.threads);
+    if (logN - a <= 4) {
+        hipLaunchKernelGGL((k_ntt_step2_small<INV, COLS>), blocks, tpb, 0, st, src, dst, logN, a, cols,
+                           ninv, rt);
+        return;
+    }
+    with_length(logN - a, [&](auto l) {
+        constexpr int L = decltype(l)::value;
+#define TVH_STEP2(T)                                                                                \
+    hipLaunchKernelGGL((k_ntt_step2<INV, COLS, T, L>), blocks, tpb, g.lds, st, src, dst, logN, a, cols, \
+                       ninv, rt)
+        if (lt == 12) TVH_STEP2(12);
+        else if (lt == 13) TVH_STEP2(13);
+        else TVH_STEP2(14);
+#undef TVH_STEP2
+    });
+}
+
+int launch_k_ntt_step2(bool inv, u32 lt, const LaunchShape& g, hipStream_t st, const u64* src,
+                       u64* dst, u32 logN, u32 a, u64 cols, u64 ninv, const Roots& rt) {
+    if (a == 0) {
+        if (inv) launch_step2<true, true>(lt, g, st, src, dst, logN, a, cols, ninv, rt);
+        else launch_step2<false, true>(lt, g, st, src, dst, logN, a, cols, ninv, rt);
+    } else {
+        if (inv) launch_step2<true, false>(lt, g, st, src, dst, logN, a, cols, ninv, rt);
+        else launch_step2<false, false>(lt, g, st, src, dst, logN, a, cols, ninv, rt);
+    }
+    return check_launch();
+}
+
+template <bool INV, bool COLS>
+static void step2_kernels(std::vector<const void*>& fns) {
+    for (u32 l = 5; l <= 12; l++)
+        with_length(l, [&](auto c) {
+            constexpr int L = decltype(c)::value;
+            fns.insert(fns.end(), {(const void*)k_ntt_step2<INV, COLS, 12, L>,
+                                   (const void*)k_ntt_step2<INV, COLS, 13, L>,
+                                   (const void*)k_ntt_step2<INV, COLS, 14, L>});
+        });
+}
+int set_attributes_step2(int bytes) {
+    std::vector<const void*> fns;
+    step2_kernels<true, true>(fns);
+    step2_kernels<true, false>(fns);
+    step2_kernels<false, true>(fns);
+    step2_kernels<false, false>(fns);
+    return set_lds_attribute(fns, bytes);
+}
+
+}  // namespace tvh

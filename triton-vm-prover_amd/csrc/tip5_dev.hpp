@@ -260,9 +260,9 @@ __device__ __forceinline__ void round_m(u64 s[WORDS], int r, const Wave& W) {
     bool carry[WORDS];
 #pragma unroll
     for (int v = 0; v < WORDS; v++)
-        s[v] = gl::join_bytes_rare(W.J, (u32)y[0][v], (u32)y[1][v], (u32)y[2][v], (u32)y[3][v],
-                                   (u32)y[4][v], (u32)y[5][v], (u32)y[6][v], (u32)y[7][v],
-                                   carry[v]);
+        s[v] = gl::join_rare(
+            W.J, gl::join_half(W.J, (u32)y[0][v], (u32)y[1][v], (u32)y[2][v], (u32)y[3][v]),
+            gl::join_half(W.J, (u32)y[4][v], (u32)y[5][v], (u32)y[6][v], (u32)y[7][v]), carry[v]);
     if (__builtin_expect(carry[0] | carry[1] | carry[2] | carry[3], 0)) {
 #pragma unroll
         for (int v = 0; v < WORDS; v++)

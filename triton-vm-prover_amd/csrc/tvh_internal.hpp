@@ -21,13 +21,12 @@ using gl::u64;
 //   r4096[d][e] = w_4096^(+-e)               e < 4096
 //   lo[d][e]    = w^(+-e), hi[d][e] = w^(+-4096 e)   e < 4096
 // so w_N^x = lo[x & 4095] * hi[x >> 12] for x < 2^24 after scaling x by 2^24/N.
-// All entries are stored in Montgomery form (w * 2^64 mod p, canonical) and
-// applied with gl::mont_mul, which returns the canonical product for a
-// canonical operand.
+// dft[d]: the matrix sets of the 2-, 4-, 8- and 16-point DFTs (ntt_dev.hpp).
 struct Roots {
     const u64* r4096[2];
     const u64* lo[2];
     const u64* hi[2];
+    const u32* dft[2];
 };
 
 constexpr u32 kMaxLogN = 24;
@@ -90,7 +89,7 @@ struct NttScale {
 constexpr u64 kNttScaleTableElems = 8192;  // N1 + N2 <= 2 * 4096
 // What the column step reads (NttScale with the launch's tables filled in):
 // element i = n1 * N2 + n2 takes base^i = p1[n1] * p2[n2], p1[n1] = base^(N2 n1),
-// p2[n2] = base^n2 (Montgomery form).
+// p2[n2] = base^n2.
 struct NttScaleDev {
     const u64* p1;
     const u64* p2;
@@ -133,37 +132,34 @@ struct Step1Args {
     u64* dst;
     u64 dstride;
     u32 logN, a, E;
-    u64 ntr;
-    u32 logNT;
+    u64 factor;  // of every output (N^-1 of an inverse NTT; 1)
 };
 struct Step3Args {
     u64* out;
     u32 logN, a, logE;
-    u64 cols, M;
-    u32 logNT;
+    u32 log_c;  // order of its input (LdeArgs)
+    u64 M;
 };
 struct LdeArgs {
     u64* out;
     u32 logN, a, E, logE;
+    // cosets: one after the other (lde_cosets_body), in runs of 2^log_c outputs
+    u32 cosets, log_c;
     u64 cols, M;
     const u64* src;    // rows of step 2: src[c*src_col_stride + k1*src_row_stride + n2]
     u64 src_col_stride, src_row_stride;
-    const u64* pa;     // pa[s*N1 + k1] = N^-1 * beta_s^k1      (Montgomery form)
-    const u64* pb;     // pb[s*N2 + k2] = beta_s^(N1*k2)         (Montgomery form)
+    const u64* pa;     // pa[s*N1 + k1] = N^-1 * beta_s^k1
+    const u64* pb;     // pb[s*N2 + k2] = beta_s^(N1*k2)
     u64 delta_n[16];   // (g^N w_E^s - o^N) * N  (or -o^N * N when truncating with E = 1)
     u64 toff;          // o
     RandSpec rs;
-    u32 logNT;
 };
-// LDE kernel variant: bits 0-1 the form of the fused row step (LDE_WIDE: one
-// kernel, all E cosets of a row in one 1024-thread LDS tile; LDE_SPLIT: the
-// inverse row DFTs as a kernel of their own, then the expansion); bits 2-3 the
-// column kernels' tile, 2^(14 - code) elements with 16 per thread; bit 4
-// (LDE_SPLIT only) halves the row kernels' tile to 2^13 elements (512 threads,
-// two blocks per CU), which also halves the row length N2 when E * N2 would
-// not fit (all cosets of a row stay in one block); bit 5 (LDE_SPLIT only, not
-// with bit 4) gives only the inverse row kernel the 2^13 tile; bit 6 (LDE_SPLIT
-// only, alone) gives both row kernels 2^12-element tiles (256 threads).
+// LDE kernel variant: bits 0-1 the form (LDE_WIDE, LDE_SPLIT: the codes of two
+// row steps that are one now), bits 2-3 the column kernels' tile, 2^(14 - code)
+// elements with 16 per thread; bits 4 and 6 (LDE_SPLIT only, one of them) bound
+// the row kernel's tile by 2^13 or 2^12 elements in place of 2^14, and with it
+// the row length N2 (E * N2 elements share a tile); bit 5 (LDE_SPLIT only, alone)
+// has no effect.
 enum LdeVariant {
     LDE_AUTO = 0,
     LDE_WIDE = 1,
@@ -182,24 +178,22 @@ bool lde_variant_valid(int v);
 // v = LDE_AUTO restores the default; wc < 0 sets every width class
 int set_lde_variant(u32 logN, u32 logE, int v, int wc = -1);
 
+// Blocks, threads and LDS of a launch of transforms in tiles of 2^lt elements.
+struct LaunchShape {
+    u32 blocks = 0, threads = 0;
+    size_t lds = 0;
+};
 struct LdePlan {
     bool k1, k3;
-    int k2_variant;  // full variant code (form | tile << 2 | LDE_ROW_HALF)
-    bool split;      // LDE_SPLIT: s2inv (k_lde_rowinv) runs before s2 (k_lde_expand)
-    LdeArgs s2inv;
-    u32 inv_logNT, inv_blocks;  // s2inv.logNT == inv_logNT
-    size_t inv_lds;
+    int k2_variant;  // full variant code
     u32 col_lt;      // log2 tile of the column kernels (K1, K3)
-    u32 row_lt;      // log2 tile of the row kernels (k_lde_expand; the split's bound)
-    u32 inv_lt;      // log2 tile of k_lde_rowinv
+    u32 row_lt;      // log2 tile of the row kernel (bounds the row length)
     Step1Args s1;
     LdeArgs s2;
     Step3Args s3;
-    u32 s1_blocks, s2_blocks, s3_blocks;
-    size_t s1_lds, s2_lds, s3_lds;
+    LaunchShape g1, g2, g3;
 };
-// batch = true plans the column and row kernels with the multi-table tiles
-// (kBatchColLt, kBatchRowLt; the wide form keeps its full tile).
+// batch = true plans the column kernels with the multi-table tile (kBatchColLt).
 int prepare_lde(const u64* trace, u64 cols, u64 n, const RandSpec& rs, u64 toff, u64 goff,
                 u64 m, bool truncate, u64* out, LdePlan* plan, bool batch);
 // Builds (once) the coset tables every LDE variant of this shape and these
@@ -210,14 +204,11 @@ int lde_release_consts();
 // Phases of the multi-table LDE, in launch order.
 enum LdePhase {
     LDE_PHASE_STEP1 = 0,   // k_step1_multi<true>
-    LDE_PHASE_ROWINV = 1,  // k_lde_rowinv_multi (split-form tables)
-    LDE_PHASE_STEP2 = 2,   // k_lde_step2_multi (wide-form tables)
-    LDE_PHASE_EXPAND = 3,  // k_lde_expand_multi (split-form tables)
+    LDE_PHASE_ROWS = 1,    // k_lde_rows_multi with tiles of 2^12, then 2^13 and 2^14
     LDE_PHASE_STEP3 = 4,   // k_lde_step3_multi
     LDE_PHASES = 5
 };
 constexpr u32 kBatchColLt = 13;  // column-kernel tile of multi-table launches
-constexpr u32 kBatchRowLt = 13;  // row-kernel tile of multi-table launches (measured best over 2^12..2^14)
 int launch_lde_multi(int phase, const void* d_args, const u32* d_start, u32 nseg, u32 blocks,
                      size_t lds, hipStream_t st);
 int launch_fill_uniform(u64* d, u64 count, u64 seed, hipStream_t st);
@@ -230,7 +221,7 @@ int launch_xfe_interleave(const u64* src, u64* dst, u64 cols, u64 len, bool to_l
 u64 scale_table_elems(u64 n);
 int launch_scale_table(const u64* x, u64* y, u64 n, u64 cols, u64 base, const u64* rand, u64 k,
                        u64 delta, u64* tables, hipStream_t st);
-// t[i] = base^i for i < count, Montgomery form
+// t[i] = base^i for i < count
 int launch_pow_table(u64* t, u64 base, u64 count, hipStream_t st);
 // leaves[(j * num_cosets + coset) * 5 + e] = dig[j * 5 + e], j < len
 int launch_scatter_digests(const u64* dig, u64* leaves, u64 len, u64 coset, u64 num_cosets,
@@ -286,5 +277,9 @@ int launch_merkle_levels(u64* tree, u64 n, int layout, hipStream_t st);
 int launch_gather_heap(const u64* tree, u64 n, int layout, const u64* idx, u64 count, u64* out,
                        hipStream_t st);
 int ntt_set_attributes();
+int set_lds_attribute(const std::vector<const void*>& kernels, int bytes);
+// Matrix sets of the small DFTs of one direction (kDftSetsWords u32), for Roots::dft.
+void build_dft_matrices(bool inverse, u32* out);
+u32 dft_matrices_words();
 
 }  // namespace tvh

@@ -56,3 +56,25 @@ def test_merkle_edge_leaves(T, oracle, logn):
     T.lib.merkle_tree(T.dev(leaves), tree, n, 0)
     want = oracle.merkle_level_order(leaves.reshape(n, 5))
     assert np.array_equal(T.host(tree).reshape(-1), np.asarray(want).reshape(-1))
+
+
+@pytest.mark.parametrize("rows", [3, 4, 5, 16383, 16384, 16385])
+def test_hash_rows_few_and_many(T, oracle, rows):
+    """Four sponges to a wave up to 2^14 rows, 16 above: partial waves of both."""
+    cols = 21
+    t = edge_words(rows, rows * cols)
+    dg = T.empty(rows * 5)
+    T.lib.hash_bfield_rows(T.dev(t), rows, cols, dg)
+    assert np.array_equal(T.host(dg, rows * 5).reshape(rows, 5), oracle.hash_rows(t, rows, cols))
+
+
+@pytest.mark.parametrize("logn", [1, 3, 14, 15])
+def test_merkle_few_parents(T, oracle, logn):
+    """Levels of up to 2^14 parents, four to a wave; 2^15 leaves are the largest
+    tree of only such levels."""
+    n = 1 << logn
+    leaves = edge_words(40 + logn, 5 * n)
+    tree = T.empty(5 * (2 * n - 1))
+    T.lib.merkle_tree(T.dev(leaves), tree, n, 0)
+    want = oracle.merkle_level_order(leaves.reshape(n, 5))
+    assert np.array_equal(T.host(tree).reshape(-1), np.asarray(want).reshape(-1))

@@ -248,9 +248,14 @@ __host__ __device__ __forceinline__ u64 mul(u64 a, u64 b) { return canon_raw(mul
 // no word for the carry out of v_mad_u64_u32 and the compiler turns sums with
 // two carries in into selects.  gfx950 wants two wait states between a VALU
 // write of an SGPR and a VALU read of it, and the compiler does not look into
-// asm: the forms take N >= 3 values at a time and do each step for all of them,
-// so that two other instructions lie between (volatile asm keeps its order).
+// asm: the forms take N values at a time and do each step for all of them, so
+// that for N >= 3 two other instructions lie between (volatile asm keeps its
+// order); fewer values take s_nops.
 typedef u64 mask;  // a bit per lane, uniform
+template <int N>
+__device__ __forceinline__ void carry_wait() {
+    if constexpr (N < 3) asm volatile("s_nop %0" ::"n"(N < 3 ? 2 - N : 0));
+}
 
 __device__ __forceinline__ bool in_mask(mask m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
@@ -288,14 +293,15 @@ __device__ __forceinline__ void note_rare(mask& bad, int, mask& k, mask c) {
 template <int N, class Bad>
 __device__ __forceinline__ void fold128_rare(u64 (&r)[N], const u64 (&l)[N], const u32 (&h0)[N],
                                              const u32 (&h1)[N], Bad& bad) {
-    static_assert(N >= 3, "wait states");
     u64 u[N];
     u32 r0[N], r1[N];
     mask c[N], k[N], none;
 #pragma unroll
     for (int i = 0; i < N; i++) GL_MAD_EPS_CO(u[i], c[i], h0[i], l[i]);
+    carry_wait<N>();
 #pragma unroll
     for (int i = 0; i < N; i++) GL_SUBB_CO(r0[i], k[i], (u32)u[i], h1[i], c[i]);  // - h1 - c
+    carry_wait<N>();
 #pragma unroll
     for (int i = 0; i < N; i++) GL_SUBB_0(r1[i], k[i], (u32)(u[i] >> 32), k[i]);
 #pragma unroll
@@ -314,7 +320,6 @@ __device__ __forceinline__ void fold128_rare(u64 (&r)[N], const u64 (&l)[N], con
 // cycles (hashing 2^22 rows of 379: 19.9 -> 18.6 ms, LDE 2^20 x 379: 19.1 -> 18.8).
 template <int N, class Bad>
 __device__ __forceinline__ void mul_rare(u64 (&r)[N], const u64 (&a)[N], const u64 (&b)[N], Bad& bad) {
-    static_assert(N >= 3, "wait states");
     u64 l[N], q[N];
     u32 h0[N], h1[N];
     mask cm[N], none;
@@ -328,6 +333,7 @@ __device__ __forceinline__ void mul_rare(u64 (&r)[N], const u64 (&a)[N], const u
         l[i] = mk64((u32)p, (u32)y);
         h0[i] = (u32)q[i];
     }
+    carry_wait<N>();
 #pragma unroll
     for (int i = 0; i < N; i++) GL_ADDC_0(h1[i], none, (u32)(q[i] >> 32), cm[i]);
     fold128_rare(r, l, h0, h1, bad);

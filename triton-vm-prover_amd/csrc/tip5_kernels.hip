@@ -1,7 +1,7 @@
 // Tip5 hashing kernels: row digests, pair hashing, Merkle trees, auth paths.
 //
-// Every kernel runs 16 sponges per wave (tip5_dev.hpp): lane 16g + n holds
-// words 4v + g (v = 0..3) of sponge n.  State words 0..9 are the rate.
+// The kernels run 16 sponges per wave, or four where that would leave SIMDs
+// without a wave (tip5_dev.hpp).  State words 0..9 are the rate.
 //
 // Row hashing restates Tip5::hash_varlen (src/hash/tip5.cpp:246-282) over a
 // column-major table (element (r, c) at c*rows + r, the reference GPU layout,
@@ -13,8 +13,9 @@
 // Node (level l, index i) of an n-leaf tree lives at base(l) + i with
 //   level order (merkle_kernel.cu:60-102): base(l) = 2n - (2n >> l)
 //   heap        (merkle_tree.cpp:12-33):   base(l) = n >> l      (1-indexed)
-// Large levels take a launch each; below them a block hashes up to 256 parents,
-// keeps them in LDS and continues to their subtree root.
+// Large levels take a launch each; below them a block hashes up to 64 parents (256
+// in launches over many trees), keeps them in LDS and continues to their subtree
+// root.
 #include "tvh_internal.hpp"
 
 namespace tvh {
@@ -23,11 +24,13 @@ using gl::u32;
 using gl::u64;
 
 // Sponge states are kept in Montgomery form (tip5_dev.hpp); digests leave
-// canonical.  Word 4v + g < 5 of the lane's sponge goes to dst[4v + g].
-__device__ __forceinline__ void store_digest(u64* dst, const u64 s[tip5::WORDS],
-                                             const tip5::Wave& W) {
-    dst[W.g] = tip5::from_m(s[0]);
-    if (W.g == 0) dst[4] = tip5::from_m(s[1]);
+// canonical.  The kernels are templates over the wave's form Wv: 16 sponges
+// (tip5::Wave) or four (tip5::QuadWave).
+template <class Wv>
+__device__ __forceinline__ void store_digest(u64* dst, const u64 (&s)[Wv::kWords], const Wv& W) {
+#pragma unroll
+    for (int v = 0; v < Wv::kWords; v++)
+        if (W.word(v) < (u32)tip5::DIGEST) dst[W.word(v)] = tip5::from_m(s[v]);
 }
 
 // Segment lookup for multi-table launches (start[nseg] = total blocks).
@@ -41,62 +44,87 @@ __device__ __forceinline__ u32 find_seg(const u32* __restrict__ start, u32 nseg,
     return lo;
 }
 
-// First sponge of the wave: block blk of kSpongesPerBlock sponges.
+// First sponge of the wave in block blk.
+template <class Wv>
 __device__ __forceinline__ u64 wave_first(u64 blk) {
-    return blk * kSpongesPerBlock + (threadIdx.x >> 6) * tip5::GROUP;
+    return (blk * (blockDim.x >> 6) + (threadIdx.x >> 6)) * Wv::kSponges;
 }
 
-// Absorbs one full rate block: elem(i) is element i (0..9), canonical.
-template <class F>
-__device__ __forceinline__ void absorb(u64 s[tip5::WORDS], const tip5::Wave& W, const F& elem) {
-    const u64 x[3] = {elem(W.g), elem(4 + W.g), W.g < 2 ? elem(8 + W.g) : 0};
-    u64 m[3];
-    gl::mask bad = 0;
-    gl::to_mont_rare(m, x, bad);
-    if (__builtin_expect(gl::in_mask(bad), 0)) {
+// The lane's elements of a full rate block: elem(i) is element i (0..9), canonical.
+template <class Wv>
+constexpr int kRateWords = Wv::kWords < 3 ? Wv::kWords : 3;
+template <class Wv, class F>
+__device__ __forceinline__ void rate_elements(u64 (&x)[kRateWords<Wv>], const Wv& W, const F& elem) {
 #pragma unroll
-        for (int i = 0; i < 3; i++) m[i] = tip5::to_m(x[i]);
+    for (int v = 0; v < kRateWords<Wv>; v++)
+        x[v] = W.word(v) < (u32)tip5::RATE ? elem(W.word(v)) : 0;
+}
+// Absorbs them.
+template <class Wv>
+__device__ __forceinline__ void absorb(u64 (&s)[Wv::kWords], const Wv& W,
+                                       const u64 (&x)[kRateWords<Wv>]) {
+    constexpr int N = kRateWords<Wv>;
+    u64 m[N];
+    if constexpr (N >= 3) {
+        gl::mask bad = 0;
+        gl::to_mont_rare(m, x, bad);
+        if (__builtin_expect(gl::in_mask(bad), 0)) {
+#pragma unroll
+            for (int i = 0; i < N; i++) m[i] = tip5::to_m(x[i]);
+        }
+    } else {
+        m[0] = tip5::to_m(x[0]);
     }
-    s[0] = m[0];
-    s[1] = m[1];
-    s[2] = W.g < 2 ? m[2] : s[2];
+#pragma unroll
+    for (int v = 0; v < N; v++) s[v] = W.word(v) < (u32)tip5::RATE ? m[v] : s[v];
 }
 
 // Absorbs the padding block [rest elements, 1, 0...], rest < 10.
-template <class F>
-__device__ __forceinline__ void absorb_last(u64 s[tip5::WORDS], const tip5::Wave& W, u32 rest,
-                                            const F& elem) {
+template <class Wv, class F>
+__device__ __forceinline__ void absorb_last(u64 (&s)[Wv::kWords], const Wv& W, u32 rest, const F& elem) {
 #pragma unroll
-    for (int v = 0; v < 3; v++) {
-        const u32 i = 4 * v + W.g;
+    for (int v = 0; v < kRateWords<Wv>; v++) {
+        const u32 i = W.word(v);
         if (i < (u32)tip5::RATE)
             s[v] = i < rest ? tip5::to_m(elem(i)) : (i == rest ? tip5::kOneM : 0ull);
     }
 }
 
+// Absorbs `total` elements, elem(i), and permutes after each rate block; the
+// elements past the last full block are left (their count is returned).
+template <class Wv, class F>
+__device__ __forceinline__ u32 absorb_blocks(u64 (&s)[Wv::kWords], const Wv& W, u32 total, const F& elem) {
+    u32 used = 0;
+    for (; used + tip5::RATE <= total; used += tip5::RATE) {
+        u64 x[kRateWords<Wv>];
+        rate_elements(x, W, [&](u32 i) { return elem(used + i); });
+        absorb(s, W, x);
+        tip5::permutation_m(s, W);
+    }
+    return total - used;
+}
+
 // rows x cols column-major table -> rows digests (5 u64 each, row-major).
-__device__ __forceinline__ void hash_rows_body(const HashArgs& A, u64 blk, const tip5::Wave& W) {
-    const u64 row = wave_first(blk) + W.n;
+template <class Wv>
+__device__ __forceinline__ void hash_rows_body(const HashArgs& A, u64 blk, const Wv& W) {
+    const u64 row = wave_first<Wv>(blk) + W.n;
     const u64 rows = A.rows;
     const u32 cols = A.cols;
     // lanes past the last row hash it again (they take part in the matrix products)
     const u64* p = A.tab + (row < rows ? row : rows - 1);
-    u64 s[tip5::WORDS] = {0, 0, 0, 0};
-    u32 used = 0;
-    for (; used + tip5::RATE <= cols; used += tip5::RATE) {
-        absorb(s, W, [&](u32 i) { return __builtin_nontemporal_load(p + (u64)(used + i) * rows); });
-        tip5::permutation_m(s, W);
-    }
-    absorb_last(s, W, cols - used,
-                [&](u32 i) { return __builtin_nontemporal_load(p + (u64)(used + i) * rows); });
+    auto elem = [&](u32 i) { return __builtin_nontemporal_load(p + (u64)i * rows); };
+    u64 s[Wv::kWords] = {};
+    const u32 rest = absorb_blocks(s, W, cols, elem);
+    absorb_last(s, W, rest, [&](u32 i) { return elem(cols - rest + i); });
     tip5::permutation_m(s, W);
     if (row < rows) store_digest(A.dig + row * tip5::DIGEST, s, W);
 }
 
+template <class Wv>
 __global__ void __launch_bounds__(kHashThreads, 4) k_hash_rows(HashArgs A) {
-    __shared__ tip5::Tables T;
+    __shared__ typename Wv::Tables T;
     tip5::load_tables(T);
-    const tip5::Wave W = tip5::make_wave(T);
+    const Wv W = tip5::make_wave(T);
     __syncthreads();
     hash_rows_body(A, blockIdx.x, W);
 }
@@ -121,29 +149,24 @@ __global__ void __launch_bounds__(kHashThreads, 4) k_hash_rows_multi(
 // (state[i*rows + row]).  The FINAL chunk absorbs the padding block
 // [rest, 1, 0...] and writes the canonical digest (tip5.cpp:246-282).  The
 // carried state is in Montgomery form, the carried elements are canonical.
-template <bool FINAL>
+template <bool FINAL, class Wv>
 __global__ void __launch_bounds__(kHashThreads, 4)
     k_absorb_chunk(const u64* __restrict__ chunk, u64 rows, u32 ccols, u64* __restrict__ state,
                    u64* __restrict__ pend, u32 npend, int first, u64* __restrict__ dig) {
-    __shared__ tip5::Tables T;
+    __shared__ typename Wv::Tables T;
     tip5::load_tables(T);
-    const tip5::Wave W = tip5::make_wave(T);
+    const Wv W = tip5::make_wave(T);
     __syncthreads();
-    const u64 row = wave_first(blockIdx.x) + W.n;
+    const u64 row = wave_first<Wv>(blockIdx.x) + W.n;
     const u64 r = row < rows ? row : rows - 1;  // lanes past the end repeat the last row
-    u64 s[tip5::WORDS];
+    u64 s[Wv::kWords];
 #pragma unroll
-    for (int v = 0; v < tip5::WORDS; v++) s[v] = first ? 0ull : state[(u64)(4 * v + W.g) * rows + r];
+    for (int v = 0; v < Wv::kWords; v++) s[v] = first ? 0ull : state[(u64)W.word(v) * rows + r];
     auto elem = [&](u32 j) -> u64 {
         return j < npend ? pend[(u64)j * rows + r] : chunk[(u64)(j - npend) * rows + r];
     };
     const u32 total = npend + ccols;
-    u32 used = 0;
-    for (; used + tip5::RATE <= total; used += tip5::RATE) {
-        absorb(s, W, [&](u32 i) { return elem(used + i); });
-        tip5::permutation_m(s, W);
-    }
-    const u32 rest = total - used;
+    const u32 rest = absorb_blocks(s, W, total, elem), used = total - rest;
     if (FINAL) {
         absorb_last(s, W, rest, [&](u32 i) { return elem(used + i); });
         tip5::permutation_m(s, W);
@@ -151,30 +174,31 @@ __global__ void __launch_bounds__(kHashThreads, 4)
     } else if (row < rows) {
         // carried elements: position i is read and written by the same lane
 #pragma unroll
-        for (int v = 0; v < 3; v++) {
-            const u32 i = 4 * v + W.g;
+        for (int v = 0; v < kRateWords<Wv>; v++) {
+            const u32 i = W.word(v);
             if (i < rest) pend[(u64)i * rows + row] = elem(used + i);
         }
 #pragma unroll
-        for (int v = 0; v < tip5::WORDS; v++) state[(u64)(4 * v + W.g) * rows + row] = s[v];
+        for (int v = 0; v < Wv::kWords; v++) state[(u64)W.word(v) * rows + row] = s[v];
     }
 }
 
 // Tip5 permutation of num states (16 u64 each, in place); outputs canonical.
+template <class Wv>
 __global__ void __launch_bounds__(kHashThreads, 4) k_permutation(u64* __restrict__ st, u64 num) {
-    __shared__ tip5::Tables T;
+    __shared__ typename Wv::Tables T;
     tip5::load_tables(T);
-    const tip5::Wave W = tip5::make_wave(T);
+    const Wv W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first(blockIdx.x) + W.n;
-    const u64* in = st + (i < num ? i : num - 1) * tip5::STATE + W.g;
-    u64 s[tip5::WORDS];
+    const u64 i = wave_first<Wv>(blockIdx.x) + W.n;
+    const u64* in = st + (i < num ? i : num - 1) * tip5::STATE;
+    u64 s[Wv::kWords];
 #pragma unroll
-    for (int v = 0; v < tip5::WORDS; v++) s[v] = tip5::to_m(in[4 * v]);
+    for (int v = 0; v < Wv::kWords; v++) s[v] = tip5::to_m(in[W.word(v)]);
     tip5::permutation_m(s, W);
     if (i >= num) return;
 #pragma unroll
-    for (int v = 0; v < tip5::WORDS; v++) st[i * tip5::STATE + W.g + 4 * v] = tip5::from_m(s[v]);
+    for (int v = 0; v < Wv::kWords; v++) st[i * tip5::STATE + W.word(v)] = tip5::from_m(s[v]);
 }
 
 // Rounds [first, first + count) of the permutation on num states (in place).
@@ -187,7 +211,7 @@ __global__ void __launch_bounds__(kHashThreads) k_permutation_rounds(u64* __rest
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first(blockIdx.x) + W.n;
+    const u64 i = wave_first<tip5::Wave>(blockIdx.x) + W.n;
     const bool live = i < num;
     const u64* in = st + (live ? i : num - 1) * tip5::STATE + W.g;
     u64* tr = trace && live ? trace + i * (count + 1) * tip5::STATE + W.g : nullptr;
@@ -211,77 +235,88 @@ __global__ void __launch_bounds__(kHashThreads) k_permutation_rounds(u64* __rest
     for (int v = 0; v < tip5::WORDS; v++) st[i * tip5::STATE + W.g + 4 * v] = tip5::from_m(s[v]);
 }
 
-// hash_pair: the two digests are words 0..9 (elem), the capacity is ones.
-template <class F>
-__device__ __forceinline__ void hash_pair(u64 s[tip5::WORDS], const tip5::Wave& W, const F& elem) {
-    s[2] = s[3] = tip5::kOneM;
-    absorb(s, W, elem);
+// hash_pair: the two digests are words 0..9 (x: the lane's), the capacity is ones.
+template <class Wv>
+__device__ __forceinline__ void hash_pair(u64 (&s)[Wv::kWords], const Wv& W, const u64 (&x)[kRateWords<Wv>]) {
+#pragma unroll
+    for (int v = 0; v < Wv::kWords; v++) s[v] = tip5::kOneM;
+    absorb(s, W, x);
     tip5::permutation_m(s, W);
 }
 
 // out[i] = hash_pair(left[i], right[i])  (Backend::hash_pairs, backend.hpp:110-115)
+template <class Wv>
 __global__ void __launch_bounds__(kHashThreads, 4) k_hash_pairs(const u64* __restrict__ left,
                                                                 const u64* __restrict__ right,
                                                                 u64* __restrict__ out, u64 count) {
-    __shared__ tip5::Tables T;
+    __shared__ typename Wv::Tables T;
     tip5::load_tables(T);
-    const tip5::Wave W = tip5::make_wave(T);
+    const Wv W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first(blockIdx.x) + W.n;
+    const u64 i = wave_first<Wv>(blockIdx.x) + W.n;
     const u64 r = i < count ? i : count - 1;
-    u64 s[tip5::WORDS];
-    hash_pair(s, W, [&](u32 k) { return k < 5 ? left[5 * r + k] : right[5 * r + k - 5]; });
+    u64 s[Wv::kWords], x[kRateWords<Wv>];
+    rate_elements(x, W, [&](u32 k) { return k < 5 ? left[5 * r + k] : right[5 * r + k - 5]; });
+    hash_pair(s, W, x);
     if (i < count) store_digest(out + 5 * i, s, W);
 }
 
 // One launch of the Merkle build: children are the nodes of one level; each
-// block hashes 2T children into T parents (16 per wave, T <= 16 waves) and
+// block hashes 2T children into T parents (T <= its waves' sponges) and
 // continues for `levels` levels inside LDS.  Level j (1-based) parents go to
 // dst[j-1] + index.
-__device__ __forceinline__ void merkle_body(const MerkleArgs& A, u64 blk, const tip5::Wave& W,
-                                            u64* buf) {
-    const u32 first = (threadIdx.x >> 6) * tip5::GROUP;  // the wave's first parent
+template <class Wv>
+__device__ __forceinline__ void merkle_body(const MerkleArgs& A, u64 blk, const Wv& W, u64* buf) {
+    const u32 first = (threadIdx.x >> 6) * Wv::kSponges;  // the wave's first parent
     const u32 t = first + W.n;
     u32 width = A.T;
-    u64 s[tip5::WORDS];
+    u64 s[Wv::kWords], x[kRateWords<Wv>];
     if (first < width) {  // (whole waves)
         const u64* c = A.src + 10 * (blk * width + (t < width ? t : 0));
-        hash_pair(s, W, [&](u32 k) { return c[k]; });
+        rate_elements(x, W, [&](u32 k) { return c[k]; });
+        hash_pair(s, W, x);
     }
     for (u32 j = 0;; j++) {
         const bool last = j + 1 == A.levels;
         if (t < width) {
             u64* d = A.dst[j] + 5 * (blk * width + t);
-            const u64 x = tip5::from_m(s[0]);
-            d[W.g] = x;
-            if (!last) buf[5 * t + W.g] = x;
-            if (W.g == 0) {
-                const u64 z = tip5::from_m(s[1]);
-                d[4] = z;
-                if (!last) buf[5 * t + 4] = z;
-            }
+#pragma unroll
+            for (int v = 0; v < Wv::kWords; v++)
+                if (W.word(v) < (u32)tip5::DIGEST) {
+                    const u64 y = tip5::from_m(s[v]);
+                    d[W.word(v)] = y;
+                    if (!last) buf[5 * t + W.word(v)] = y;
+                }
         }
         if (last) break;
         __syncthreads();  // this level's digests are in buf
         width >>= 1;
-        u64 in[3] = {0, 0, 0};
-        if (first < width) {
-            const u64* c = buf + 10 * (t < width ? t : 0);
-            in[0] = c[W.g];
-            in[1] = c[4 + W.g];
-            if (W.g < 2) in[2] = c[8 + W.g];
-        }
+        if (first < width) rate_elements(x, W, [&](u32 k) { return buf[10 * (t < width ? t : 0) + k]; });
         __syncthreads();  // every read of buf precedes the next level's writes
-        if (first < width) hash_pair(s, W, [&](u32 k) { return in[k >> 2]; });
+        if (first < width) hash_pair(s, W, x);
     }
 }
 
-template <int THREADS>
-__global__ void __launch_bounds__(THREADS) k_merkle_subtrees(MerkleArgs A) {
+// One level, kSpongesPerBlock parents to a block.
+__global__ void __launch_bounds__(kHashThreads) k_merkle_level(MerkleArgs A) {
     __shared__ tip5::Tables T;
-    __shared__ u64 buf[THREADS / 64 * tip5::GROUP * 5];
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
+    __syncthreads();
+    const u64 i = wave_first<tip5::Wave>(blockIdx.x) + W.n;
+    const u64* c = A.src + 10 * i;
+    u64 s[tip5::WORDS], x[3];
+    rate_elements(x, W, [&](u32 k) { return c[k]; });
+    hash_pair(s, W, x);
+    store_digest(A.dst[0] + 5 * i, s, W);
+}
+
+// Levels of few parents, up to kQuadSponges to a block, four to a wave.
+__global__ void __launch_bounds__(kMerkleThreads) k_merkle_subtrees(MerkleArgs A) {
+    __shared__ tip5::QuadTables T;
+    __shared__ u64 buf[kQuadSponges * 5];
+    tip5::load_tables(T);
+    const tip5::QuadWave W = tip5::make_wave(T);
     __syncthreads();
     merkle_body(A, blockIdx.x, W, buf);
 }
@@ -321,24 +356,36 @@ __global__ void k_gather_heap(const u64* __restrict__ tree, u64 n, u32 logn, int
 
 // ------------------------------------------------------------------ host side
 
+// The 16-sponge form, or the four-sponge one where that leaves few waves.
+#define TVH_SPONGES(count, kernel, ...)                                                            \
+    do {                                                                                           \
+        if ((count) <= kQuadMaxSponges)                                                            \
+            hipLaunchKernelGGL(kernel<tip5::QuadWave>, dim3(quad_blocks(count)), dim3(kHashThreads), \
+                               0, st, __VA_ARGS__);                                                \
+        else                                                                                       \
+            hipLaunchKernelGGL(kernel<tip5::Wave>, dim3(sponge_blocks(count)), dim3(kHashThreads), \
+                               0, st, __VA_ARGS__);                                                \
+    } while (0)
+template <class Wv>
+constexpr auto k_absorb_chunk_final = k_absorb_chunk<true, Wv>;
+template <class Wv>
+constexpr auto k_absorb_chunk_more = k_absorb_chunk<false, Wv>;
+
 int launch_hash_rows(const u64* tab, u64 rows, u64 cols, u64* dig, hipStream_t st) {
     if (rows == 0) return TVH_OK;
     if (cols > 0xFFFFFFFFull) return TVH_ERR_INVALID_ARG;
-    hipLaunchKernelGGL(k_hash_rows, dim3(sponge_blocks(rows)), dim3(kHashThreads), 0, st,
-                       HashArgs{tab, rows, (u32)cols, dig});
+    const HashArgs A{tab, rows, (u32)cols, dig};
+    TVH_SPONGES(rows, k_hash_rows, A);
     return check_launch();
 }
 
 int launch_absorb_chunk(const u64* chunk, u64 rows, u64 ccols, u64* state, u64* pend, u32 npend,
                         bool first, bool final_chunk, u64* dig, hipStream_t st) {
     if (rows == 0) return TVH_OK;
-    const dim3 blocks(sponge_blocks(rows)), tpb(kHashThreads);
     if (final_chunk)
-        hipLaunchKernelGGL(k_absorb_chunk<true>, blocks, tpb, 0, st, chunk, rows, (u32)ccols, state,
-                           pend, npend, (int)first, dig);
+        TVH_SPONGES(rows, k_absorb_chunk_final, chunk, rows, (u32)ccols, state, pend, npend, (int)first, dig);
     else
-        hipLaunchKernelGGL(k_absorb_chunk<false>, blocks, tpb, 0, st, chunk, rows, (u32)ccols, state,
-                           pend, npend, (int)first, dig);
+        TVH_SPONGES(rows, k_absorb_chunk_more, chunk, rows, (u32)ccols, state, pend, npend, (int)first, dig);
     return check_launch();
 }
 
@@ -346,7 +393,7 @@ int launch_absorb_chunk(const u64* chunk, u64 rows, u64 ccols, u64* state, u64* 
 // the reference's device transcript (fiat_shamir_kernel.cu: fs_absorb_device_gpu
 // pads [data..., 1, 0...] to a multiple of 10 and overwrites the rate before
 // each permutation; squeeze reads the rate, then permutes).  One wave runs the
-// whole absorption in one launch; its 16 sponges are the same one.
+// whole absorption in one launch; its four sponges are the same one.
 // mode 0 absorb, 1 squeeze, 2 init (zeros; a kernel rather than a memset so
 // that the call can be captured in a graph).
 __global__ void __launch_bounds__(64) k_sponge(u64* __restrict__ state,
@@ -356,31 +403,26 @@ __global__ void __launch_bounds__(64) k_sponge(u64* __restrict__ state,
         if (threadIdx.x < tip5::STATE) state[threadIdx.x] = 0;
         return;
     }
-    __shared__ tip5::Tables T;
+    __shared__ tip5::QuadTables T;
     tip5::load_tables(T);
-    const tip5::Wave W = tip5::make_wave(T);
-    u64 s[tip5::WORDS];
-#pragma unroll
-    for (int v = 0; v < tip5::WORDS; v++) s[v] = tip5::to_m(state[4 * v + W.g]);
+    const tip5::QuadWave W = tip5::make_wave(T);
+    u64 s[1] = {tip5::to_m(state[W.own])};
     __syncthreads();  // (also: every lane has read the state before lanes n = 0 write it)
     if (mode == 1) {
-#pragma unroll
-        for (int v = 0; v < 3; v++)
-            if (W.n == 0 && 4 * v + W.g < (u32)tip5::RATE) out[4 * v + W.g] = tip5::from_m(s[v]);
+        if (W.n == 0 && W.own < (u32)tip5::RATE) out[W.own] = tip5::from_m(s[0]);
         tip5::permutation_m(s, W);
     } else {
         u64 base = 0;
         for (; base + tip5::RATE <= len; base += tip5::RATE) {
-            absorb(s, W, [&](u32 i) { return data[base + i]; });
+            u64 x[1];
+            rate_elements(x, W, [&](u32 i) { return data[base + i]; });
+            absorb(s, W, x);
             tip5::permutation_m(s, W);
         }
         absorb_last(s, W, (u32)(len - base), [&](u32 i) { return data[base + i]; });
         tip5::permutation_m(s, W);
     }
-    if (W.n == 0) {
-#pragma unroll
-        for (int v = 0; v < tip5::WORDS; v++) state[4 * v + W.g] = tip5::from_m(s[v]);
-    }
+    if (W.n == 0) state[W.own] = tip5::from_m(s[0]);
 }
 
 int launch_sponge(u64* state, const u64* data, u64 len, u64* out, int mode, hipStream_t st) {
@@ -410,8 +452,7 @@ int launch_xfe_leaves(const u64* xfe, u64 n, u64* leaves, hipStream_t st) {
 
 int launch_permutation(u64* states, u64 num, hipStream_t st) {
     if (num == 0) return TVH_OK;
-    hipLaunchKernelGGL(k_permutation, dim3(sponge_blocks(num)), dim3(kHashThreads), 0, st, states,
-                       num);
+    TVH_SPONGES(num, k_permutation, states, num);
     return check_launch();
 }
 
@@ -425,8 +466,7 @@ int launch_permutation_rounds(u64* states, u64 num, u32 first, u32 count, u64* t
 
 int launch_hash_pairs(const u64* l, const u64* r, u64* out, u64 count, hipStream_t st) {
     if (count == 0) return TVH_OK;
-    hipLaunchKernelGGL(k_hash_pairs, dim3(sponge_blocks(count)), dim3(kHashThreads), 0, st, l, r, out,
-                       count);
+    TVH_SPONGES(count, k_hash_pairs, l, r, out, count);
     return check_launch();
 }
 
@@ -436,7 +476,8 @@ u64 merkle_level_base(u64 n, u32 level, int layout) {
 
 // Launch groups of the Merkle build of an n-leaf tree whose leaves are already
 // at level 0: group g covers up to 9 levels; T parents per block at its first.
-// A launch over many tables (multi) has one block size for all of them.
+// A launch over many tables (multi) has one block size for all of them.  For a
+// single tree, levels of at most kQuadMaxSponges parents go four to a wave.
 int merkle_groups(u64* tree, u64 n, int layout, bool multi, std::vector<MerkleGroup>& groups) {
     groups.clear();
     u32 logn = log2u(n);
@@ -444,8 +485,8 @@ int merkle_groups(u64* tree, u64 n, int layout, bool multi, std::vector<MerkleGr
     while (lvl < logn) {
         u64 nchild = n >> lvl;
         u64 parents = nchild / 2;
-        const bool wide = parents > kMerkleSubtreeParents;
-        const u64 most = wide && !multi ? kSpongesPerBlock : kMerkleSponges;
+        const bool wide = parents > (multi ? kMerkleSubtreeParents : kQuadMaxSponges);
+        const u64 most = multi ? kMerkleSponges : wide ? kSpongesPerBlock : kQuadSponges;
         u32 T = (u32)(parents < most ? parents : most);  // parents is a power of two
         u32 maxlev = wide ? 1 : log2u(T) + 1;            // T = 256 -> 9 levels
         u32 levels = logn - lvl < maxlev ? logn - lvl : maxlev;
@@ -455,6 +496,7 @@ int merkle_groups(u64* tree, u64 n, int layout, bool multi, std::vector<MerkleGr
             g.args.dst[j] = j < levels ? tree + 5 * merkle_level_base(n, lvl + j + 1, layout) : nullptr;
         g.args.levels = levels;
         g.args.T = T;
+        g.quad = !multi && !wide;
         g.blocks = (u32)(parents / T);
         groups.push_back(g);
         lvl += levels;
@@ -467,12 +509,11 @@ int launch_merkle_levels(u64* tree, u64 n, int layout, hipStream_t st) {
     std::vector<MerkleGroup> groups;
     merkle_groups(tree, n, layout, false, groups);
     for (const MerkleGroup& g : groups) {
-        if (g.args.T <= kSpongesPerBlock)
-            hipLaunchKernelGGL(k_merkle_subtrees<kHashThreads>, dim3(g.blocks), dim3(kHashThreads), 0,
-                               st, g.args);
+        if (g.quad)  // (waves for the first level's parents)
+            hipLaunchKernelGGL(k_merkle_subtrees, dim3(g.blocks),
+                               dim3((g.args.T + tip5::QUAD - 1) / tip5::QUAD * 64), 0, st, g.args);
         else
-            hipLaunchKernelGGL(k_merkle_subtrees<kMerkleThreads>, dim3(g.blocks),
-                               dim3(kMerkleThreads), 0, st, g.args);
+            hipLaunchKernelGGL(k_merkle_level, dim3(g.blocks), dim3(kHashThreads), 0, st, g.args);
         int rc = check_launch();
         if (rc) return rc;
     }

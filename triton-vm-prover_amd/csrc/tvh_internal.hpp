@@ -237,10 +237,18 @@ u64 fill_table_scratch_elems();
 // 16 sponges per wave: a block of the hashing kernels takes 64 of them.
 constexpr u32 kHashThreads = 256, kSpongesPerBlock = kHashThreads / 64 * tip5::GROUP;
 inline u32 sponge_blocks(u64 count) { return (u32)((count + kSpongesPerBlock - 1) / kSpongesPerBlock); }
+// Up to kQuadMaxSponges sponges run four to a wave, kQuadSponges to a block of the
+// Merkle kernel.
+constexpr u64 kQuadMaxSponges = 16384;
+inline u32 quad_blocks(u64 count) {
+    const u32 per = kHashThreads / 64 * tip5::QUAD;
+    return (u32)((count + per - 1) / per);
+}
 // Merkle levels of at most kMerkleSubtreeParents parents run several levels to
 // a launch, in blocks of up to kMerkleSponges parents.
 constexpr u32 kMerkleThreads = 1024, kMerkleSponges = kMerkleThreads / 64 * tip5::GROUP;
 constexpr u64 kMerkleSubtreeParents = 1u << 15;
+constexpr u32 kQuadSponges = kMerkleThreads / 64 * tip5::QUAD;
 struct HashArgs {
     const u64* tab;
     u64 rows;
@@ -256,6 +264,7 @@ struct MerkleArgs {
 struct MerkleGroup {
     MerkleArgs args;
     u32 blocks;
+    bool quad;
 };
 int merkle_groups(u64* tree, u64 n, int layout, bool multi, std::vector<MerkleGroup>& groups);
 int launch_hash_rows_multi(const HashArgs* d_args, const u32* d_start, u32 nseg, u32 blocks,

@@ -485,6 +485,18 @@ __device__ __forceinline__ u32 find_segment(const u32* __restrict__ start, u32 n
     return __builtin_amdgcn_readfirstlane(lo);
 }
 
+// Blocks go to the eight XCDs in turn, each with its own L2.  Of `blocks` blocks,
+// 2^lb to a column, the one that XCD x = blk mod 8 runs in turn: a column's blocks
+// follow each other on one XCD, the same in every step.  So the cache lines that
+// several of them write in part are completed in one L2, and what a step leaves
+// in an L2 the next one reads there.
+__device__ __forceinline__ u64 column_on_xcd(u32 blk, u32 blocks, u32 lb) {
+    const u32 full = (blocks >> (lb + 3)) << (lb + 3);  // of whole groups of eight columns
+    if (blk >= full) return blk;
+    const u32 y = blk >> 3;
+    return ((((y >> lb) << 3) + (blk & 7)) << lb) + (y & ((1u << lb) - 1));
+}
+
 // Where a block's transforms are: transform t0 + t of column c, `valid` of them.
 // A column of 2^log_per transforms takes max(1, 2^log_per / NT) blocks, so blocks
 // never span columns; where every column is a single transform (log_per = 0,
@@ -493,7 +505,9 @@ struct BlockPlace {
     u64 c;
     u32 t0, valid;
 };
-__device__ __forceinline__ BlockPlace block_place(u64 blk, u32 log_nt, u32 log_per, u64 cols, bool flat) {
+// blocks: of a launch whose columns go by XCD, or 0.
+__device__ __forceinline__ BlockPlace block_place(u64 blk, u32 log_nt, u32 log_per, u64 cols, bool flat,
+                                                  u32 blocks = 0) {
     BlockPlace B;
     if (flat) {
         B.c = blk << log_nt;
@@ -502,6 +516,7 @@ __device__ __forceinline__ BlockPlace block_place(u64 blk, u32 log_nt, u32 log_p
         return B;
     }
     const u32 lb = log_per > log_nt ? log_per - log_nt : 0;  // log2 blocks of a column
+    if (blocks) blk = column_on_xcd((u32)blk, blocks, lb);
     B.c = blk >> lb;
     B.t0 = ((u32)blk & ((1u << lb) - 1)) << log_nt;
     B.valid = 1u << (log_per < log_nt ? log_per : log_nt);
@@ -558,7 +573,7 @@ struct Step1 {
                                      u64 blk, u32 log_nt)
         : A(A_), S(S_), rt(rt_) {
         const u32 b = A.logN - A.a;
-        B = block_place(blk, log_nt, b, 0, false);
+        B = block_place(blk, log_nt, b, 0, false, A.by_xcd);
         in = {A.src + B.c * A.sstride + B.t0, 0, 1, 0, 1u << b};
         out = {A.dst + B.c * A.dstride + B.t0, 0, 1, 0, A.E << b};
     }

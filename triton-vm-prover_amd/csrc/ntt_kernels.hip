@@ -287,7 +287,7 @@ int prepare_lde(const u64* trace, u64 cols, u64 n, const RandSpec& rs, u64 toff,
     // map trace -> Y, so K2 then reads the trace itself.
     P->k1 = a > 0;
     if (P->k1) {
-        P->s1 = Step1Args{trace, n, out, m, logN, a, E, 1};
+        P->s1 = Step1Args{trace, n, out, m, logN, a, E, 1, 0};
         P->g1 = launch_shape(P->col_lt, a, b, cols, false);
     }
     // K2: INTT step 2 + coset scaling + forward step 1
@@ -412,15 +412,18 @@ int launch_ntt_batched(const u64* src, u64* dst, u64 n, u64 cols, bool inverse, 
     DeviceState* ds = current_device();
     if (!ds) return TVH_ERR_DEVICE;
     // Split N = N1 * N2 and tiles, measured on MI355X over 2^13..2^24 rows and 4 to
-    // 1000 columns.  Two passes in each step where both lengths can be at most 2^8
-    // to 2^10 (2^16 x 379: N1 = 2^8 190 us, 2^7 218), rows of 2^12 above 2^20.
-    // Column tiles of 2^13 elements (2^12 while those are fewer than four blocks a
-    // CU: 2^14 x 60 21 us, 25 in 2^13 tiles, 35 in 2^14; 2^14 beyond 2^22 rows, where
-    // 2^13 would hold 4 or 2 columns' transforms, 32 or 16 B segments).  The row
-    // step stores each block's rows transposed, in runs as long as its row count:
-    // the shortest tile that holds 8 rows (2^17 x 251: 276 us in 2^12, 296 in 2^13;
-    // 2^18 x 379: 0.98 ms in 2^14, 0.88 in 2^13, 0.92 with 4 rows in 2^12).
-    u32 a = logN <= 14 ? logN / 2 : logN <= 19 ? 8 : logN == 20 ? 10 : logN - 12;
+    // 1000 columns.  N1 = 2^8, two passes, wherever N2 fits in 2^12 (2^16 x 379: 186
+    // us, N1 = 2^7 220; 2^20 x 379: 3.89 ms, N1 = 2^9 4.34, 2^10 4.46).  Column tiles
+    // of 2^13 elements (2^12 while those are fewer than four blocks a CU: 2^14 x 60 21
+    // us, 25 in 2^13 tiles, 35 in 2^14; 2^14 beyond 2^22 rows, where 2^13 would hold 4
+    // or 2 columns' transforms, 32 or 16 B segments).  The row step stores a block's
+    // rows transposed, in runs as long as its row count: the shortest tile that holds
+    // 8 rows.  Blocks of one column go to one XCD, whose L2 completes their cache
+    // lines (column_on_xcd).  Shorter runs can be faster by themselves and slow down
+    // the kernel that reads them next: evaluating a coset of 2^19 x 379 takes 2.17 ms
+    // in column order, 2.07 as here, 1.97 in 2^13 tiles; with the row hashes after it
+    // 4.54, 4.46 and 4.66.
+    u32 a = logN <= 14 ? logN / 2 : logN <= 20 ? 8 : logN - 12;
     // up to 2^12 rows the row step alone (2^10 x 100: 9.4 us in 2^12 tiles, 19.6 in 2^14)
     if (logN <= 12 && !scale) a = 0;
     const u32 b = logN - a;
@@ -451,7 +454,7 @@ int launch_ntt_batched(const u64* src, u64* dst, u64 n, u64 cols, bool inverse, 
         const bool one_step = a == 0 && !scale;
         if (!one_step) {
             const LaunchShape s1 = launch_shape(col_lt, a, b, g, false);
-            Step1Args A{sg, n, scratch, n, logN, a, 1u, inverse ? ninv : 1};
+            Step1Args A{sg, n, scratch, n, logN, a, 1u, inverse ? ninv : 1, s1.blocks};
             if (scale) {
                 NttScaleDev Sg = S;
                 if (Sg.rand) Sg.rand += c0 * Sg.k;  // the group's first column

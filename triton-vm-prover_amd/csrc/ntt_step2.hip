@@ -16,10 +16,10 @@ struct RowStep {
     Place<u64> out;
     u64 ninv;
     __device__ __forceinline__ RowStep(const u64* src, u64* dst, u32 logN, u32 a, u64 cols, u64 ninv_,
-                                       u64 blk, u32 log_nt)
+                                       u64 blk, u32 log_nt, u32 blocks = 0)
         : ninv(ninv_) {
         const u32 b = logN - a;
-        B = block_place(blk, log_nt, a, cols, COLS);
+        B = block_place(blk, log_nt, a, cols, COLS, blocks);
         in = {src + (B.c << logN) + ((u64)B.t0 << b), 0, 1u << b, 0, 1};
         out = {dst + (B.c << logN) + B.t0, 0, COLS ? 1u << logN : 1u, 0, 1u << a};
     }
@@ -37,7 +37,7 @@ __global__ void __launch_bounds__(1 << (LT - 4), 4) k_ntt_step2(const u64* src, 
                                                                 u32 a, u64 cols, u64 ninv, Roots rt) {
     extern __shared__ u64 lds[];
     typedef Shape<LT, LOGL> Z;
-    const RowStep<INV, COLS> P(src, dst, logN, a, cols, ninv, blockIdx.x, Z::logNT);
+    const RowStep<INV, COLS> P(src, dst, logN, a, cols, ninv, blockIdx.x, Z::logNT, gridDim.x);
     load_tile<Z, false>(lds, P.in, P.B.valid, [](u32, u32, const u32 (&)[4], u64 (&)[4]) {});
     dft_block<Z>(lds, Z::logNT, rt.dft[INV], rt.r4096[INV]);
     store_tile<Z, !COLS>(lds, P.out, P.B.valid, [&](u64 (&x)[4]) { P.finish(x); });

@@ -133,6 +133,7 @@ struct Step1Args {
     u64 dstride;
     u32 logN, a, E;
     u64 factor;  // of every output (N^-1 of an inverse NTT; 1)
+    u32 by_xcd;  // blocks of a launch whose columns go by XCD (column_on_xcd), or 0
 };
 struct Step3Args {
     u64* out;

@@ -162,12 +162,12 @@ __device__ const MdsStarts kMdsStarts = mds_starts();
 // ---- LDS tables of a block -----------------------------------------------------
 struct alignas(16) Tables {
     u32 start[ROUNDS * 4 * 16];
-    uint8_t lut[256];  // the S-box ((x+1)^3 mod 257) - 1
+    uint8_t lut[256];  // the S-box ((x+1)^3 mod 257) - 1, its top bit flipped
 };
 __device__ __forceinline__ void load_lut(uint8_t* lut) {
     for (u32 x = threadIdx.x; x < 256; x += blockDim.x) {
         u32 t = x + 1;
-        lut[x] = (uint8_t)(((t * t % 257) * t % 257) - 1);
+        lut[x] = (uint8_t)((((t * t % 257) * t % 257) - 1) ^ 0x80);
     }
 }
 // Fills them (the caller synchronises the block before use).
@@ -219,9 +219,28 @@ __device__ __forceinline__ void pow7_rare(u64 (&y)[N], const u64 (&x)[N], gl::ma
     gl::mul_rare(y, x3, x4, bad);
 }
 
+// Four bytes through the table.  The loads zero-extend them, which the compiler does
+// not make use of (3 operations for its 5: hashing 2^22 rows of 379, 19.3 -> 19.1 ms);
+// but it places its own operations behind the x^7, where the loads have arrived,
+// which is what a lone wave (LONE) wants.
+#define TIP5_LSHL_OR(r, b, n, a) asm("v_lshl_or_b32 %0, %1, " #n ", %2" : "=v"(r) : "v"(b), "v"(a))
+template <bool LONE>
+__device__ __forceinline__ u32 lookup_bytes(u32 x, const uint8_t* lut) {
+    if constexpr (LONE)
+        return (u32)lut[x & 0xff] | ((u32)lut[(x >> 8) & 0xff] << 8) |
+               ((u32)lut[(x >> 16) & 0xff] << 16) | ((u32)lut[x >> 24] << 24);
+    u32 lo, hi, r;
+    TIP5_LSHL_OR(lo, (u32)lut[(x >> 8) & 0xff], 8, (u32)lut[x & 0xff]);
+    TIP5_LSHL_OR(hi, (u32)lut[x >> 24], 8, (u32)lut[(x >> 16) & 0xff]);
+    TIP5_LSHL_OR(r, hi, 16, lo);
+    return r;
+}
+#undef TIP5_LSHL_OR
+
 // S-box of words 0..3 on a Montgomery-form value: bytes of the canonical value
 // through the table; the result is the Montgomery form of the reference's
-// output (tip5.cpp split_and_lookup).
+// output (tip5.cpp split_and_lookup), less kKappa byte by byte (y ^ kKappa).
+template <bool LONE>
 __device__ __forceinline__ u64 split_and_lookup(u64 m, const uint8_t* lut) {
     u32 lo = (u32)m, hi = (u32)(m >> 32);
     // p <= m < 2^64 only with a high word of ones and a nonzero low word
@@ -231,11 +250,7 @@ __device__ __forceinline__ u64 split_and_lookup(u64 m, const uint8_t* lut) {
             hi = 0;
         }
     }
-    const u32 olo = (u32)lut[lo & 0xff] | ((u32)lut[(lo >> 8) & 0xff] << 8) |
-                    ((u32)lut[(lo >> 16) & 0xff] << 16) | ((u32)lut[lo >> 24] << 24);
-    const u32 ohi = (u32)lut[hi & 0xff] | ((u32)lut[(hi >> 8) & 0xff] << 8) |
-                    ((u32)lut[(hi >> 16) & 0xff] << 16) | ((u32)lut[hi >> 24] << 24);
-    return ((u64)ohi << 32) | olo;
+    return gl::mk64(lookup_bytes<LONE>(lo, lut), lookup_bytes<LONE>(hi, lut));
 }
 
 // ---- one round, the permutation --------------------------------------------------
@@ -247,18 +262,17 @@ __device__ __forceinline__ void round_m(u64 s[WORDS], int r, const Wave& W) {
     u64 y7[3];
     gl::mask bad = 0;
     pow7_rare(y7, x, bad);
-    s[0] = split_and_lookup(s[0], W.T->lut);
+    const u64 look = split_and_lookup<false>(s[0], W.T->lut);
     if (__builtin_expect(gl::in_mask(bad), 0)) {
 #pragma unroll
         for (int i = 0; i < 3; i++) y7[i] = pow7(x[i]);
     }
-#pragma unroll
-    for (int i = 0; i < 3; i++) s[1 + i] = y7[i];
     v4i lo, hi;
 #pragma unroll
     for (int v = 0; v < WORDS; v++) {
-        lo[v] = (int)((u32)s[v] ^ (u32)kKappa);
-        hi[v] = (int)((u32)(s[v] >> 32) ^ (u32)kKappa);
+        const u64 y = v ? y7[v - 1] ^ kKappa : look;
+        lo[v] = (int)(u32)y;
+        hi[v] = (int)(u32)(y >> 32);
     }
     const v4i* start = (const v4i*)(W.T->start + r * 64) + W.g;
     v4i y[8];
@@ -361,7 +375,7 @@ __device__ __forceinline__ void round_m(u64 s[1], int r, const QuadWave& W) {
     const u64 x = s[0];
     const v4i* start = (const v4i*)(W.T->start) + r * 32 + W.own;
     v4i ya = start[0], yb = start[16];
-    const u64 look = split_and_lookup(x, W.T->lut);  // (of use in words 0..3)
+    const u64 look = split_and_lookup<true>(x, W.T->lut);  // (of use in words 0..3)
     gl::mask bad = 0;
     const u64 x1[1] = {x};
     u64 x2[1], x34[2], y7[1];
@@ -371,8 +385,8 @@ __device__ __forceinline__ void round_m(u64 s[1], int r, const QuadWave& W) {
     const u64 x3[1] = {x34[0]}, x4[1] = {x34[1]};
     gl::mul_rare(y7, x3, x4, bad);
     if (__builtin_expect(gl::in_mask(bad), 0)) y7[0] = pow7(x);
-    const u64 y = W.own < 4 ? look : y7[0];
-    const int l = (int)((u32)y ^ (u32)kKappa), h = (int)((u32)(y >> 32) ^ (u32)kKappa);
+    const u64 y = W.own < 4 ? look : y7[0] ^ kKappa;
+    const int l = (int)(u32)y, h = (int)(u32)(y >> 32);
     // (row_ror:n reads lane i - n of the row)
 #define TIP5_ROR(a, n) __builtin_amdgcn_mov_dpp(a, 0x120 + n, 0xF, 0xF, true)
     const v4i lo = {l, TIP5_ROR(l, 12), TIP5_ROR(l, 8), TIP5_ROR(l, 4)};

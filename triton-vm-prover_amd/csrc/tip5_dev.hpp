@@ -240,7 +240,6 @@ __device__ __forceinline__ u32 lookup_bytes(u32 x, const uint8_t* lut) {
 // S-box of words 0..3 on a Montgomery-form value: bytes of the canonical value
 // through the table; the result is the Montgomery form of the reference's
 // output (tip5.cpp split_and_lookup), less kKappa byte by byte (y ^ kKappa).
-template <bool LONE>
 __device__ __forceinline__ u64 split_and_lookup(u64 m, const uint8_t* lut) {
     u32 lo = (u32)m, hi = (u32)(m >> 32);
     // p <= m < 2^64 only with a high word of ones and a nonzero low word
@@ -250,7 +249,11 @@ __device__ __forceinline__ u64 split_and_lookup(u64 m, const uint8_t* lut) {
             hi = 0;
         }
     }
-    return gl::mk64(lookup_bytes<LONE>(lo, lut), lookup_bytes<LONE>(hi, lut));
+    return gl::mk64(lookup_bytes<false>(lo, lut), lookup_bytes<false>(hi, lut));
+}
+// ... of m < p, in a lone wave
+__device__ __forceinline__ u64 lookup_canonical(u64 m, const uint8_t* lut) {
+    return gl::mk64(lookup_bytes<true>((u32)m, lut), lookup_bytes<true>((u32)(m >> 32), lut));
 }
 
 // ---- one round, the permutation --------------------------------------------------
@@ -262,7 +265,7 @@ __device__ __forceinline__ void round_m(u64 s[WORDS], int r, const Wave& W) {
     u64 y7[3];
     gl::mask bad = 0;
     pow7_rare(y7, x, bad);
-    const u64 look = split_and_lookup<false>(s[0], W.T->lut);
+    const u64 look = split_and_lookup(s[0], W.T->lut);
     if (__builtin_expect(gl::in_mask(bad), 0)) {
 #pragma unroll
         for (int i = 0; i < 3; i++) y7[i] = pow7(x[i]);
@@ -311,9 +314,9 @@ __device__ __forceinline__ void permutation_m(u64 s[WORDS], const Wave& W) {
 // its result is rotated alike: output word g of the column is the lane's own word
 // 4w + g.  Only those four rows are needed, so the other rows of a product hold
 // other byte places (register v: place v, or 4 + v): four products a round in place
-// of twelve, and one join.  A permutation takes 2.1 us where the form above takes
-// 4.0, and twice the issue slots per sponge: 16384 rows of 379 160 us against 170,
-// 4096 rows 86 against 157.
+// of twelve, and one join.  A permutation takes 1.9 us where the form above takes
+// 4.0, and twice the issue slots per sponge: 16384 rows of 379 163 us against 170,
+// 4096 rows 82 against 157.
 constexpr int QUAD = 4;  // sponges per wave
 
 // First operands: product 2 P + h, row 4g' + v' is place 4 P + v' of output word g',
@@ -375,8 +378,10 @@ __device__ __forceinline__ void round_m(u64 s[1], int r, const QuadWave& W) {
     const u64 x = s[0];
     const v4i* start = (const v4i*)(W.T->start) + r * 32 + W.own;
     v4i ya = start[0], yb = start[16];
-    const u64 look = split_and_lookup<true>(x, W.T->lut);  // (of use in words 0..3)
-    gl::mask bad = 0;
+    u64 look = lookup_canonical(x, W.T->lut);  // (of use in words 0..3)
+    // p <= x < 2^64 only with a high word of ones: left to the branch of the products
+    // (with one of its own a permutation took 2.06 us, without 1.94)
+    gl::mask bad = __builtin_amdgcn_ballot_w64((u32)(x >> 32) == 0xFFFFFFFFu);
     const u64 x1[1] = {x};
     u64 x2[1], x34[2], y7[1];
     gl::mul_rare(x2, x1, x1, bad);
@@ -384,7 +389,10 @@ __device__ __forceinline__ void round_m(u64 s[1], int r, const QuadWave& W) {
     gl::mul_rare(x34, xs, x22, bad);
     const u64 x3[1] = {x34[0]}, x4[1] = {x34[1]};
     gl::mul_rare(y7, x3, x4, bad);
-    if (__builtin_expect(gl::in_mask(bad), 0)) y7[0] = pow7(x);
+    if (__builtin_expect(gl::in_mask(bad), 0)) {
+        y7[0] = pow7(x);
+        look = lookup_canonical(gl::canon(x), W.T->lut);
+    }
     const u64 y = W.own < 4 ? look : y7[0] ^ kKappa;
     const int l = (int)(u32)y, h = (int)(u32)(y >> 32);
     // (row_ror:n reads lane i - n of the row)

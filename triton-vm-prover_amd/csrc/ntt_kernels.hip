@@ -1,7 +1,8 @@
 // Host side of the batched Goldilocks NTT and the coset low-degree extension:
 // kernel variants and plans, the per-shape coset tables, launches, the
 // synthetic fill and the XFE relayout.  The kernels themselves are in
-// ntt_dev.hpp (device code) and ntt_step1.hip, lde_rows.hip, lde_step3.hip (instantiations and launchers).
+// ntt_dev.hpp (device code) and ntt_step1.hip, ntt_step2.hip, lde_rows.hip,
+// lde_step3.hip (instantiations and launchers).
 #include <atomic>
 #include <map>
 #include <mutex>

@@ -222,18 +222,19 @@ __device__ __forceinline__ void pow7_rare(u64 (&y)[N], const u64 (&x)[N], gl::ma
 // Four bytes through the table.  The loads zero-extend them, which the compiler does
 // not make use of (3 operations for its 5: hashing 2^22 rows of 379, 19.3 -> 19.1 ms);
 // but it places its own operations behind the x^7, where the loads have arrived,
-// which is what a lone wave (LONE) wants.
+// which is what a lone wave (LONE) wants.  The last operation is the compiler's: the
+// result goes to a matrix product, which wants two wait states after a VALU write of
+// its operand, and the compiler does not look into asm.
 #define TIP5_LSHL_OR(r, b, n, a) asm("v_lshl_or_b32 %0, %1, " #n ", %2" : "=v"(r) : "v"(b), "v"(a))
 template <bool LONE>
 __device__ __forceinline__ u32 lookup_bytes(u32 x, const uint8_t* lut) {
     if constexpr (LONE)
         return (u32)lut[x & 0xff] | ((u32)lut[(x >> 8) & 0xff] << 8) |
                ((u32)lut[(x >> 16) & 0xff] << 16) | ((u32)lut[x >> 24] << 24);
-    u32 lo, hi, r;
+    u32 lo, hi;
     TIP5_LSHL_OR(lo, (u32)lut[(x >> 8) & 0xff], 8, (u32)lut[x & 0xff]);
     TIP5_LSHL_OR(hi, (u32)lut[x >> 24], 8, (u32)lut[(x >> 16) & 0xff]);
-    TIP5_LSHL_OR(r, hi, 16, lo);
-    return r;
+    return (hi << 16) | lo;
 }
 #undef TIP5_LSHL_OR
 

@@ -44,6 +44,9 @@ __device__ __forceinline__ u32 find_seg(const u32* __restrict__ start, u32 nseg,
     return lo;
 }
 
+// Block index of a hash_grid launch.
+__device__ __forceinline__ u64 grid_block() { return (u64)blockIdx.y * gridDim.x + blockIdx.x; }
+
 // First sponge of the wave in block blk.
 template <class Wv>
 __device__ __forceinline__ u64 wave_first(u64 blk) {
@@ -126,7 +129,7 @@ __global__ void __launch_bounds__(kHashThreads, 4) k_hash_rows(HashArgs A) {
     tip5::load_tables(T);
     const Wv W = tip5::make_wave(T);
     __syncthreads();
-    hash_rows_body(A, blockIdx.x, W);
+    hash_rows_body(A, grid_block(), W);
 }
 
 __global__ void __launch_bounds__(kHashThreads, 4) k_hash_rows_multi(
@@ -135,9 +138,11 @@ __global__ void __launch_bounds__(kHashThreads, 4) k_hash_rows_multi(
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    u32 seg = find_seg(start, nseg, blockIdx.x);
+    const u32 blk = (u32)grid_block();
+    if (blk >= start[nseg]) return;
+    u32 seg = find_seg(start, nseg, blk);
     HashArgs A = args[seg];
-    hash_rows_body(A, blockIdx.x - start[seg], W);
+    hash_rows_body(A, blk - start[seg], W);
 }
 
 // Column-chunk absorption for the streaming ("frugal") commit: each row's
@@ -157,7 +162,7 @@ __global__ void __launch_bounds__(kHashThreads, 4)
     tip5::load_tables(T);
     const Wv W = tip5::make_wave(T);
     __syncthreads();
-    const u64 row = wave_first<Wv>(blockIdx.x) + W.n;
+    const u64 row = wave_first<Wv>(grid_block()) + W.n;
     const u64 r = row < rows ? row : rows - 1;  // lanes past the end repeat the last row
     u64 s[Wv::kWords];
 #pragma unroll
@@ -190,7 +195,7 @@ __global__ void __launch_bounds__(kHashThreads, 4) k_permutation(u64* __restrict
     tip5::load_tables(T);
     const Wv W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first<Wv>(blockIdx.x) + W.n;
+    const u64 i = wave_first<Wv>(grid_block()) + W.n;
     const u64* in = st + (i < num ? i : num - 1) * tip5::STATE;
     u64 s[Wv::kWords];
 #pragma unroll
@@ -211,7 +216,7 @@ __global__ void __launch_bounds__(kHashThreads) k_permutation_rounds(u64* __rest
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first<tip5::Wave>(blockIdx.x) + W.n;
+    const u64 i = wave_first<tip5::Wave>(grid_block()) + W.n;
     const bool live = i < num;
     const u64* in = st + (live ? i : num - 1) * tip5::STATE + W.g;
     u64* tr = trace && live ? trace + i * (count + 1) * tip5::STATE + W.g : nullptr;
@@ -253,7 +258,7 @@ __global__ void __launch_bounds__(kHashThreads, 4) k_hash_pairs(const u64* __res
     tip5::load_tables(T);
     const Wv W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first<Wv>(blockIdx.x) + W.n;
+    const u64 i = wave_first<Wv>(grid_block()) + W.n;
     const u64 r = i < count ? i : count - 1;
     u64 s[Wv::kWords], x[kRateWords<Wv>];
     rate_elements(x, W, [&](u32 k) { return k < 5 ? left[5 * r + k] : right[5 * r + k - 5]; });
@@ -303,7 +308,7 @@ __global__ void __launch_bounds__(kHashThreads) k_merkle_level(MerkleArgs A) {
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first<tip5::Wave>(blockIdx.x) + W.n;
+    const u64 i = wave_first<tip5::Wave>(grid_block()) + W.n;
     const u64* c = A.src + 10 * i;
     u64 s[tip5::WORDS], x[3];
     rate_elements(x, W, [&](u32 k) { return c[k]; });
@@ -328,9 +333,11 @@ __global__ void __launch_bounds__(kMerkleThreads) k_merkle_subtrees_multi(
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    u32 seg = find_seg(start, nseg, blockIdx.x);
+    const u32 blk = (u32)grid_block();
+    if (blk >= start[nseg]) return;
+    u32 seg = find_seg(start, nseg, blk);
     const MerkleArgs& A = args[seg];  // read in place: a private copy would spill dst[]
-    merkle_body(A, blockIdx.x - start[seg], W, buf);
+    merkle_body(A, blk - start[seg], W, buf);
 }
 
 // Gather: out[q] = node with heap index idx[q] (1 <= idx < 2n) of a tree in
@@ -356,6 +363,14 @@ __global__ void k_gather_heap(const u64* __restrict__ tree, u64 n, u32 logn, int
 
 // ------------------------------------------------------------------ host side
 
+// A sponge takes 4 threads or 16, and a launch can have 2^32 threads along one grid
+// axis (more are cut off without an error): past 2^31 the blocks go on along the
+// second one.  Kernels take grid_block() and leave out the last row's surplus.
+static dim3 hash_grid(u64 blocks, u32 threads) {
+    const u64 row = (1ull << 31) / threads;
+    return blocks <= row ? dim3((u32)blocks) : dim3((u32)row, (u32)((blocks + row - 1) / row));
+}
+
 // The 16-sponge form, or the four-sponge one where that leaves few waves.
 #define TVH_SPONGES(count, kernel, ...)                                                            \
     do {                                                                                           \
@@ -363,8 +378,8 @@ __global__ void k_gather_heap(const u64* __restrict__ tree, u64 n, u32 logn, int
             hipLaunchKernelGGL(kernel<tip5::QuadWave>, dim3(quad_blocks(count)), dim3(kHashThreads), \
                                0, st, __VA_ARGS__);                                                \
         else                                                                                       \
-            hipLaunchKernelGGL(kernel<tip5::Wave>, dim3(sponge_blocks(count)), dim3(kHashThreads), \
-                               0, st, __VA_ARGS__);                                                \
+            hipLaunchKernelGGL(kernel<tip5::Wave>, hash_grid(sponge_blocks(count), kHashThreads), \
+                               dim3(kHashThreads), 0, st, __VA_ARGS__);                            \
     } while (0)
 template <class Wv>
 constexpr auto k_absorb_chunk_final = k_absorb_chunk<true, Wv>;
@@ -459,8 +474,8 @@ int launch_permutation(u64* states, u64 num, hipStream_t st) {
 int launch_permutation_rounds(u64* states, u64 num, u32 first, u32 count, u64* trace,
                               hipStream_t st) {
     if (num == 0) return TVH_OK;
-    hipLaunchKernelGGL(k_permutation_rounds, dim3(sponge_blocks(num)), dim3(kHashThreads), 0, st,
-                       states, num, first, count, trace);
+    hipLaunchKernelGGL(k_permutation_rounds, hash_grid(sponge_blocks(num), kHashThreads),
+                       dim3(kHashThreads), 0, st, states, num, first, count, trace);
     return check_launch();
 }
 
@@ -513,7 +528,8 @@ int launch_merkle_levels(u64* tree, u64 n, int layout, hipStream_t st) {
             hipLaunchKernelGGL(k_merkle_subtrees, dim3(g.blocks),
                                dim3((g.args.T + tip5::QUAD - 1) / tip5::QUAD * 64), 0, st, g.args);
         else
-            hipLaunchKernelGGL(k_merkle_level, dim3(g.blocks), dim3(kHashThreads), 0, st, g.args);
+            hipLaunchKernelGGL(k_merkle_level, hash_grid(g.blocks, kHashThreads), dim3(kHashThreads), 0,
+                               st, g.args);
         int rc = check_launch();
         if (rc) return rc;
     }
@@ -523,16 +539,16 @@ int launch_merkle_levels(u64* tree, u64 n, int layout, hipStream_t st) {
 int launch_hash_rows_multi(const HashArgs* d_args, const u32* d_start, u32 nseg, u32 blocks,
                            hipStream_t st) {
     if (!blocks) return TVH_OK;
-    hipLaunchKernelGGL(k_hash_rows_multi, dim3(blocks), dim3(kHashThreads), 0, st, d_args, d_start,
-                       nseg);
+    hipLaunchKernelGGL(k_hash_rows_multi, hash_grid(blocks, kHashThreads), dim3(kHashThreads), 0, st,
+                       d_args, d_start, nseg);
     return check_launch();
 }
 
 int launch_merkle_multi(const MerkleArgs* d_args, const u32* d_start, u32 nseg, u32 blocks,
                         hipStream_t st) {
     if (!blocks) return TVH_OK;
-    hipLaunchKernelGGL(k_merkle_subtrees_multi, dim3(blocks), dim3(kMerkleThreads), 0, st, d_args,
-                       d_start, nseg);
+    hipLaunchKernelGGL(k_merkle_subtrees_multi, hash_grid(blocks, kMerkleThreads),
+                       dim3(kMerkleThreads), 0, st, d_args, d_start, nseg);
     return check_launch();
 }
 

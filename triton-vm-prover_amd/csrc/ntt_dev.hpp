@@ -387,10 +387,13 @@ struct Tile {
     }
 };
 
-// Global to LDS; scale(t, i, iq, x) changes four elements i + iq[v] of transform
-// t (TF) on the way.  valid: transforms of the tile that exist.
+// Global to LDS; scale(t, tq, i, iq, x) changes four elements i + iq[v] of
+// transforms t + tq[v] on the way.  valid: transforms of the tile that exist.
 // log_e: transforms e*C + u of each run of C * 2^log_e, C = 2^log_c, change places
 // to u * 2^log_e + e (TF).
+struct Unscaled {
+    __device__ __forceinline__ void operator()(u32, const u32 (&)[4], u32, const u32 (&)[4], u64 (&)[4]) const {}
+};
 template <class Z, bool TF, class Scale>
 __device__ __forceinline__ void load_tile(u64* buf, const Place<const u64>& from, u32 valid,
                                           const Scale& scale, u32 log_c = 0, u32 log_e = 0) {
@@ -416,8 +419,9 @@ __device__ __forceinline__ void load_tile(u64* buf, const Place<const u64>& from
 #pragma unroll
     for (u32 q = 0; q < Z::kPer; q += 4) {
         u64 y[4] = {x[q], x[q + 1], x[q + 2], x[q + 3]};
+        const u32 tq[4] = {Ti::tq(q), Ti::tq(q + 1), Ti::tq(q + 2), Ti::tq(q + 3)};
         const u32 iq[4] = {Ti::iq(q), Ti::iq(q + 1), Ti::iq(q + 2), Ti::iq(q + 3)};
-        scale(T.t, T.i, iq, y);
+        scale(T.t, tq, T.i, iq, y);
 #pragma unroll
         for (u32 v = 0; v < 4; v++) lane_p[Ti::tq(q + v) * Z::pitch + lds_index(iq[v])] = y[v];
     }
@@ -606,7 +610,7 @@ __device__ __forceinline__ void step1_body(const Step1Args& A, const NttScaleDev
     typedef Shape<LT, LOGL> Z;
     const Step1<INV, SCALED> P(A, S, rt, blk, Z::logNT);
     load_tile<Z, true>(lds, P.in, P.B.valid,
-                       [&](u32 t, u32 i, const u32 (&iq)[4], u64 (&x)[4]) {
+                       [&](u32 t, const u32 (&)[4], u32 i, const u32 (&iq)[4], u64 (&x)[4]) {
                            if constexpr (SCALED) P.scale(t, i, iq, x);
                        });
     dft_block<Z>(lds, Z::logNT, rt.dft[INV], rt.r4096[INV]);
@@ -616,28 +620,6 @@ __device__ __forceinline__ void step1_body(const Step1Args& A, const NttScaleDev
     FactorChain F(gl::mul_lazy(P.constant(T.t), twiddle(rt, INV, n2 * T.i, A.logN)),
                   twiddle(rt, INV, n2 * (Z::L / 16), A.logN));
     store_tile<Z, true>(lds, P.out, P.B.valid, [&](u64 (&x)[4]) { F.apply(x); });
-}
-__device__ __forceinline__ void step1_small(const Step1Args& A, const NttScaleDev& S, u64 blk,
-                                            const Roots& rt) {
-    const Step1<false, true> P(A, S, rt, blk, kSmallLogNT);
-    const gl::JoinConsts J = gl::join_consts();
-    small_groups(A.a, [&](const u32 (&t)[4], const u32 (&i)[4]) {
-        u64 x[4];
-#pragma unroll
-        for (int v = 0; v < 4; v++) {  // (each in a transform of its own)
-            const u32 zero[4] = {0, 0, 0, 0};
-            x[v] = t[v] < P.B.valid ? P.in.base[P.in.off(t[v], i[v])] : 0;
-            u64 y[4] = {x[v], x[v], x[v], x[v]};
-            P.scale(t[v], i[v], zero, y);
-            x[v] = y[0];
-        }
-        small_dft(A.a, rt.dft[0], J, x);
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const u64 f = gl::mul_lazy(P.constant(t[v]), twiddle(rt, 0, (P.B.t0 + t[v]) * i[v], A.logN));
-            if (t[v] < P.B.valid) P.out.base[P.out.off(t[v], i[v])] = gl::mul_lazy(x[v], f);
-        }
-    });
 }
 
 // ---------------------------------------------------------------- LDE step 2
@@ -803,7 +785,7 @@ __device__ __forceinline__ void lde_cosets_body(const LdeArgs& A, u64 blk, const
     typedef Tile<Z, false> Ti;
     const Rows P(A, blk, Z::logNT);
     const Ti T;
-    load_tile<Z, false>(lds, P.in, Z::NT, [](u32, u32, const u32 (&)[4], u64 (&)[4]) {});
+    load_tile<Z, false>(lds, P.in, Z::NT, Unscaled{});
     dft_block<Z>(lds, Z::logNT, rt.dft[1], rt.r4096[1]);
     u64 f[Z::kPer];
     auto factors = [&](u32 s) {
@@ -887,7 +869,7 @@ __device__ __forceinline__ void lde_step3_body(const Step3Args& A, u64 blk, cons
     u64* col = A.out + B.c * A.M + B.t0;
     // every input of the block is read before any output is written
     load_tile<Z, true>(lds, Place<const u64>{col, 0, 1, 0, 1u << logQ}, B.valid,
-                       [](u32, u32, const u32 (&)[4], u64 (&)[4]) {}, A.log_c, A.log_c ? A.logE : 0);
+                       Unscaled{}, A.log_c, A.log_c ? A.logE : 0);
     dft_block<Z>(lds, Z::logNT, rt.dft[0], rt.r4096[0]);
     store_tile<Z, true>(lds, Place<u64>{col, 0, 1, 0, 1u << logQ}, B.valid,
                         [](u64 (&x)[4]) { gl::canon_n(x); });
@@ -924,6 +906,8 @@ int set_attributes_step1(int lds_bytes);
 // ntt_step2.hip
 int launch_k_ntt_step2(bool inv, u32 lt, const LaunchShape& g, hipStream_t st, const u64* src,
                        u64* dst, u32 logN, u32 a, u64 cols, u64 ninv, const Roots& rt);
+int launch_k_ntt_cols_scaled(const LaunchShape& g, hipStream_t st, const u64* src, u64* dst, u32 logN,
+                             u64 cols, const NttScaleDev& S, const Roots& rt);
 int set_attributes_step2(int lds_bytes);
 // lde_rows.hip
 int launch_k_lde_rows(u32 lt, const LaunchShape& g, hipStream_t st, const LdeArgs& A, const Roots& rt);

@@ -424,9 +424,9 @@ int launch_ntt_batched(const u64* src, u64* dst, u64 n, u64 cols, bool inverse, 
     // the kernel that reads them next: evaluating a coset of 2^19 x 379 takes 2.17 ms
     // in column order, 2.07 as here, 1.97 in 2^13 tiles; with the row hashes after it
     // 4.54, 4.46 and 4.66.
-    u32 a = logN <= 14 ? logN / 2 : logN <= 20 ? 8 : logN - 12;
-    // up to 2^12 rows the row step alone (2^10 x 100: 9.4 us in 2^12 tiles, 19.6 in 2^14)
-    if (logN <= 12 && !scale) a = 0;
+    // Up to 2^12 rows the row step alone (2^10 x 100: 9.4 us in 2^12 tiles, 19.6 in
+    // 2^14), the scaled form too.
+    const u32 a = logN <= 12 ? 0 : logN <= 14 ? logN / 2 : logN <= 20 ? 8 : logN - 12;
     const u32 b = logN - a;
     const u32 col_lt = logN > 22 ? LOG_TILE : (cols << logN) < (1ull << 23) && a < 10 ? 12 : 13;
     const u32 row_lt = a == 0 ? 12 : std::min(std::max(b + 3, 12u), (u32)LOG_TILE);
@@ -436,11 +436,12 @@ int launch_ntt_batched(const u64* src, u64* dst, u64 n, u64 cols, bool inverse, 
         S = NttScaleDev{scale->tables, scale->tables + (1ull << a), scale->rand, scale->k,
                         scale->delta};
         int rc;
-        if ((rc = launch_pow_table(scale->tables, gl::pow(scale->base, 1ull << b), 1ull << a, st)) ||
+        if ((a && (rc = launch_pow_table(scale->tables, gl::pow(scale->base, 1ull << b), 1ull << a, st))) ||
             (rc = launch_pow_table(scale->tables + (1ull << a), scale->base, 1ull << b, st)))
             return rc;
     }
-    // step 1 writes each group of columns to the scratch, step 2 writes it back
+    // step 1 writes each group of columns to the scratch, step 2 writes it back (the
+    // row step alone needs no scratch, and asks for it all the same)
     u64 group = scratch_elems / n;
     if (!scratch || group == 0)
         return set_error(TVH_ERR_INVALID_ARG, "NTT scratch of %llu elements < n = %llu",
@@ -452,23 +453,20 @@ int launch_ntt_batched(const u64* src, u64* dst, u64 n, u64 cols, bool inverse, 
         u64 g = cols - c0 < group ? cols - c0 : group;
         const u64* sg = src + c0 * n;  // step 1 reads the group from src
         u64* d = dst + c0 * n;         // step 2 writes it to dst
-        const bool one_step = a == 0 && !scale;
-        if (!one_step) {
+        NttScaleDev Sg = S;
+        if (Sg.rand) Sg.rand += c0 * Sg.k;  // the group's first column
+        if (a) {
             const LaunchShape s1 = launch_shape(col_lt, a, b, g, false);
             Step1Args A{sg, n, scratch, n, logN, a, 1u, inverse ? ninv : 1, s1.blocks};
-            if (scale) {
-                NttScaleDev Sg = S;
-                if (Sg.rand) Sg.rand += c0 * Sg.k;  // the group's first column
-                rc = launch_k_step1_scaled(col_lt, s1, st, A, Sg, ds->roots);
-            } else {
-                rc = launch_k_step1(inverse, col_lt, s1, st, A, ds->roots);
-            }
+            rc = scale ? launch_k_step1_scaled(col_lt, s1, st, A, Sg, ds->roots)
+                       : launch_k_step1(inverse, col_lt, s1, st, A, ds->roots);
             if (rc) return rc;
         }
         const LaunchShape s2 = launch_shape(row_lt, b, a, g, a == 0);
-        if ((rc = launch_k_ntt_step2(inverse, row_lt, s2, st, one_step ? sg : scratch, d, logN, a, g,
-                                     ninv, ds->roots)))
-            return rc;
+        rc = scale && !a ? launch_k_ntt_cols_scaled(s2, st, sg, d, logN, g, Sg, ds->roots)
+                         : launch_k_ntt_step2(inverse, row_lt, s2, st, a ? scratch : sg, d, logN, a, g, ninv,
+                                              ds->roots);
+        if (rc) return rc;
     }
     return TVH_OK;
 }

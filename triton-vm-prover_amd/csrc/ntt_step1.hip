@@ -13,11 +13,6 @@ __global__ void __launch_bounds__(1 << (LT - 4), 4) k_step1_scaled(Step1Args A, 
                                                                    Roots rt) {
     step1_body<false, true, LT, LOGL>(A, S, blockIdx.x, rt);
 }
-// columns of at most 16 points (short scaled transforms; every other split has
-// longer columns)
-__global__ void __launch_bounds__(kSmallThreads) k_step1_small(Step1Args A, NttScaleDev S, Roots rt) {
-    step1_small(A, S, blockIdx.x, rt);
-}
 
 template <int LT>
 __global__ void __launch_bounds__(1 << (LT - 4), 4) k_step1_multi(const Step1Args* __restrict__ args,
@@ -54,10 +49,6 @@ int launch_k_step1(bool inv, u32 lt, const LaunchShape& g, hipStream_t st, const
 int launch_k_step1_scaled(u32 lt, const LaunchShape& g, hipStream_t st, const Step1Args& A,
                           const NttScaleDev& S, const Roots& rt) {
     const dim3 blocks(g.blocks), tpb(g.threads);
-    if (A.a <= 4) {
-        hipLaunchKernelGGL(k_step1_small, blocks, tpb, 0, st, A, S, rt);
-        return check_launch();
-    }
     with_length(A.a, [&](auto l) {
         constexpr int L = decltype(l)::value;
 #define TVH_STEP1(T) hipLaunchKernelGGL((k_step1_scaled<T, L>), blocks, tpb, g.lds, st, A, S, rt)

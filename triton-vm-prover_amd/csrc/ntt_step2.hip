@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(1 << (LT - 4), 4) k_ntt_step2(const u64* src, 
     extern __shared__ u64 lds[];
     typedef Shape<LT, LOGL> Z;
     const RowStep<INV, COLS> P(src, dst, logN, a, cols, ninv, blockIdx.x, Z::logNT, gridDim.x);
-    load_tile<Z, false>(lds, P.in, P.B.valid, [](u32, u32, const u32 (&)[4], u64 (&)[4]) {});
+    load_tile<Z, false>(lds, P.in, P.B.valid, Unscaled{});
     dft_block<Z>(lds, Z::logNT, rt.dft[INV], rt.r4096[INV]);
     store_tile<Z, !COLS>(lds, P.out, P.B.valid, [&](u64 (&x)[4]) { P.finish(x); });
 }
@@ -58,6 +58,75 @@ __global__ void __launch_bounds__(kSmallThreads) k_ntt_step2_small(const u64* sr
         for (int v = 0; v < 4; v++)
             if (t[v] < P.B.valid) P.out.base[P.out.off(t[v], i[v])] = x[v];
     });
+}
+
+// Whole transforms of a column each, forward, of a scaled input: element i of
+// column c enters as (x + [i < k] rand[c*k + i] * delta) * base^i, base^i = p2[i]
+// (NttScaleDev, N1 = 1).  Blocks take as many columns as a tile holds: with the
+// column and row steps of longer transforms a block has one column alone, and 2^21
+// columns of 4 rows took 9.4 ms.
+struct ScaledCols {
+    const NttScaleDev& S;
+    RowStep<false, true> P;
+    __device__ __forceinline__ ScaledCols(const u64* src, u64* dst, u32 logN, u64 cols, const NttScaleDev& S_,
+                                          u64 blk, u32 log_nt)
+        : S(S_), P(src, dst, logN, 0, cols, 1, blk, log_nt) {}
+    __device__ __forceinline__ void scale(u32 t, const u32 (&tq)[4], u32 i, const u32 (&iq)[4],
+                                          u64 (&x)[4]) const {
+        u64 f[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) f[v] = load_at(S.p2 + iq[v], i * 8);
+        if (S.k) {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                if (iq[v] + i < S.k && t + tq[v] < P.B.valid)
+                    x[v] = gl::add(x[v], gl::mul(S.rand[(P.B.c + t + tq[v]) * S.k + iq[v] + i], S.delta));
+        }
+        gl::mul_n(x, x, f);
+    }
+};
+template <int LOGL>
+__global__ void __launch_bounds__(1 << 8, 4) k_ntt_cols_scaled(const u64* src, u64* dst, u64 cols,
+                                                               NttScaleDev S, Roots rt) {
+    extern __shared__ u64 lds[];
+    typedef Shape<12, LOGL> Z;
+    const ScaledCols C(src, dst, LOGL, cols, S, blockIdx.x, Z::logNT);
+    load_tile<Z, false>(lds, C.P.in, C.P.B.valid,
+                        [&](u32 t, const u32 (&tq)[4], u32 i, const u32 (&iq)[4], u64 (&x)[4]) {
+                            C.scale(t, tq, i, iq, x);
+                        });
+    dft_block<Z>(lds, Z::logNT, rt.dft[0], rt.r4096[0]);
+    store_tile<Z, false>(lds, C.P.out, C.P.B.valid, [&](u64 (&x)[4]) { C.P.finish(x); });
+}
+// columns of at most 16 elements
+__global__ void __launch_bounds__(kSmallThreads) k_ntt_cols_scaled_small(const u64* src, u64* dst, u32 logN,
+                                                                         u64 cols, NttScaleDev S, Roots rt) {
+    const ScaledCols C(src, dst, logN, cols, S, blockIdx.x, kSmallLogNT);
+    const gl::JoinConsts J = gl::join_consts();
+    small_groups(logN, [&](const u32 (&t)[4], const u32 (&i)[4]) {
+        u64 x[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) x[v] = t[v] < C.P.B.valid ? C.P.in.base[C.P.in.off(t[v], i[v])] : 0;
+        C.scale(0, t, 0, i, x);
+        small_dft(logN, rt.dft[0], J, x);
+        C.P.finish(x);
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (t[v] < C.P.B.valid) C.P.out.base[C.P.out.off(t[v], i[v])] = x[v];
+    });
+}
+
+int launch_k_ntt_cols_scaled(const LaunchShape& g, hipStream_t st, const u64* src, u64* dst, u32 logN,
+                             u64 cols, const NttScaleDev& S, const Roots& rt) {
+    const dim3 blocks(g.blocks), tpb(g.threads);
+    if (logN <= 4)
+        hipLaunchKernelGGL(k_ntt_cols_scaled_small, blocks, tpb, 0, st, src, dst, logN, cols, S, rt);
+    else
+        with_length(logN, [&](auto l) {
+            hipLaunchKernelGGL(k_ntt_cols_scaled<decltype(l)::value>, blocks, tpb, g.lds, st, src, dst, cols,
+                               S, rt);
+        });
+    return check_launch();
 }
 
 template <bool INV, bool COLS>

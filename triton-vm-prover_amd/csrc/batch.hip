@@ -66,10 +66,10 @@ int tvh_batch_plan_create(const tvh_table_desc* tables, size_t count, tvh_batch_
     DeviceState* ds = current_device();
     if (!ds) return TVH_ERR_DEVICE;
     std::vector<Step1Args> s1;
-    std::vector<LdeArgs> s2[3];  // by row tile: 2^12, 2^13, 2^14
+    std::vector<LdeArgs> s2[4];  // by row tile: 2^12, 2^13, 2^14, kBatchShort
     std::vector<Step3Args> s3;
-    std::vector<u32> b1, b2[3], b3;
-    std::vector<size_t> l1, l2[3], l3;
+    std::vector<u32> b1, b2[4], b3;
+    std::vector<size_t> l1, l2[4], l3;
     std::vector<HashArgs> h;
     std::vector<u32> hb;
     std::vector<std::vector<MerkleArgs>> ma;
@@ -125,7 +125,7 @@ int tvh_batch_plan_create(const tvh_table_desc* tables, size_t count, tvh_batch_
     plan->device = ds->device;
     std::vector<uint8_t> blob;
     add_phase(blob, plan->lde[LDE_PHASE_STEP1], s1, b1, l1);
-    for (int q = 0; q < 3; q++) add_phase(blob, plan->lde[LDE_PHASE_ROWS + q], s2[q], b2[q], l2[q]);
+    for (int q = 0; q < 4; q++) add_phase(blob, plan->lde[LDE_PHASE_ROWS + q], s2[q], b2[q], l2[q]);
     add_phase(blob, plan->lde[LDE_PHASE_STEP3], s3, b3, l3);
     add_phase(blob, plan->hash, h, hb, {});
     plan->merkle.resize(ma.size());

@@ -10,9 +10,14 @@ __global__ void __launch_bounds__(1 << (LT - 4), 4) k_lde_rows(LdeArgs A, Roots 
 __global__ void __launch_bounds__(kCosetsThreads, 4) k_lde_cosets(LdeArgs A, Roots rt) {
     lde_cosets_body(A, blockIdx.x, rt);
 }
-// transforms of at most 16 points
-__global__ void __launch_bounds__(kSmallThreads) k_lde_rows_small(LdeArgs A, Roots rt) {
-    lde_rows_small(A, blockIdx.x, rt);
+// columns of at most 16 elements (two waves a SIMD: both matrices stay in registers)
+__global__ void __launch_bounds__(kShortThreads, 2) k_lde_short(LdeArgs A, Roots rt) {
+    lde_short_body(A, blockIdx.x, rt);
+}
+__global__ void __launch_bounds__(kShortThreads, 2)
+    k_lde_short_multi(const LdeArgs* __restrict__ args, const u32* __restrict__ start, u32 nseg, Roots rt) {
+    const u32 seg = find_segment(start, nseg, blockIdx.x);
+    lde_short_body(args[seg], blockIdx.x - start[seg], rt);
 }
 
 // (longer tiles only where E * N2 needs them: N2 of at least 2^(LT - 4))
@@ -22,7 +27,6 @@ __global__ void __launch_bounds__(1 << (LT - 4), 4)
     const u32 seg = find_segment(start, nseg, blockIdx.x);
     const LdeArgs& A = args[seg];  // read in place
     const u64 blk = blockIdx.x - start[seg];
-    if (LT == 12 && A.logN - A.a <= 4) return lde_rows_small(A, blk, rt);
     with_length(A.logN - A.a, [&](auto l) {
         constexpr int L = decltype(l)::value;
         if constexpr (LT == 12 || L >= LT - 4) lde_rows_body<LT, L>(A, blk, rt);
@@ -31,8 +35,8 @@ __global__ void __launch_bounds__(1 << (LT - 4), 4)
 
 int launch_k_lde_rows(u32 lt, const LaunchShape& g, hipStream_t st, const LdeArgs& A, const Roots& rt) {
     const dim3 blocks(g.blocks), tpb(g.threads);
-    if (A.logN - A.a <= 4) {
-        hipLaunchKernelGGL(k_lde_rows_small, blocks, tpb, 0, st, A, rt);
+    if (A.products) {
+        hipLaunchKernelGGL(k_lde_short, blocks, tpb, g.lds, st, A, rt);
         return check_launch();
     }
     if (A.cosets) {
@@ -55,8 +59,9 @@ int launch_k_lde_rows(u32 lt, const LaunchShape& g, hipStream_t st, const LdeArg
 
 int launch_k_lde_rows_multi(u32 lt, const LdeArgs* args, const u32* start, u32 nseg, u32 blocks,
                             size_t lds, hipStream_t st, const Roots& rt) {
-    const dim3 grid(blocks), tpb(1u << (lt - 4));
-    if (lt == 12) hipLaunchKernelGGL(k_lde_rows_multi<12>, grid, tpb, lds, st, args, start, nseg, rt);
+    const dim3 grid(blocks), tpb(lt == kBatchShort ? kShortThreads : 1u << (lt - 4));
+    if (lt == kBatchShort) hipLaunchKernelGGL(k_lde_short_multi, grid, tpb, lds, st, args, start, nseg, rt);
+    else if (lt == 12) hipLaunchKernelGGL(k_lde_rows_multi<12>, grid, tpb, lds, st, args, start, nseg, rt);
     else if (lt == 13) hipLaunchKernelGGL(k_lde_rows_multi<13>, grid, tpb, lds, st, args, start, nseg, rt);
     else hipLaunchKernelGGL(k_lde_rows_multi<14>, grid, tpb, lds, st, args, start, nseg, rt);
     return check_launch();

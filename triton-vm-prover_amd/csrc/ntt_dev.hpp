@@ -623,20 +623,21 @@ __device__ __forceinline__ void step1_body(const Step1Args& A, const NttScaleDev
 }
 
 // ---------------------------------------------------------------- LDE step 2
-// Randomizer term of coefficient r of column c in coset s (canonical).
-__device__ __forceinline__ u64 rand_term(const LdeArgs& A, u64 c, u32 s, u64 r) {
-    const RandSpec& rs = A.rs;
+// Randomizer r of column c (null: its limb carries none).
+__device__ __forceinline__ const u64* rand_at(const RandSpec& rs, u64 c, u64 r) {
     u32 limb = (u32)(c % rs.group);
-    if (!((rs.limb_mask >> limb) & 1)) return 0;
-    const u64* p = rs.ptr + (c / rs.group) * rs.group_stride + limb * rs.limb_stride +
-                   r * rs.elem_stride;
+    if (!((rs.limb_mask >> limb) & 1)) return nullptr;
+    return rs.ptr + (c / rs.group) * rs.group_stride + limb * rs.limb_stride + r * rs.elem_stride;
+}
+// Factor of randomizer r in coset s.
+__device__ __forceinline__ u64 rand_factor(const LdeArgs& A, u32 s, u64 r) {
     // select delta_n[s] without a dynamic index (a dynamic index into the
     // by-value kernel argument would copy it to scratch)
     u64 d = A.delta_n[0];
 #pragma unroll
     for (u32 i = 1; i < 16; i++)
         if (s == i) d = A.delta_n[i];
-    return gl::mul(gl::mul(*p, d), gl::pow(A.toff, r));
+    return gl::mul(d, gl::pow(A.toff, r));
 }
 
 // A block takes NT rows (c, k1) (NT * E * N2 = 2^LT) of Y: inverse row DFT to
@@ -661,12 +662,13 @@ struct Rows {
     }
     // k1 of row t (a column of its own: 0)
     __device__ __forceinline__ u32 k1(u32 t) const { return A.a ? B.t0 + t : 0; }
-    // coefficient k2 of row t with its randomizer term: element k2 of row k1 is
+    // randomizer term of element k2 of row t in coset sl (canonical): the element is
     // coefficient k1 + k2 * N1, which carries one when below rand_len
-    __device__ __forceinline__ u64 randomized(u32 t, u32 sl, u32 k2, u64 x) const {
+    __device__ __forceinline__ u64 rand_term(u32 t, u32 sl, u32 k2) const {
         const u64 r = k1(t) + ((u64)k2 << A.a);
-        if (r >= A.rs.k || t >= B.valid) return x;
-        return gl::add(gl::canon(x), rand_term(A, A.a ? B.c : B.c + t, sl, r));
+        if (r >= A.rs.k || t >= B.valid) return 0;
+        const u64* p = rand_at(A.rs, A.a ? B.c : B.c + t, r);
+        return p ? gl::mul(*p, rand_factor(A, sl, r)) : 0;
     }
     // The randomizer terms of the scaled coefficients of 2^log_rows rows in cosets
     // s0 .. s0 + 2^log_s - 1 in LDS (transform t * 2^log_s + s): the few elements
@@ -686,7 +688,7 @@ struct Rows {
             const u32 k2 = e >> (log_s + log_rows);
             u64* const p = lds + ((t << log_s) + s) * Z::pitch + lds_index(k2);
             *p = gl::add(gl::canon(*p),
-                         gl::mul(randomized(t, s0 + s, k2, 0), A.pb[((s0 + s) << logL) + k2]));
+                         gl::mul(rand_term(t, s0 + s, k2), A.pb[((s0 + s) << logL) + k2]));
         }
     }
 };
@@ -829,32 +831,75 @@ __device__ __forceinline__ void lde_cosets_body(const LdeArgs& A, u64 blk, const
         out.base += 1u << A.log_c;
     }
 }
-// Rows of at most 16 elements: a group's rows stay with their lanes, every coset
-// is computed from registers (a row is read before it is overwritten).
-__device__ __forceinline__ void lde_rows_small(const LdeArgs& A, u64 blk, const Roots& rt) {
-    const u32 a = A.a, b = A.logN - a;
-    const Rows P(A, blk, kSmallLogNT);
+// Columns of N <= 16 elements, E * N outputs each (no column step).  One matrix
+// product takes 256 outputs, which are whole columns and lie together: its transforms
+// are all cosets of 256 / (E N) columns, cosets fastest, each with the column's
+// inverse transform of its own (the cosets one after the other in a lane cost their
+// latency each: 2^4 rows in 16 cosets took 75 us, here they take 4).  What
+// depends on coset and element alone is the lane's for the whole kernel.  The
+// outputs go through LDS to be stored in order.  A wave takes A.products of them.
+constexpr u32 kShortThreads = 256, kShortOut = 256, kShortPitch = kShortOut + kShortOut / 16;
+constexpr u32 kShortLds = (kShortThreads / 64 * kShortPitch + 64) * 8;  // outputs; starts of both matrices
+__device__ __forceinline__ void lde_short_body(const LdeArgs& A, u64 blk, const Roots& rt) {
+    extern __shared__ u64 lds[];
+    const u32 logN = A.logN, sub = 4 - logN;
+    const u32 lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    constexpr u32 kWaves = kShortThreads / 64;
+    u32* const starts = (u32*)(lds + kWaves * kShortPitch);
+    const u32 set = (logN ? logN - 1 : 0) * kDftWords;  // (N = 1: no product)
+    if (threadIdx.x < 128)
+        starts[threadIdx.x] = (rt.dft[threadIdx.x < 64] + set + kDftStarts)[threadIdx.x & 63];
+    const Matrix inv = load_matrix(rt.dft[1] + set, starts), fwd = load_matrix(rt.dft[0] + set, starts + 64);
     const gl::JoinConsts J = gl::join_consts();
-    small_groups(b, [&](const u32 (&t)[4], const u32 (&i)[4]) {
+    // element i of transform q, in column t of the product's, coset s
+    u32 t[4], from[4], to[4];
+    u64 pb[4], pa[4], rf[4];
+#pragma unroll
+    for (u32 v = 0; v < 4; v++) {
+        const u32 e = 4 * v + g, q = (n << sub) + (e & ((1u << sub) - 1)), i = e >> sub;
+        const u32 s = q & (A.E - 1), o = (((q >> A.logE) << logN) + i) * A.E + s;
+        t[v] = q >> A.logE;
+        from[v] = ((t[v] << logN) + i) * 8;
+        to[v] = o + (o >> 4);
+        pb[v] = load_at(A.pb, ((s << logN) + i) * 8);
+        pa[v] = load_at(A.pa, s * 8);
+        rf[v] = i < A.rs.k ? rand_factor(A, s, i) : 0;
+    }
+    u64* const buf = lds + wave_index() * kShortPitch;
+    const u32 log_cols = 8 - logN - A.logE;  // columns of a product
+    __syncthreads();
+#pragma unroll 1
+    for (u32 j = 0; j < A.products; j++) {
+        const u64 p = (blk * A.products + j) * kWaves + wave_index(), c0 = p << log_cols;
+        if (c0 >= A.cols) break;
+        const u32 valid = A.cols - c0 < 1u << log_cols ? (u32)(A.cols - c0) : 1u << log_cols;
         u64 x[4];
 #pragma unroll
-        for (int v = 0; v < 4; v++) x[v] = t[v] < P.B.valid ? P.in.base[P.in.off(t[v], i[v])] : 0;
-        small_dft(b, rt.dft[1], J, x);
-        for (u32 sl = 0; sl < A.E; sl++) {
-            u64 y[4];
+        for (u32 v = 0; v < 4; v++) x[v] = t[v] < valid ? load_at(A.src + (c0 << logN), from[v]) : 0;
+        if (logN) dft16(inv, J, x);
+        if (A.rs.k) {
 #pragma unroll
-            for (int v = 0; v < 4; v++)
-                y[v] = gl::mul_lazy(P.randomized(t[v], sl, i[v], x[v]), A.pb[(sl << b) + i[v]]);
-            small_dft(b, rt.dft[0], J, y);
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                if (t[v] >= P.B.valid) continue;
-                u64 f = A.pa[((u64)sl << a) + P.k1(t[v])];
-                if (a) f = gl::mul_lazy(f, twiddle(rt, 0, P.k1(t[v]) * i[v], A.logN));
-                P.out.base[P.out.off((t[v] << A.logE) + sl, i[v])] = gl::canon(gl::mul_lazy(y[v], f));
+            for (u32 v = 0; v < 4; v++) {
+                const u32 i = (4 * v + g) >> sub;
+                if (i >= A.rs.k || t[v] >= valid) continue;
+                const u64* r = rand_at(A.rs, c0 + t[v], i);
+                if (r) x[v] = gl::add(gl::canon(x[v]), gl::mul(*r, rf[v]));
             }
         }
-    });
+        gl::mul_n(x, x, pb);
+        if (logN) dft16(fwd, J, x);
+        gl::mul_n(x, x, pa);
+        gl::canon_n(x);
+#pragma unroll
+        for (u32 v = 0; v < 4; v++) buf[to[v]] = x[v];
+        wave_handoff();
+#pragma unroll
+        for (u32 v = 0; v < 4; v++) {
+            const u32 o = 64 * v + lane;
+            if (o >> (logN + A.logE) < valid) store_at(A.out + p * kShortOut, o * 8, buf[o + (o >> 4)]);
+        }
+        wave_handoff();
+    }
 }
 
 // ---------------------------------------------------------------- LDE step 3
@@ -911,6 +956,7 @@ int launch_k_ntt_cols_scaled(const LaunchShape& g, hipStream_t st, const u64* sr
 int set_attributes_step2(int lds_bytes);
 // lde_rows.hip
 int launch_k_lde_rows(u32 lt, const LaunchShape& g, hipStream_t st, const LdeArgs& A, const Roots& rt);
+// lt: as above, or kBatchShort
 int launch_k_lde_rows_multi(u32 lt, const LdeArgs* args, const u32* start, u32 nseg, u32 blocks,
                             size_t lds, hipStream_t st, const Roots& rt);
 int set_attributes_rows(int lds_bytes);

@@ -105,15 +105,16 @@ static u32 passes(u32 l) { return l <= 4 ? 1 : l <= 8 ? 2 : 3; }
 // the strided step).  A column step has at least 2^5 points (shorter ones leave
 // part of the matrices idle) and, if it can, at most 2^9: longer ones leave less
 // than a cache line of adjacent columns in a 2^13 tile (2^20 x 140, E = 4, in
-// 2^13 row tiles: 7.2 ms with 2^9, 13.5 with 2^12).  Above 2^12 columns the shape
-// is refused (a > 12).
+// 2^13 row tiles: 7.2 ms with 2^9, 13.5 with 2^12).  Rows have at least 2^5
+// elements too; where that cannot be (2^9 rows, E = 16, 2^12 tiles) the whole
+// transform takes the next tile.  Above 2^12 columns the shape is refused (a > 12).
 static u32 choose_split(u32 logN, u32 E, u32 row_lt) {
     u32 bmax = row_lt - log2u(E);
     if (bmax > 12) bmax = 12;
-    if (logN <= bmax) return 0;
+    if (logN <= bmax || logN < 10) return 0;
     if (logN - bmax > 12) return logN - bmax;
     u32 best = 0, cost = ~0u;
-    for (u32 a = logN - bmax > 5 ? logN - bmax : 5; a <= 9 && a < logN; a++) {
+    for (u32 a = logN - bmax > 5 ? logN - bmax : 5; a <= 9 && a + 5 <= logN; a++) {
         const u32 c = passes(a) + passes(logN - a);
         if (c < cost) {
             cost = c;
@@ -322,7 +323,17 @@ int prepare_lde(const u64* trace, u64 cols, u64 n, const RandSpec& rs, u64 toff,
         // (2^18 x 379, E = 8: LDE 10.1 against 8.4 ms; 2^19 x 264, E = 4: 7.6, 6.7).
         A.cosets = a > 0 && b == kCosetsLt && logE >= 2 && !batch;
         A.log_c = 0;
-        if (A.cosets) {  // whole runs to a block of step 3; 16 elements are a cache line
+        A.products = 0;
+        if (b <= 4) {  // a = 0
+            // waves for the whole GPU first, then up to 16 products each
+            const u64 products = ((cols << (b + logE)) + kShortOut - 1) / kShortOut;
+            const u64 waves = kShortThreads / 64;
+            A.products = (u32)std::min<u64>(std::max<u64>(products >> 13, 1), 16);
+            P->row_lt = kBatchShort;
+            P->g2.blocks = (u32)((products + waves * A.products - 1) / (waves * A.products));
+            P->g2.threads = kShortThreads;
+            P->g2.lds = kShortLds;
+        } else if (A.cosets) {  // whole runs to a block of step 3; 16 elements are a cache line
             const u32 log_nt = P->col_lt - a;
             A.log_c = log_nt > logE ? std::min(log_nt - logE, 4u) : 0;
             P->g2 = launch_shape(kCosetsLt, b, a, cols, false);
@@ -330,7 +341,7 @@ int prepare_lde(const u64* trace, u64 cols, u64 n, const RandSpec& rs, u64 toff,
             P->g2.lds += sizeof(u64) << kCosetsLt;
         } else {
             P->row_lt = std::max(b + logE, 12u);  // the shortest tile that holds a row's cosets
-            P->g2 = launch_shape(P->row_lt, b, a, cols, a == 0, b > 4 ? logE : 0);
+            P->g2 = launch_shape(P->row_lt, b, a, cols, a == 0, logE);
         }
     }
     // K3: forward step 2 for all cosets (identity when N1 = 1)

@@ -144,8 +144,9 @@ struct Step3Args {
 struct LdeArgs {
     u64* out;
     u32 logN, a, E, logE;
-    // cosets: one after the other (lde_cosets_body), in runs of 2^log_c outputs
-    u32 cosets, log_c;
+    // cosets: one after the other (lde_cosets_body), in runs of 2^log_c outputs;
+    // products: of a wave, for columns of at most 16 elements (lde_short_body), else 0
+    u32 cosets, log_c, products;
     u64 cols, M;
     const u64* src;    // rows of step 2: src[c*src_col_stride + k1*src_row_stride + n2]
     u64 src_col_stride, src_row_stride;
@@ -205,10 +206,11 @@ int lde_release_consts();
 // Phases of the multi-table LDE, in launch order.
 enum LdePhase {
     LDE_PHASE_STEP1 = 0,   // k_step1_multi<true>
-    LDE_PHASE_ROWS = 1,    // k_lde_rows_multi with tiles of 2^12, then 2^13 and 2^14
-    LDE_PHASE_STEP3 = 4,   // k_lde_step3_multi
-    LDE_PHASES = 5
+    LDE_PHASE_ROWS = 1,    // k_lde_rows_multi with tiles of 2^12, 2^13 and 2^14, k_lde_short_multi
+    LDE_PHASE_STEP3 = 5,   // k_lde_step3_multi
+    LDE_PHASES = 6
 };
+constexpr u32 kBatchShort = 15;  // the row tile that stands for k_lde_short_multi
 constexpr u32 kBatchColLt = 13;  // column-kernel tile of multi-table launches
 int launch_lde_multi(int phase, const void* d_args, const u32* d_start, u32 nseg, u32 blocks,
                      size_t lds, hipStream_t st);

@@ -116,3 +116,10 @@ def test_cosets_are_not_in_turn(T, log_n, E, E_few):
         return min(t)
 
     assert best(E) < 4 * best(E_few)
+
+
+@pytest.mark.parametrize("log_n,E,cols,k", [(5, 2, 3, 32), (7, 1, 1, 98), (7, 4, 33, 98), (8, 8, 3, 200)])
+def test_randomizers_of_a_part_filled_tile(T, oracle, log_n, E, cols, k):
+    """The randomizer terms are spread over the rows that the tile holds, not over
+    those it could hold (one column of 2^7 rows: 47 us, 14 with its terms alone)."""
+    test_lde_short_columns(T, oracle, log_n, E, cols, k)

@@ -666,26 +666,26 @@ struct Rows {
     // coefficient k1 + k2 * N1, which carries one when below rand_len
     __device__ __forceinline__ u64 rand_term(u32 t, u32 sl, u32 k2) const {
         const u64 r = k1(t) + ((u64)k2 << A.a);
-        if (r >= A.rs.k || t >= B.valid) return 0;
+        if (r >= A.rs.k) return 0;
         const u64* p = rand_at(A.rs, A.a ? B.c : B.c + t, r);
         return p ? gl::mul(*p, rand_factor(A, sl, r)) : 0;
     }
-    // The randomizer terms of the scaled coefficients of 2^log_rows rows in cosets
+    // The randomizer terms of the scaled coefficients of the block's rows in cosets
     // s0 .. s0 + 2^log_s - 1 in LDS (transform t * 2^log_s + s): the few elements
     // that carry one, spread over the block (a term is ~20 dependent products, which
     // would hold up the block in the one wave that has them: 2^16 x 156 with 98
-    // randomizers, 0.57 against 0.43 ms).
+    // randomizers, 0.57 against 0.43 ms), and over the rows that exist (2^7 x 1 with
+    // 98, a tile of 32 rows: 47 us with all of them, 15 with one).
     template <class Z>
-    __device__ __forceinline__ void add_randomizers(u64* lds, u32 logL, u32 log_rows, u32 s0, u32 log_s) const {
+    __device__ __forceinline__ void add_randomizers(u64* lds, u32 logL, u32 s0, u32 log_s) const {
         const u64 first = A.a ? B.t0 : 0;  // the smallest coefficient index
         if (first >= A.rs.k) return;
         lds_barrier();
         const u64 per = ((A.rs.k - 1 - first) >> A.a) + 1;
-        const u32 n = per < Z::L ? (u32)per : Z::L;
+        const u32 n = per < Z::L ? (u32)per : Z::L, rows = B.valid;
 #pragma unroll 1
-        for (u32 e = threadIdx.x; e < n << (log_rows + log_s); e += Z::kThreads) {
-            const u32 s = e & ((1u << log_s) - 1), t = (e >> log_s) & ((1u << log_rows) - 1);
-            const u32 k2 = e >> (log_s + log_rows);
+        for (u32 e = threadIdx.x; e < (n * rows) << log_s; e += Z::kThreads) {
+            const u32 s = e & ((1u << log_s) - 1), k2 = (e >> log_s) / rows, t = (e >> log_s) - k2 * rows;
             u64* const p = lds + ((t << log_s) + s) * Z::pitch + lds_index(k2);
             *p = gl::add(gl::canon(*p),
                          gl::mul(rand_term(t, s0 + s, k2), A.pb[((s0 + s) << logL) + k2]));
@@ -746,7 +746,7 @@ __device__ __forceinline__ void lde_rows_body(const LdeArgs& A, u64 blk, const R
             }
         }
     }
-    P.template add_randomizers<Z>(lds, LOGL, Z::logNT - A.logE, 0, A.logE);
+    P.template add_randomizers<Z>(lds, LOGL, 0, A.logE);
     dft_block<Z>(lds, Z::logNT, rt.dft[0], rt.r4096[0]);
     // the thread's results are u1 = u0 + q * N2/16 of transform T: the factor
     // advances by w_N^(k1 * N2/16)
@@ -820,7 +820,7 @@ __device__ __forceinline__ void lde_cosets_body(const LdeArgs& A, u64 blk, const
 #pragma unroll
             for (u32 v = 0; v < 4; v++) to[Ti::tq(q + v) * Z::pitch + lds_index(Ti::iq(q + v))] = y[v];
         }
-        P.template add_randomizers<Z>(lds, kCosetsLt, Z::logNT, s, 0);
+        P.template add_randomizers<Z>(lds, kCosetsLt, s, 0);
         // (opaque: no twiddle is kept in registers from one coset to the next)
         const u64* r4096 = rt.r4096[0];
         asm("" : "+s"(r4096) : "s"(s));

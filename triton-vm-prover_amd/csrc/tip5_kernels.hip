@@ -138,8 +138,7 @@ __global__ void __launch_bounds__(kHashThreads, 4) k_hash_rows_multi(
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    const u32 blk = (u32)grid_block();
-    if (blk >= start[nseg]) return;
+    const u32 blk = (u32)grid_block();  // (surplus: the last table's, past its rows)
     u32 seg = find_seg(start, nseg, blk);
     HashArgs A = args[seg];
     hash_rows_body(A, blk - start[seg], W);

@@ -44,8 +44,14 @@ __device__ __forceinline__ u32 find_seg(const u32* __restrict__ start, u32 nseg,
     return lo;
 }
 
-// Block index of a hash_grid launch.
-__device__ __forceinline__ u64 grid_block() { return (u64)blockIdx.y * gridDim.x + blockIdx.x; }
+// Blocks of `threads` threads along the first axis of a hash_grid launch that has a
+// second one, and the block's index (launches of the four-sponge form are short).
+__host__ __device__ constexpr u64 grid_row(u32 threads) { return (1ull << 31) / threads; }
+template <class Wv, u32 THREADS = kHashThreads>
+__device__ __forceinline__ u64 grid_block() {
+    if constexpr (Wv::kSponges == (u32)tip5::QUAD) return blockIdx.x;
+    return blockIdx.y * grid_row(THREADS) + blockIdx.x;
+}
 
 // First sponge of the wave in block blk.
 template <class Wv>
@@ -129,7 +135,7 @@ __global__ void __launch_bounds__(kHashThreads, 4) k_hash_rows(HashArgs A) {
     tip5::load_tables(T);
     const Wv W = tip5::make_wave(T);
     __syncthreads();
-    hash_rows_body(A, grid_block(), W);
+    hash_rows_body(A, grid_block<Wv>(), W);
 }
 
 __global__ void __launch_bounds__(kHashThreads, 4) k_hash_rows_multi(
@@ -138,7 +144,7 @@ __global__ void __launch_bounds__(kHashThreads, 4) k_hash_rows_multi(
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    const u32 blk = (u32)grid_block();  // (surplus: the last table's, past its rows)
+    const u32 blk = (u32)grid_block<tip5::Wave>();  // (surplus: the last table's, past its rows)
     u32 seg = find_seg(start, nseg, blk);
     HashArgs A = args[seg];
     hash_rows_body(A, blk - start[seg], W);
@@ -161,7 +167,7 @@ __global__ void __launch_bounds__(kHashThreads, 4)
     tip5::load_tables(T);
     const Wv W = tip5::make_wave(T);
     __syncthreads();
-    const u64 row = wave_first<Wv>(grid_block()) + W.n;
+    const u64 row = wave_first<Wv>(grid_block<Wv>()) + W.n;
     const u64 r = row < rows ? row : rows - 1;  // lanes past the end repeat the last row
     u64 s[Wv::kWords];
 #pragma unroll
@@ -194,7 +200,7 @@ __global__ void __launch_bounds__(kHashThreads, 4) k_permutation(u64* __restrict
     tip5::load_tables(T);
     const Wv W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first<Wv>(grid_block()) + W.n;
+    const u64 i = wave_first<Wv>(grid_block<Wv>()) + W.n;
     const u64* in = st + (i < num ? i : num - 1) * tip5::STATE;
     u64 s[Wv::kWords];
 #pragma unroll
@@ -215,7 +221,7 @@ __global__ void __launch_bounds__(kHashThreads) k_permutation_rounds(u64* __rest
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first<tip5::Wave>(grid_block()) + W.n;
+    const u64 i = wave_first<tip5::Wave>(grid_block<tip5::Wave>()) + W.n;
     const bool live = i < num;
     const u64* in = st + (live ? i : num - 1) * tip5::STATE + W.g;
     u64* tr = trace && live ? trace + i * (count + 1) * tip5::STATE + W.g : nullptr;
@@ -257,7 +263,7 @@ __global__ void __launch_bounds__(kHashThreads, 4) k_hash_pairs(const u64* __res
     tip5::load_tables(T);
     const Wv W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first<Wv>(grid_block()) + W.n;
+    const u64 i = wave_first<Wv>(grid_block<Wv>()) + W.n;
     const u64 r = i < count ? i : count - 1;
     u64 s[Wv::kWords], x[kRateWords<Wv>];
     rate_elements(x, W, [&](u32 k) { return k < 5 ? left[5 * r + k] : right[5 * r + k - 5]; });
@@ -307,7 +313,7 @@ __global__ void __launch_bounds__(kHashThreads) k_merkle_level(MerkleArgs A) {
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first<tip5::Wave>(grid_block()) + W.n;
+    const u64 i = wave_first<tip5::Wave>(grid_block<tip5::Wave>()) + W.n;
     const u64* c = A.src + 10 * i;
     u64 s[tip5::WORDS], x[3];
     rate_elements(x, W, [&](u32 k) { return c[k]; });
@@ -332,8 +338,8 @@ __global__ void __launch_bounds__(kMerkleThreads) k_merkle_subtrees_multi(
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    const u32 blk = (u32)grid_block();
-    if (blk >= start[nseg]) return;
+    const u32 blk = (u32)grid_block<tip5::Wave, kMerkleThreads>();
+    if (blockIdx.y && blk >= start[nseg]) return;  // surplus
     u32 seg = find_seg(start, nseg, blk);
     const MerkleArgs& A = args[seg];  // read in place: a private copy would spill dst[]
     merkle_body(A, blk - start[seg], W, buf);
@@ -366,7 +372,7 @@ __global__ void k_gather_heap(const u64* __restrict__ tree, u64 n, u32 logn, int
 // axis (more are cut off without an error): past 2^31 the blocks go on along the
 // second one.  Kernels take grid_block() and leave out the last row's surplus.
 static dim3 hash_grid(u64 blocks, u32 threads) {
-    const u64 row = (1ull << 31) / threads;
+    const u64 row = grid_row(threads);
     return blocks <= row ? dim3((u32)blocks) : dim3((u32)row, (u32)((blocks + row - 1) / row));
 }
 

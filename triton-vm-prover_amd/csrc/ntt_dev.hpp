@@ -206,6 +206,9 @@ __device__ __forceinline__ void lds_barrier() {
 // so only the compiler has to keep theirs.
 __device__ __forceinline__ void wave_handoff() { asm volatile("" ::: "memory"); }
 
+// The least l with n <= 2^l (n > 0).
+__device__ __forceinline__ u32 log_ceil(u32 n) { return n > 1 ? 32 - __builtin_clz(n - 1) : 0; }
+
 __device__ __forceinline__ u32 wave_index() {
     return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }
@@ -371,6 +374,13 @@ __device__ __forceinline__ void dft_block(u64* buf, u32 log_t, const u32* mats,
     dft_passes<Z>(buf, log_t, M, mats, r4096);
 }
 
+// Whether a tile of whole columns that is not full (few columns) takes its passes over
+// those that exist: up to 2^8 elements (2^5 x 1, one coset: 9.6 us, 13.5 with passes over
+// all 128).  Longer ones are few to a tile, and a fixed count serves them better (2^10
+// x 379, four cosets: the commit 137 us, 138.5 with a count at run time).
+template <class Z>
+constexpr bool part_tile() { return Z::rA == 0; }
+
 // Elements tid + q * kThreads of the tile (q < 16): transform and index, the
 // thread's part (t, i) and the part of q (tq, iq), which share no bit.  TF
 // (transform-fastest): adjacent threads take adjacent transforms.
@@ -530,25 +540,22 @@ __device__ __forceinline__ BlockPlace block_place(u64 blk, u32 log_nt, u32 log_p
 }
 
 // Transforms of length 2^logL <= 16: one product, no LDS; 16 / L transforms make a
-// group of the matrix product (lanes past the end: the last group again).
-// body(t, i) handles elements (t[v], i[v]), v < 4, of the lane; results have the
-// same indices.  A block takes 2^kSmallLogNT transforms.
-constexpr u32 kSmallLogNT = 8, kSmallThreads = 256;
+// group of the matrix product.  A block takes 2^(10 - logL) transforms, a product to
+// a wave, `valid` of which exist.  body(t, i) handles elements (t[v], i[v]), v < 4, of
+// the lane; results have the same indices.
+constexpr u32 kSmallTile = 10, kSmallThreads = 256;
 template <class Body>
-__device__ __forceinline__ void small_groups(u32 logL, const Body& body) {
+__device__ __forceinline__ void small_groups(u32 logL, u32 valid, const Body& body) {
     const u32 g = (threadIdx.x & 63) >> 4, n = threadIdx.x & 15, sub = 4 - logL;
-    const u32 total = (1u << kSmallLogNT) >> sub;  // (at least 16)
-#pragma unroll 1
-    for (u32 w0 = wave_index() * 16; w0 < total; w0 += blockDim.x / 4) {
-        u32 t[4], i[4];
+    if ((wave_index() * 16) << sub >= valid) return;
+    u32 t[4], i[4];
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const u32 e = 4 * v + g;
-            t[v] = ((w0 + n) << sub) + (e & ((1u << sub) - 1));
-            i[v] = e >> sub;
-        }
-        body(t, i);
+    for (int v = 0; v < 4; v++) {
+        const u32 e = 4 * v + g;
+        t[v] = ((wave_index() * 16 + n) << sub) + (e & ((1u << sub) - 1));
+        i[v] = e >> sub;
     }
+    body(t, i);
 }
 // The small DFT of 2^logL points (none for one point).
 __device__ __forceinline__ void small_dft(u32 logL, const u32* mats, const gl::JoinConsts& J, u64 (&x)[4]) {
@@ -682,10 +689,12 @@ struct Rows {
         if (first >= A.rs.k) return;
         lds_barrier();
         const u64 per = ((A.rs.k - 1 - first) >> A.a) + 1;
-        const u32 n = per < Z::L ? (u32)per : Z::L, rows = B.valid;
+        const u32 n = per < Z::L ? (u32)per : Z::L, log_rows = log_ceil(B.valid);
 #pragma unroll 1
-        for (u32 e = threadIdx.x; e < (n * rows) << log_s; e += Z::kThreads) {
-            const u32 s = e & ((1u << log_s) - 1), k2 = (e >> log_s) / rows, t = (e >> log_s) - k2 * rows;
+        for (u32 e = threadIdx.x; e < n << (log_rows + log_s); e += Z::kThreads) {
+            const u32 s = e & ((1u << log_s) - 1), t = (e >> log_s) & ((1u << log_rows) - 1);
+            const u32 k2 = e >> (log_s + log_rows);
+            if (t >= B.valid) continue;
             u64* const p = lds + ((t << log_s) + s) * Z::pitch + lds_index(k2);
             *p = gl::add(gl::canon(*p),
                          gl::mul(rand_term(t, s0 + s, k2), A.pb[((s0 + s) << logL) + k2]));
@@ -715,7 +724,8 @@ __device__ __forceinline__ void lde_rows_body(const LdeArgs& A, u64 blk, const R
             if ((q << A.logE) < 16 && T.t + Ti::tq(q) < Z::NT >> A.logE)
                 lane_p[Ti::tq(q) * Z::pitch + lds_index(Ti::iq(q))] = x[q];
     }
-    dft_block<Z>(lds, Z::logNT - A.logE, rt.dft[1], rt.r4096[1]);
+    const u32 log_rows = part_tile<Z>() ? log_ceil(P.B.valid) : Z::logNT - A.logE;
+    dft_block<Z>(lds, log_rows, rt.dft[1], rt.r4096[1]);
     // coefficients to registers, then to every coset's transform: product j of
     // the thread is element q = j / E in coset j mod E
     {
@@ -747,7 +757,7 @@ __device__ __forceinline__ void lde_rows_body(const LdeArgs& A, u64 blk, const R
         }
     }
     P.template add_randomizers<Z>(lds, LOGL, 0, A.logE);
-    dft_block<Z>(lds, Z::logNT, rt.dft[0], rt.r4096[0]);
+    dft_block<Z>(lds, part_tile<Z>() ? log_rows + A.logE : Z::logNT, rt.dft[0], rt.r4096[0]);
     // the thread's results are u1 = u0 + q * N2/16 of transform T: the factor
     // advances by w_N^(k1 * N2/16)
     const Tile<Z, true> U;

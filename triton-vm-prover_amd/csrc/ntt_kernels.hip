@@ -126,9 +126,11 @@ static u32 choose_split(u32 logN, u32 E, u32 row_lt) {
 
 LaunchShape launch_shape(u32 lt, u32 logL, u32 log_per, u64 cols, bool flat, u32 log_e) {
     LaunchShape g;
-    u32 log_nt = kSmallLogNT;
-    g.threads = kSmallThreads;
-    if (logL > 4) {
+    u32 log_nt;
+    if (logL <= 4) {
+        log_nt = kSmallTile - logL;
+        g.threads = kSmallThreads;
+    } else {
         log_nt = lt - logL - log_e;
         g.threads = 1u << (lt - 4);
         // (the pitch of Shape<LT, LOGL>, then two sets of accumulator starts)

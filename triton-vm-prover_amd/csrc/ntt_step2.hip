@@ -39,16 +39,16 @@ __global__ void __launch_bounds__(1 << (LT - 4), 4) k_ntt_step2(const u64* src, 
     typedef Shape<LT, LOGL> Z;
     const RowStep<INV, COLS> P(src, dst, logN, a, cols, ninv, blockIdx.x, Z::logNT, gridDim.x);
     load_tile<Z, false>(lds, P.in, P.B.valid, Unscaled{});
-    dft_block<Z>(lds, Z::logNT, rt.dft[INV], rt.r4096[INV]);
+    dft_block<Z>(lds, COLS && part_tile<Z>() ? log_ceil(P.B.valid) : Z::logNT, rt.dft[INV], rt.r4096[INV]);
     store_tile<Z, !COLS>(lds, P.out, P.B.valid, [&](u64 (&x)[4]) { P.finish(x); });
 }
 // rows of at most 16 elements
 template <bool INV, bool COLS>
 __global__ void __launch_bounds__(kSmallThreads) k_ntt_step2_small(const u64* src, u64* dst, u32 logN,
                                                                    u32 a, u64 cols, u64 ninv, Roots rt) {
-    const RowStep<INV, COLS> P(src, dst, logN, a, cols, ninv, blockIdx.x, kSmallLogNT);
+    const RowStep<INV, COLS> P(src, dst, logN, a, cols, ninv, blockIdx.x, kSmallTile - (logN - a));
     const gl::JoinConsts J = gl::join_consts();
-    small_groups(logN - a, [&](const u32 (&t)[4], const u32 (&i)[4]) {
+    small_groups(logN - a, P.B.valid, [&](const u32 (&t)[4], const u32 (&i)[4]) {
         u64 x[4];
 #pragma unroll
         for (int v = 0; v < 4; v++) x[v] = t[v] < P.B.valid ? P.in.base[P.in.off(t[v], i[v])] : 0;
@@ -95,15 +95,15 @@ __global__ void __launch_bounds__(1 << 8, 4) k_ntt_cols_scaled(const u64* src, u
                         [&](u32 t, const u32 (&tq)[4], u32 i, const u32 (&iq)[4], u64 (&x)[4]) {
                             C.scale(t, tq, i, iq, x);
                         });
-    dft_block<Z>(lds, Z::logNT, rt.dft[0], rt.r4096[0]);
+    dft_block<Z>(lds, part_tile<Z>() ? log_ceil(C.P.B.valid) : Z::logNT, rt.dft[0], rt.r4096[0]);
     store_tile<Z, false>(lds, C.P.out, C.P.B.valid, [&](u64 (&x)[4]) { C.P.finish(x); });
 }
 // columns of at most 16 elements
 __global__ void __launch_bounds__(kSmallThreads) k_ntt_cols_scaled_small(const u64* src, u64* dst, u32 logN,
                                                                          u64 cols, NttScaleDev S, Roots rt) {
-    const ScaledCols C(src, dst, logN, cols, S, blockIdx.x, kSmallLogNT);
+    const ScaledCols C(src, dst, logN, cols, S, blockIdx.x, kSmallTile - logN);
     const gl::JoinConsts J = gl::join_consts();
-    small_groups(logN, [&](const u32 (&t)[4], const u32 (&i)[4]) {
+    small_groups(logN, C.P.B.valid, [&](const u32 (&t)[4], const u32 (&i)[4]) {
         u64 x[4];
 #pragma unroll
         for (int v = 0; v < 4; v++) x[v] = t[v] < C.P.B.valid ? C.P.in.base[C.P.in.off(t[v], i[v])] : 0;

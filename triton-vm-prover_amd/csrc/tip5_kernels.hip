@@ -214,6 +214,9 @@ __global__ void __launch_bounds__(kHashThreads, 4) k_permutation(u64* __restrict
 // Rounds [first, first + count) of the permutation on num states (in place).
 // trace (may be null) receives, per state, the input and the state after each
 // of those rounds: trace[(i * (count + 1) + j) * 16 + k].  Outputs canonical.
+// Without a trace (TRACED) a block takes its sets of 64 states in turn: its tables and
+// operands (12 KB a wave) outweigh the states (2 KB) where there are few rounds.
+template <bool TRACED>
 __global__ void __launch_bounds__(kHashThreads) k_permutation_rounds(u64* __restrict__ st, u64 num,
                                                                      u32 first, u32 count,
                                                                      u64* __restrict__ trace) {
@@ -221,28 +224,33 @@ __global__ void __launch_bounds__(kHashThreads) k_permutation_rounds(u64* __rest
     tip5::load_tables(T);
     const tip5::Wave W = tip5::make_wave(T);
     __syncthreads();
-    const u64 i = wave_first<tip5::Wave>(grid_block<tip5::Wave>()) + W.n;
-    const bool live = i < num;
-    const u64* in = st + (live ? i : num - 1) * tip5::STATE + W.g;
-    u64* tr = trace && live ? trace + i * (count + 1) * tip5::STATE + W.g : nullptr;
-    u64 s[tip5::WORDS];
+    u64 blk = blockIdx.x;
+    do {
+        const u64 i = wave_first<tip5::Wave>(blk) + W.n;
+        const bool live = i < num;
+        const u64* in = st + (live ? i : num - 1) * tip5::STATE + W.g;
+        u64* tr = TRACED && live ? trace + i * (count + 1) * tip5::STATE + W.g : nullptr;
+        u64 s[tip5::WORDS];
 #pragma unroll
-    for (int v = 0; v < tip5::WORDS; v++) {
-        const u64 x = in[4 * v];
-        if (tr) tr[4 * v] = x;
-        s[v] = tip5::to_m(x);
-    }
-    for (u32 r = 0; r < count; r++) {
-        tip5::round_m(s, (int)(first + r), W);
-        if (tr) {
-#pragma unroll
-            for (int v = 0; v < tip5::WORDS; v++)
-                tr[(r + 1) * tip5::STATE + 4 * v] = tip5::from_m(s[v]);
+        for (int v = 0; v < tip5::WORDS; v++) {
+            const u64 x = in[4 * v];
+            if (tr) tr[4 * v] = x;
+            s[v] = tip5::to_m(x);
         }
-    }
-    if (!live) return;
+        for (u32 r = 0; r < count; r++) {
+            tip5::round_m(s, (int)(first + r), W);
+            if (tr) {
 #pragma unroll
-    for (int v = 0; v < tip5::WORDS; v++) st[i * tip5::STATE + W.g + 4 * v] = tip5::from_m(s[v]);
+                for (int v = 0; v < tip5::WORDS; v++)
+                    tr[(r + 1) * tip5::STATE + 4 * v] = tip5::from_m(s[v]);
+            }
+        }
+        if (live) {
+#pragma unroll
+            for (int v = 0; v < tip5::WORDS; v++) st[i * tip5::STATE + W.g + 4 * v] = tip5::from_m(s[v]);
+        }
+        blk += gridDim.x;
+    } while (!TRACED && blk * kSpongesPerBlock < num);
 }
 
 // hash_pair: the two digests are words 0..9 (x: the lane's), the capacity is ones.
@@ -479,8 +487,17 @@ int launch_permutation(u64* states, u64 num, hipStream_t st) {
 int launch_permutation_rounds(u64* states, u64 num, u32 first, u32 count, u64* trace,
                               hipStream_t st) {
     if (num == 0) return TVH_OK;
-    hipLaunchKernelGGL(k_permutation_rounds, hash_grid(sponge_blocks(num), kHashThreads),
-                       dim3(kHashThreads), 0, st, states, num, first, count, trace);
+    const u64 sets = (num + kSpongesPerBlock - 1) / kSpongesPerBlock;
+    const dim3 tpb(kHashThreads);
+    if (trace) {
+        hipLaunchKernelGGL(k_permutation_rounds<true>, dim3((u32)sets), tpb, 0, st, states, num, first, count,
+                           trace);
+    } else {
+        // eight blocks to a CU (one round of 2^20 states: 59 us, 86 with a block to every
+        // 64; a trace's stores want those: 346 us for five rounds of 2^20, else 433)
+        hipLaunchKernelGGL(k_permutation_rounds<false>, dim3((u32)(sets < 2048 ? sets : 2048)), tpb, 0, st,
+                           states, num, first, count, trace);
+    }
     return check_launch();
 }
 

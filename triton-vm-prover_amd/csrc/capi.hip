@@ -721,9 +721,8 @@ struct HostCall {
 };
 
 static int check_canonical(const u64* p, size_t n) {
-    for (size_t i = 0; i < n; i++)
-        if (p[i] >= TVH_P) return set_error(TVH_ERR_NOT_CANONICAL, "element %zu >= p", i);
-    return TVH_OK;
+    const size_t i = first_at_least(p, n, TVH_P);
+    return i < n ? set_error(TVH_ERR_NOT_CANONICAL, "element %zu >= p", i) : TVH_OK;
 }
 
 static int ntt_host(uint64_t* data, size_t n, bool inv) {
@@ -885,27 +884,32 @@ int tvh_commit_host(const uint64_t* trace, size_t cols, size_t n, const uint64_t
                     uint64_t* root_out) {
     if (!trace || !root_out || (k && !rand)) return set_error(TVH_ERR_INVALID_ARG, "null buffer");
     if (!is_pow2(m)) return set_error(TVH_ERR_NOT_POW2, "target_len");
-    // The inputs are checked while the GPU works on them (it takes any u64), and before
-    // anything is written to the caller; the check's status comes before any other
-    // (2^12 x 379: 1.23 -> 0.94 ms a call).
+    // A refusal comes before any other status, and before the commit is queued: for the
+    // first elements before anything is done, for tables of up to 32 MB (a staging slot;
+    // queued at once) after the copy to the device, beside which the check then runs
+    // (2^12 x 379: 0.88 ms a call, 0.98 with the check first), for larger ones first.
+    const size_t len = cols * n, rand_len = cols * k;
+    const bool beside = len + rand_len <= (4u << 20);
+    int rc = check_canonical(trace, beside && len > 8192 ? 8192 : len);
+    if (!rc && !beside && k) rc = check_canonical(rand, rand_len);
+    if (rc) return rc;
     auto checked = [&](int status) {
-        const int bad = check_canonical(trace, cols * n);
-        if (bad || !k) return bad ? bad : status;
-        const int bad_rand = check_canonical(rand, cols * k);
-        return bad_rand ? bad_rand : status;
+        int bad = beside ? check_canonical(trace, len) : TVH_OK;
+        if (!bad && beside && k) bad = check_canonical(rand, rand_len);
+        return bad ? bad : status;
     };
-    int rc;
     HostCall hc;
     if (hc.rc) return checked(hc.rc);
-    u64* dt = hc.alloc(cols * n);
-    u64* dr = hc.alloc(cols * k);
+    u64* dt = hc.alloc(len);
+    u64* dr = hc.alloc(rand_len);
     u64* dcw = hc.alloc(cols * m);
     u64* dtree = hc.alloc((2 * m - 1) * 5);
     if (hc.rc) return checked(hc.rc);
-    if ((rc = hc.up(dt, trace, cols * n)) || (rc = hc.up(dr, rand, cols * k))) return checked(rc);
-    rc = checked(tvh_commit_dev(dt, cols, n, k ? dr : nullptr, k, toff, goff, m, dcw, dtree,
-                                TVH_TREE_LEVEL_ORDER, hc.st));
-    if (rc) return rc;
+    if ((rc = hc.up(dt, trace, len)) || (rc = hc.up(dr, rand, rand_len))) return checked(rc);
+    if ((rc = checked(TVH_OK))) return rc;
+    if ((rc = tvh_commit_dev(dt, cols, n, k ? dr : nullptr, k, toff, goff, m, dcw, dtree,
+                             TVH_TREE_LEVEL_ORDER, hc.st)))
+        return rc;
     if (cw_out && (rc = hc.down(cw_out, dcw, cols * m))) return rc;
     if (dg_out && (rc = hc.down(dg_out, dtree, m * 5))) return rc;
     if ((rc = hc.down(root_out, dtree + 5 * (2 * m - 2), 5))) return rc;

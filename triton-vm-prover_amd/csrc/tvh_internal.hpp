@@ -55,6 +55,8 @@ DeviceState* initialized_device();
 // the device's page-locked staging ring (stager.hip); returns once every piece
 // is queued (the source may then be reused).  Calls on one device take turns.
 int staged_h2d(void* dst, const void* src, size_t bytes, hipStream_t st);
+// Index of the first of n host elements that is at least `limit`, or n.
+size_t first_at_least(const u64* p, size_t n, u64 limit);
 
 // State of the current device, initialised on first use (thread-safe).
 // Returns nullptr and sets the error on failure.

@@ -8,8 +8,11 @@
 //
 // The 64x64 product is built from four 32x32->64 multiply-adds
 // (v_mad_u64_u32); the 128-bit result is folded with 2^64 = 2^32 - 1 and
-// 2^96 = -1 (mod p).  Multiplication by 2^k (the radix-64 twiddles: the
-// reference's w_64 = 7^((p-1)/64) equals 2^39) is a shift plus the same fold.
+// 2^96 = -1 (mod p).  The kernels take their products and folds from the forms
+// that set a rare borrow aside (mul_rare, mul_n, ...) and the exact ones where
+// that case is redone, in set-up and on the host.  add_lazy, sqr_wide, mont_sqr,
+// mont_mul, lin52 and the shift multiplies (mul_pow2...) have only the native
+// checks as callers now.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -81,7 +84,7 @@ __host__ __device__ __forceinline__ u64 sub(u64 a, u64 b) {
     return b1 ? mk64(e0, e1) : mk64(d0, d1);
 }
 
-// a any u64, b canonical -> lazy (any u64).  Used to add round constants.
+// a any u64, b canonical -> lazy (any u64).
 __host__ __device__ __forceinline__ u64 add_lazy(u64 a, u64 b) {
     u32 c0, c1, c2, c3;
     u32 s0 = __builtin_addc((u32)a, (u32)b, 0u, &c0);
@@ -181,7 +184,7 @@ __host__ __device__ __forceinline__ u64 montyred(u64 lo, u64 hi) {
     return mk64(r0, r1);
 }
 
-// L + H * 2^32 mod p for L, H < 2^52 (the MDS recombination) -> < 2^64, in
+// L + H * 2^32 mod p for L, H < 2^52 -> < 2^64, in
 // 32-bit words: with 2^64 = 2^32 - 1 mod p the value is (L0 - H1) +
 // (L1 + H0 + H1) * 2^32; a carry out of the high word is folded back as 2^32 - 1.
 __host__ __device__ __forceinline__ u64 lin52(u64 L, u64 H) {
@@ -259,11 +262,7 @@ __device__ __forceinline__ void carry_wait() {
 
 __device__ __forceinline__ bool in_mask(mask m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
-// r = a + b, a + b + k, a - b - k, ... and the carry (borrow) out
-#define GL_ADD_CO(r, k, a, b) \
-    asm volatile("v_add_co_u32 %0, %1, %2, %3" : "=v"(r), "=s"(k) : "v"(a), "v"(b))
-#define GL_ADDC_CO(r, ko, a, b, k) \
-    asm volatile("v_addc_co_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(ko) : "v"(a), "v"(b), "s"(k))
+// r = a + k, a - b, a - b - k, a - k and the carry (borrow) out
 #define GL_ADDC_0(r, ko, a, k) \
     asm volatile("v_addc_co_u32 %0, %1, %2, 0, %3" : "=v"(r), "=s"(ko) : "v"(a), "s"(k))
 #define GL_SUB_CO(r, k, a, b) \
@@ -439,12 +438,6 @@ __host__ __device__ __forceinline__ u64 mul_pow2_small(u64 x) {
     return mk64(r0, r1);
 }
 
-// x any u64 -> lazy x * 2^32
-__host__ __device__ __forceinline__ u64 mul_2_32(u64 x) {
-    // x = x1*2^32 + x0 ; x*2^32 = x0*2^32 + x1*2^64 = x0*2^32 + x1*(2^32-1)
-    return fold128(x << 32, x >> 32);
-}
-
 // x * 2^E mod p for a compile-time 0 <= E < 96 and any u64 x -> canonical,
 // without a general product.  p divides 2^96 + 1, so with x << E split into
 // 32-bit words w0..w4 (E = 32q + r), the 96 low bits count positively and the
@@ -496,23 +489,6 @@ __host__ __device__ __forceinline__ u64 mul_pow2(u64 x) {
     (void)c3;
     (void)g1;
     return d1 ? mk64(s0, s1) : (k1 ? mk64(a0, a1) : mk64(u0, u1));
-}
-
-// x canonical, k runtime in [0, 192) -> canonical x * 2^k (host and tables)
-__host__ __device__ __forceinline__ u64 mul_pow2_rt(u64 x, u32 k) {
-    bool negate = k >= 96;
-    if (negate) k -= 96;
-    u64 r;
-    if (k == 0) {
-        r = x;
-    } else if (k < 64) {
-        r = canon(fold128(x << k, x >> (64 - k)));
-    } else {
-        u32 s = k - 64;
-        u64 y = s ? canon(fold128(x << s, x >> (64 - s))) : x;
-        r = sub(canon(mul_2_32(y)), y);
-    }
-    return negate ? neg(r) : r;
 }
 
 __host__ __device__ inline u64 pow(u64 b, u64 e) {

@@ -943,6 +943,18 @@ __host__ __device__ __forceinline__ void with_length(u32 logL, const F& f) {
         default: f(std::integral_constant<int, 12>{}); break;
     }
 }
+// Tiles of 2^12..2^14 elements likewise.
+template <class F>
+__host__ void with_tile(u32 lt, const F& f) {
+    if (lt == 12) f(std::integral_constant<int, 12>{});
+    else if (lt == 13) f(std::integral_constant<int, 13>{});
+    else f(std::integral_constant<int, 14>{});
+}
+// Row tile of the NTT: without a column step 2^12, else the shortest that holds 8 rows
+// of 2^logL, 2^12 to 2^14.
+constexpr u32 ntt_row_tile(u32 logL, bool cols) {
+    return cols || logL <= 9 ? 12 : logL == 10 ? 13 : LOG_TILE;
+}
 // A launch of `cols` columns of 2^log_per transforms (flat: one each, as
 // block_place) of length 2^logL in tiles of 2^lt elements; 2^log_e transforms of the
 // tile belong to one of a column's.
@@ -959,8 +971,8 @@ int launch_k_step1_scaled(u32 lt, const LaunchShape& g, hipStream_t st, const St
                           const NttScaleDev& S, const Roots& rt);
 int set_attributes_step1(int lds_bytes);
 // ntt_step2.hip
-int launch_k_ntt_step2(bool inv, u32 lt, const LaunchShape& g, hipStream_t st, const u64* src,
-                       u64* dst, u32 logN, u32 a, u64 cols, u64 ninv, const Roots& rt);
+int launch_k_ntt_step2(bool inv, const LaunchShape& g, hipStream_t st, const u64* src, u64* dst, u32 logN,
+                       u32 a, u64 cols, u64 ninv, const Roots& rt);
 int launch_k_ntt_cols_scaled(const LaunchShape& g, hipStream_t st, const u64* src, u64* dst, u32 logN,
                              u64 cols, const NttScaleDev& S, const Roots& rt);
 int set_attributes_step2(int lds_bytes);

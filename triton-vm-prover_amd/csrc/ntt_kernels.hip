@@ -442,7 +442,7 @@ int launch_ntt_batched(const u64* src, u64* dst, u64 n, u64 cols, bool inverse, 
     const u32 a = logN <= 12 ? 0 : logN <= 14 ? logN / 2 : logN <= 20 ? 8 : logN - 12;
     const u32 b = logN - a;
     const u32 col_lt = logN > 22 ? LOG_TILE : (cols << logN) < (1ull << 23) && a < 10 ? 12 : 13;
-    const u32 row_lt = a == 0 ? 12 : std::min(std::max(b + 3, 12u), (u32)LOG_TILE);
+    const u32 row_lt = ntt_row_tile(b, a == 0);
     NttScaleDev S{};
     if (scale) {  // p1[n1] = base^(N2 n1), p2[n2] = base^n2
         if (!scale->tables) return set_error(TVH_ERR_INVALID_ARG, "no tables for the NTT scaling");
@@ -477,8 +477,7 @@ int launch_ntt_batched(const u64* src, u64* dst, u64 n, u64 cols, bool inverse, 
         }
         const LaunchShape s2 = launch_shape(row_lt, b, a, g, a == 0);
         rc = scale && !a ? launch_k_ntt_cols_scaled(s2, st, sg, d, logN, g, Sg, ds->roots)
-                         : launch_k_ntt_step2(inverse, row_lt, s2, st, a ? scratch : sg, d, logN, a, g, ninv,
-                                              ds->roots);
+                         : launch_k_ntt_step2(inverse, s2, st, a ? scratch : sg, d, logN, a, g, ninv, ds->roots);
         if (rc) return rc;
     }
     return TVH_OK;

@@ -32,27 +32,27 @@ struct RowStep {
     }
 };
 
-template <bool INV, bool COLS, int LT, int LOGL>
-__global__ void __launch_bounds__(1 << (LT - 4), 4) k_ntt_step2(const u64* src, u64* dst, u32 logN,
-                                                                u32 a, u64 cols, u64 ninv, Roots rt) {
+template <bool INV, bool COLS, int LOGL>
+__global__ void __launch_bounds__(1 << (ntt_row_tile(LOGL, COLS) - 4), 4)
+    k_ntt_step2(const u64* src, u64* dst, u32 logN, u32 a, u64 cols, u64 ninv, Roots rt) {
     extern __shared__ u64 lds[];
-    typedef Shape<LT, LOGL> Z;
+    typedef Shape<ntt_row_tile(LOGL, COLS), LOGL> Z;
     const RowStep<INV, COLS> P(src, dst, logN, a, cols, ninv, blockIdx.x, Z::logNT, gridDim.x);
     load_tile<Z, false>(lds, P.in, P.B.valid, Unscaled{});
     dft_block<Z>(lds, COLS && part_tile<Z>() ? log_ceil(P.B.valid) : Z::logNT, rt.dft[INV], rt.r4096[INV]);
     store_tile<Z, !COLS>(lds, P.out, P.B.valid, [&](u64 (&x)[4]) { P.finish(x); });
 }
-// rows of at most 16 elements
-template <bool INV, bool COLS>
+// columns of at most 16 elements
+template <bool INV>
 __global__ void __launch_bounds__(kSmallThreads) k_ntt_step2_small(const u64* src, u64* dst, u32 logN,
-                                                                   u32 a, u64 cols, u64 ninv, Roots rt) {
-    const RowStep<INV, COLS> P(src, dst, logN, a, cols, ninv, blockIdx.x, kSmallTile - (logN - a));
+                                                                   u64 cols, u64 ninv, Roots rt) {
+    const RowStep<INV, true> P(src, dst, logN, 0, cols, ninv, blockIdx.x, kSmallTile - logN);
     const gl::JoinConsts J = gl::join_consts();
-    small_groups(logN - a, P.B.valid, [&](const u32 (&t)[4], const u32 (&i)[4]) {
+    small_groups(logN, P.B.valid, [&](const u32 (&t)[4], const u32 (&i)[4]) {
         u64 x[4];
 #pragma unroll
         for (int v = 0; v < 4; v++) x[v] = t[v] < P.B.valid ? P.in.base[P.in.off(t[v], i[v])] : 0;
-        small_dft(logN - a, rt.dft[INV], J, x);
+        small_dft(logN, rt.dft[INV], J, x);
         P.finish(x);
 #pragma unroll
         for (int v = 0; v < 4; v++)
@@ -129,55 +129,49 @@ int launch_k_ntt_cols_scaled(const LaunchShape& g, hipStream_t st, const u64* sr
     return check_launch();
 }
 
+// Rows after a column step have 2^7 elements and more (launch_ntt_batched).
+template <bool COLS, int LOGL>
+constexpr bool kRowShape = COLS || LOGL >= 7;
+
 template <bool INV, bool COLS>
-static void launch_step2(u32 lt, const LaunchShape& g, hipStream_t st, const u64* src, u64* dst,
-                         u32 logN, u32 a, u64 cols, u64 ninv, const Roots& rt) {
+static int launch_step2(const LaunchShape& g, hipStream_t st, const u64* src, u64* dst, u32 logN, u32 a,
+                        u64 cols, u64 ninv, const Roots& rt) {
     const dim3 blocks(g.blocks), tpb(g.threads);
-    if (logN - a <= 4) {
-        hipLaunchKernelGGL((k_ntt_step2_small<INV, COLS>), blocks, tpb, 0, st, src, dst, logN, a, cols,
-                           ninv, rt);
-        return;
+    bool done = false;
+    if (COLS && logN <= 4) {
+        hipLaunchKernelGGL(k_ntt_step2_small<INV>, blocks, tpb, 0, st, src, dst, logN, cols, ninv, rt);
+        return check_launch();
     }
     with_length(logN - a, [&](auto l) {
         constexpr int L = decltype(l)::value;
-#define TVH_STEP2(T)                                                                                \
-    hipLaunchKernelGGL((k_ntt_step2<INV, COLS, T, L>), blocks, tpb, g.lds, st, src, dst, logN, a, cols, \
-                       ninv, rt)
-        if (lt == 12) TVH_STEP2(12);
-        else if (lt == 13) TVH_STEP2(13);
-        else TVH_STEP2(14);
-#undef TVH_STEP2
+        if constexpr (kRowShape<COLS, L>) {
+            hipLaunchKernelGGL((k_ntt_step2<INV, COLS, L>), blocks, tpb, g.lds, st, src, dst, logN, a, cols,
+                               ninv, rt);
+            done = true;
+        }
     });
+    return done ? check_launch() : set_error(TVH_ERR_UNSUPPORTED, "row step of 2^%u", logN - a);
 }
 
-int launch_k_ntt_step2(bool inv, u32 lt, const LaunchShape& g, hipStream_t st, const u64* src,
-                       u64* dst, u32 logN, u32 a, u64 cols, u64 ninv, const Roots& rt) {
-    if (a == 0) {
-        if (inv) launch_step2<true, true>(lt, g, st, src, dst, logN, a, cols, ninv, rt);
-        else launch_step2<false, true>(lt, g, st, src, dst, logN, a, cols, ninv, rt);
-    } else {
-        if (inv) launch_step2<true, false>(lt, g, st, src, dst, logN, a, cols, ninv, rt);
-        else launch_step2<false, false>(lt, g, st, src, dst, logN, a, cols, ninv, rt);
-    }
-    return check_launch();
+int launch_k_ntt_step2(bool inv, const LaunchShape& g, hipStream_t st, const u64* src, u64* dst, u32 logN,
+                       u32 a, u64 cols, u64 ninv, const Roots& rt) {
+    if (a == 0)
+        return inv ? launch_step2<true, true>(g, st, src, dst, logN, a, cols, ninv, rt)
+                   : launch_step2<false, true>(g, st, src, dst, logN, a, cols, ninv, rt);
+    return inv ? launch_step2<true, false>(g, st, src, dst, logN, a, cols, ninv, rt)
+               : launch_step2<false, false>(g, st, src, dst, logN, a, cols, ninv, rt);
 }
 
-template <bool INV, bool COLS>
-static void step2_kernels(std::vector<const void*>& fns) {
+// (2^12 tiles need no more LDS than every kernel has)
+int set_attributes_step2(int bytes) {
+    std::vector<const void*> fns;
     for (u32 l = 5; l <= 12; l++)
         with_length(l, [&](auto c) {
             constexpr int L = decltype(c)::value;
-            fns.insert(fns.end(), {(const void*)k_ntt_step2<INV, COLS, 12, L>,
-                                   (const void*)k_ntt_step2<INV, COLS, 13, L>,
-                                   (const void*)k_ntt_step2<INV, COLS, 14, L>});
+            if constexpr (ntt_row_tile(L, false) > 12)
+                fns.insert(fns.end(), {(const void*)k_ntt_step2<true, false, L>,
+                                       (const void*)k_ntt_step2<false, false, L>});
         });
-}
-int set_attributes_step2(int bytes) {
-    std::vector<const void*> fns;
-    step2_kernels<true, true>(fns);
-    step2_kernels<true, false>(fns);
-    step2_kernels<false, true>(fns);
-    step2_kernels<false, false>(fns);
     return set_lds_attribute(fns, bytes);
 }
 

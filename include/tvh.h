@@ -196,13 +196,13 @@ int tvh_lde_get_variant(uint32_t log_n, uint32_t log_e, int* variant);
 int tvh_lde_get_variant_for_width(uint32_t log_n, uint32_t log_e, size_t num_cols, int* variant);
 /* Number of variants tvh_lde_autotune times (the length of its ms array). */
 int tvh_lde_variant_count(void);
-/* Times every variant on scratch buffers of this shape (num_cols capped so
- * the codewords stay under 4 GiB), keeps the fastest for the shape and the
- * width band of num_cols, and returns
- * its code in *chosen; ms (may be NULL) receives the average milliseconds per
- * LDE of the variants 1, 2, 5, 6, 9, 10, 18, 22, 26, 34, 38, 42, 66, 70, 74 in
- * that order.  Synchronous; allocates
- * and frees its own buffers; not to be called concurrently with other work. */
+/* Times every variant (codes that give one plan once) on scratch buffers of this
+ * shape (num_cols capped so the codewords stay under 4 GiB), keeps the fastest for
+ * the shape and the width band of num_cols, and returns its code in *chosen; ms
+ * (may be NULL) receives the average milliseconds per LDE of the variants 1, 2, 5,
+ * 6, 9, 10, 18, 22, 26, 34, 38, 42, 66, 70, 74 in that order.  Synchronous;
+ * allocates and frees its own buffers; not to be called concurrently with other
+ * work. */
 int tvh_lde_autotune(size_t num_cols, size_t trace_len, size_t target_len, int* chosen,
                      float* ms);
 

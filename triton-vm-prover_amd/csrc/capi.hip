@@ -304,13 +304,24 @@ int tvh_lde_autotune(size_t cols, size_t n, size_t m, int* chosen, float* ms) {
     int prev = lde_variant(logN, logE, cols);
     if (!rc) rc = lde_prepare_consts(n, m, 1, 7);
     bool any = false;
+    // codes that give one plan are timed once (their form and LDE_INV_HALF change nothing)
+    float times[kNumLdeVariants];
+    auto plan_bits = [](int v) { return v & ~(LDE_WIDE | LDE_SPLIT | LDE_INV_HALF); };
     for (int i = 0; i < kNumLdeVariants && !rc; i++) {
+        int same = 0;
+        while (plan_bits(kLdeVariants[same]) != plan_bits(kLdeVariants[i])) same++;
+        if (same < i) {
+            times[i] = times[same];
+            if (ms) ms[i] = times[i];
+            continue;
+        }
         set_lde_variant(logN, logE, kLdeVariants[i], wc_timed);
         RandSpec none;
         rc = launch_lde(trace, tc, n, none, 1, 7, m, false, out, st);  // warm-up
         if (rc == TVH_ERR_UNSUPPORTED) {  // this variant cannot run the shape: skip it
             rc = TVH_OK;
-            if (ms) ms[i] = -1.0f;
+            times[i] = -1.0f;
+            if (ms) ms[i] = times[i];
             continue;
         }
         if (!rc && hipEventRecord(e0, st) != hipSuccess) rc = set_error(TVH_ERR_DEVICE, "event");
@@ -320,6 +331,7 @@ int tvh_lde_autotune(size_t cols, size_t n, size_t m, int* chosen, float* ms) {
         float t = 0;
         if (!rc && hipEventElapsedTime(&t, e0, e1) != hipSuccess) rc = set_error(TVH_ERR_DEVICE, "elapsed");
         t /= 3;
+        times[i] = t;
         if (ms) ms[i] = t;
         if (!rc && (!any || t < best)) {
             best = t;

@@ -113,7 +113,10 @@ int tvh_ntt_inverse_dev(uint64_t* d_data, size_t n, void* stream);
  *            (x^n - trace_offset^n) * r_c(x), r_c = d_rand[c*rand_len + i]
  *   out_c[j] = poly_c(target_offset * w_m^j), j < target_len
  * trace_len and target_len are powers of two, target_len = E * trace_len
- * with E in {1,2,4,8,16}; rand_len <= trace_len; d_rand may be NULL when
+ * with E in {1,2,4,8,16}; trace_len <= 2^23 and target_len <= 2^25
+ * (TVH_ERR_UNSUPPORTED beyond; 2^26 with a variant of the 2^14 row tile, see
+ * tvh_lde_set_variant, and 2^24 with TVH_LDE_ROW_QUARTER and E > 1);
+ * rand_len <= trace_len; d_rand may be NULL when
  * rand_len == 0.  d_trace is column-major trace_len x num_cols, d_out is
  * column-major target_len x num_cols; they must not overlap.  d_out is the
  * only working memory (no scratch).
@@ -169,7 +172,8 @@ int tvh_lde_release_constants(void);
  * TVH_LDE_WIDE or TVH_LDE_SPLIT, 2^13 with TVH_LDE_SPLIT | TVH_LDE_ROW_HALF,
  * 2^12 with TVH_LDE_SPLIT | TVH_LDE_ROW_QUARTER; TVH_LDE_INV_HALF (with
  * TVH_LDE_SPLIT only, alone) is accepted and changes nothing.  Within that the
- * library takes the shortest tile that holds the rows it chose.  Tile 0/1/2
+ * library takes the shortest tile that holds the rows it chose (columns of up to 16
+ * rows need none, and 2^9 rows in 16 cosets take 2^13 under every bound).  Tile 0/1/2
  * gives the column steps LDS tiles of 2^14/2^13/2^12 elements (1024/512/256
  * threads).  The variant is chosen per (log2 trace_len, log2 expansion, width
  * band), the width bands being tables of fewer than 64 columns, 64..255 and

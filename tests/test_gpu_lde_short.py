@@ -123,3 +123,26 @@ def test_randomizers_of_a_part_filled_tile(T, oracle, log_n, E, cols, k):
     """The randomizer terms are spread over the rows that the tile holds, not over
     those it could hold (one column of 2^7 rows: 47 us, 14 with its terms alone)."""
     test_lde_short_columns(T, oracle, log_n, E, cols, k)
+
+
+@pytest.mark.parametrize("log_n,E", [(22, 16), (23, 8)])
+def test_lde_of_2p26(T, log_n, E):
+    """Refused by default, taken by a variant with the 2^14 row tile; each coset is
+    the coset evaluation of the column's coefficients."""
+    n, m, log_e = 1 << log_n, E << log_n, E.bit_length() - 1
+    x, coeff, one, out = T.empty(n), T.empty(n), T.empty(n), T.empty(m)
+    T.lib.fill_uniform(x, n, 4)
+    P = 0xFFFFFFFF00000001
+    with pytest.raises(T.mod.TVHError, match="unsupported"):
+        T.lib.lde_batch(x, 1, n, None, 0, 1, 7, m, out)
+    T.lib.lde_set_variant(log_n, log_e, T.mod.LDE_SPLIT)
+    try:
+        T.lib.lde_batch(x, 1, n, None, 0, 1, 7, m, out)
+    finally:
+        T.lib.lde_set_variant(log_n, log_e, 0)
+    T.lib.trace_coefficients(x, 1, n, 1, coeff)
+    got = T.host(out, m)
+    w = pow(7, (P - 1) // m, P)
+    for s in (0, 1, E - 1):
+        T.lib.evaluate_coset(coeff, 1, n, None, 0, 1, 7 * pow(w, s, P) % P, one)
+        assert np.array_equal(T.host(one, n), got[s::E]), s

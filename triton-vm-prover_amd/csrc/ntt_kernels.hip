@@ -73,7 +73,9 @@ int lde_variant(u32 logN, u32 logE, u64 cols) {
     // Column tiles of 2^13, but 2^12 where those make fewer than four blocks a CU
     // (2^16 x 88: 197 against 204 us; 2^16 x 379: 983 against 916).
     const u32 all = logN + logE;
-    if (all >= 26) return LDE_SPLIT | 1 << 2 | LDE_ROW_HALF;  // (refused, as these shapes ask for a = 13)
+    // 2^26 codeword elements a column are refused by default (prepare_lde; the bound of
+    // the 2^13 row tile does it): only a variant with the 2^14 row tile takes them.
+    if (all >= 26) return LDE_SPLIT | 1 << 2 | LDE_ROW_HALF;
     const u32 b = logN < 20 ? logN - 8 : 12;
     const u32 row = all <= LOG_TILE ? all : b + logE;
     const int col = (cols << logN) < (1ull << 23) ? 2 : 1;
@@ -98,9 +100,10 @@ int set_lde_variant(u32 logN, u32 logE, int v, int wc) {
 // Passes over LDS (or one product) of a transform of length 2^l.
 static u32 passes(u32 l) { return l <= 4 ? 1 : l <= 8 ? 2 : 3; }
 
-// N = N1 * N2, N1 = 2^a.  A row's E coset transforms share one tile (E * N2 <=
-// 2^row_lt, N2 <= 4096: the row step overwrites its input row in place, so a
-// row's cosets cannot be split over blocks).  Within that the split with the
+// N = N1 * N2, N1 = 2^a.  E * N2 <= 2^row_lt, N2 <= 4096: a row's E coset transforms
+// share one tile (the row step overwrites its input row in place, so a row's cosets
+// cannot be split over blocks; rows of 2^12 in four cosets go through a smaller tile
+// one after the other, and keep to the same bound).  Within that the split with the
 // fewest passes, then the longest rows (more contiguous bytes, fewer columns of
 // the strided step).  A column step has at least 2^5 points (shorter ones leave
 // part of the matrices idle) and, if it can, at most 2^9: longer ones leave less
@@ -320,10 +323,11 @@ int prepare_lde(const u64* trace, u64 cols, u64 n, const RandSpec& rs, u64 toff,
         A.src_col_stride = P->k1 ? m : n;
         A.src_row_stride = P->k1 ? ((u64)E << b) : 0;
         // Rows of 2^12 in four cosets: one after the other in a 2^12 tile (2^20 x 379:
-        // 12.3 ms, 12.8 in one tile of 2^14).  Shorter rows in more cosets share a
-        // tile: with two matrices to reload for each coset they are slower one by one
-        // (2^18 x 379, E = 8: LDE 10.1 against 8.4 ms; 2^19 x 264, E = 4: 7.6, 6.7).
-        A.cosets = a > 0 && b == kCosetsLt && logE >= 2 && !batch;
+        // 12.3 ms, 12.8 in one tile of 2^14).  More cosets leave rows of 2^11 and shorter
+        // (choose_split), which share a tile: with two matrices to reload for each coset
+        // they are slower one by one (2^18 x 379, E = 8: LDE 10.1 against 8.4 ms; 2^19 x
+        // 264, E = 4: 7.6, 6.7).
+        A.cosets = a > 0 && b == kCosetsLt && logE == 2 && !batch;
         A.log_c = 0;
         A.products = 0;
         if (b <= 4) {  // a = 0

@@ -1,7 +1,7 @@
-"""Input checks of the host entry points, on a host without a GPU too: the first
-element that is not canonical is named, wherever it is (the caller's head, a
-piece of a worker, the last one), also where several threads check at once, and a
-table is refused before anything else is done for it."""
+"""Input checks of the host commit, on a host without a GPU too: the first element
+that is not canonical is named, wherever it is, also where several threads check
+at once; on a GPU a table is refused before its commit, by the workers that copy it.
+"""
 import re
 import threading
 import time
@@ -17,10 +17,10 @@ def lib(tvhmod):
     return tvhmod.load()
 
 
-def refusal(lib, a):
-    """(status, index named) of a host commit of one column."""
-    root = np.zeros(5, np.uint64)
-    rc = lib.raw("tvh_commit_host", a.ctypes.data, 1, a.size, None, 0, 1, 7, 4 * a.size, None, None,
+def refusal(lib, a, cols=1):
+    """(status, index named) of a host commit."""
+    root, n = np.zeros(5, np.uint64), a.size // cols
+    rc = lib.raw("tvh_commit_host", a.ctypes.data, cols, n, None, 0, 1, 7, 4 * n, None, None,
                  root.ctypes.data)
     m = re.match(r"element (\d+) >= p", lib.last_error())
     return rc, int(m.group(1)) if m else None
@@ -36,11 +36,11 @@ def test_first_bad_element_is_named(lib, log_n):
     rng = np.random.RandomState(log_n)
     status = refusal(lib, np.array([P], np.uint64))[0]
     a = rng.randint(0, P, n, dtype=np.uint64)
-    places = {0, n - 1, n // 2, min(n - 1, 8191), min(n - 1, 8192), min(n - 1, 8192 + 16384 - 1),
-              min(n - 1, 8192 + 16384)} | {int(v) for v in rng.randint(0, n, 8)}
+    places = {0, n - 1, n // 2, min(n - 1, 1023), min(n - 1, 1024), min(n - 1, 8191),
+              min(n - 1, 8192)} | {int(v) for v in rng.randint(0, n, 8)}
     for at in sorted(places):
         b = a.copy()
-        b[at] = P
+        b[rng.randint(0, n, 5)] = P - 1  # canonical, with a high word of ones
         for later in rng.randint(at, n, 3):  # more of them behind it
             b[later] = np.uint64(P + 1 + int(rng.randint(0, 1000)))
         b[at] = P
@@ -67,6 +67,26 @@ def test_threads_check_at_once(lib):
     for t in ts:
         t.join()
     assert not wrong
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("log_n,cols", [(7, 3), (12, 30), (13, 100), (14, 300)])
+def test_first_bad_element_is_named_on_the_way(tvh, log_n, cols):
+    """Copied at once, by the staging workers, and in two pieces of the ring: the ends of
+    their shares (4 KiB steps) and stretches (32 KiB), more of them behind it."""
+    n = cols << log_n
+    status = refusal(tvh, np.array([P], np.uint64))[0]
+    rng = np.random.RandomState(cols)
+    a = rng.randint(0, P, n, dtype=np.uint64)
+    a[rng.randint(0, n, 50)] = P - 1
+    piece, share = 4 << 20, -(-min(n, 4 << 20) // 8 // 512) * 512
+    places = {0, n - 1, 8192, 4096, share - 1, share, 3 * share + 4095, piece - 1, piece, piece + 5}
+    for at in sorted(p for p in places if p < n):
+        b = a.copy()
+        b[rng.randint(at, n, 3)] = P + 5
+        b[at] = P
+        assert refusal(tvh, b, cols) == (status, at)
+    assert refusal(tvh, a, cols)[0] == 0  # and then a good one
 
 
 @pytest.mark.gpu

@@ -715,9 +715,10 @@ struct HostCall {
         bufs.push_back(p);
         return (u64*)p;
     }
-    int up(u64* d, const u64* h, size_t elems) {
+    // bad: as staged_h2d
+    int up(u64* d, const u64* h, size_t elems, size_t* bad = nullptr) {
         if (!elems) return TVH_OK;
-        int e = staged_h2d(d, h, elems * sizeof(u64), st);
+        int e = staged_h2d(d, h, elems * sizeof(u64), st, bad);
         return e ? (rc = e) : TVH_OK;
     }
     int down(u64* h, const u64* d, size_t elems) {
@@ -732,9 +733,11 @@ struct HostCall {
     }
 };
 
+static int refuse_element(size_t i) { return set_error(TVH_ERR_NOT_CANONICAL, "element %zu >= p", i); }
+
 static int check_canonical(const u64* p, size_t n) {
-    const size_t i = first_at_least(p, n, TVH_P);
-    return i < n ? set_error(TVH_ERR_NOT_CANONICAL, "element %zu >= p", i) : TVH_OK;
+    const size_t i = first_not_canonical(p, n);
+    return i < n ? refuse_element(i) : TVH_OK;
 }
 
 static int ntt_host(uint64_t* data, size_t n, bool inv) {
@@ -896,19 +899,19 @@ int tvh_commit_host(const uint64_t* trace, size_t cols, size_t n, const uint64_t
                     uint64_t* root_out) {
     if (!trace || !root_out || (k && !rand)) return set_error(TVH_ERR_INVALID_ARG, "null buffer");
     if (!is_pow2(m)) return set_error(TVH_ERR_NOT_POW2, "target_len");
-    // A refusal comes before any other status, and before the commit is queued: for the
-    // first elements before anything is done, for tables of up to 32 MB (a staging slot;
-    // queued at once) after the copy to the device, beside which the check then runs
-    // (2^12 x 379: 0.88 ms a call, 0.98 with the check first), for larger ones first.
+    // An element that is not canonical is refused before any other status: the first
+    // 64 KB are checked before anything is done, the others as they are copied to the
+    // device (by the staging ring's workers, or here while a small copy is under way),
+    // and the commit is queued only when all have passed.
     const size_t len = cols * n, rand_len = cols * k;
-    const bool beside = len + rand_len <= (4u << 20);
-    int rc = check_canonical(trace, beside && len > 8192 ? 8192 : len);
-    if (!rc && !beside && k) rc = check_canonical(rand, rand_len);
+    int rc = check_canonical(trace, len < 8192 ? len : 8192);
     if (rc) return rc;
+    size_t bad = kUnchecked, bad_rand = kUnchecked;  // as staged_h2d
     auto checked = [&](int status) {
-        int bad = beside ? check_canonical(trace, len) : TVH_OK;
-        if (!bad && beside && k) bad = check_canonical(rand, rand_len);
-        return bad ? bad : status;
+        if (bad == kUnchecked) bad = first_not_canonical(trace, len);
+        if (bad < len) return refuse_element(bad);
+        if (k && bad_rand == kUnchecked) bad_rand = first_not_canonical(rand, rand_len);
+        return k && bad_rand < rand_len ? refuse_element(bad_rand) : status;
     };
     HostCall hc;
     if (hc.rc) return checked(hc.rc);
@@ -917,8 +920,10 @@ int tvh_commit_host(const uint64_t* trace, size_t cols, size_t n, const uint64_t
     u64* dcw = hc.alloc(cols * m);
     u64* dtree = hc.alloc((2 * m - 1) * 5);
     if (hc.rc) return checked(hc.rc);
-    if ((rc = hc.up(dt, trace, len)) || (rc = hc.up(dr, rand, rand_len))) return checked(rc);
-    if ((rc = checked(TVH_OK))) return rc;
+    if ((rc = hc.up(dt, trace, len, &bad))) bad = kUnchecked;
+    if (!rc && (bad == kUnchecked || bad == len) && (rc = hc.up(dr, rand, rand_len, &bad_rand)))
+        bad_rand = kUnchecked;
+    if ((rc = checked(rc))) return rc;
     if ((rc = tvh_commit_dev(dt, cols, n, k ? dr : nullptr, k, toff, goff, m, dcw, dtree,
                              TVH_TREE_LEVEL_ORDER, hc.st)))
         return rc;

@@ -638,15 +638,14 @@ __device__ __forceinline__ const u64* rand_at(const RandSpec& rs, u64 c, u64 r) 
     if (!((rs.limb_mask >> limb) & 1)) return nullptr;
     return rs.ptr + (c / rs.group) * rs.group_stride + limb * rs.limb_stride + r * rs.elem_stride;
 }
-// Factor of randomizer r in coset s.
-__device__ __forceinline__ u64 rand_factor(const LdeArgs& A, u32 s, u64 r) {
-    // select delta_n[s] without a dynamic index (a dynamic index into the
-    // by-value kernel argument would copy it to scratch)
+// delta_n[s] without a dynamic index (which would copy the by-value kernel argument
+// to scratch).  Randomizer r adds *rand_at * rand_delta * o^r to its coefficient.
+__device__ __forceinline__ u64 rand_delta(const LdeArgs& A, u32 s) {
     u64 d = A.delta_n[0];
 #pragma unroll
     for (u32 i = 1; i < 16; i++)
         if (s == i) d = A.delta_n[i];
-    return gl::mul(d, gl::pow(A.toff, r));
+    return d;
 }
 
 // A block takes NT rows (c, k1) (NT * E * N2 = 2^LT) of Y: inverse row DFT to
@@ -677,7 +676,7 @@ struct Rows {
         const u64 r = k1(t) + ((u64)k2 << A.a);
         if (r >= A.rs.k) return 0;
         const u64* p = rand_at(A.rs, A.a ? B.c : B.c + t, r);
-        return p ? gl::mul(*p, rand_factor(A, sl, r)) : 0;
+        return p ? gl::mul(gl::mul(*p, rand_delta(A, sl)), gl::pow(A.toff, r)) : 0;
     }
     // The randomizer terms of the scaled coefficients of the block's rows in cosets
     // s0 .. s0 + 2^log_s - 1 in LDS (transform t * 2^log_s + s): the few elements
@@ -875,7 +874,7 @@ __device__ __forceinline__ void lde_short_body(const LdeArgs& A, u64 blk, const 
         to[v] = o + (o >> 4);
         pb[v] = load_at(A.pb, ((s << logN) + i) * 8);
         pa[v] = load_at(A.pa, s * 8);
-        rf[v] = i < A.rs.k ? rand_factor(A, s, i) : 0;
+        rf[v] = i < A.rs.k ? gl::mul(rand_delta(A, s), gl::pow(A.toff, i)) : 0;
     }
     u64* const buf = lds + wave_index() * kShortPitch;
     const u32 log_cols = 8 - logN - A.logE;  // columns of a product

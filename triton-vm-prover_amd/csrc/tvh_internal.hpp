@@ -54,9 +54,14 @@ DeviceState* initialized_device();
 // Host-to-device copy of `bytes` from pageable host memory on stream st through
 // the device's page-locked staging ring (stager.hip); returns once every piece
 // is queued (the source may then be reused).  Calls on one device take turns.
-int staged_h2d(void* dst, const void* src, size_t bytes, hipStream_t st);
-// Index of the first of n host elements that is at least `limit`, or n.
-size_t first_at_least(const u64* p, size_t n, u64 limit);
+// bad (may be null): the u64 elements are checked on the way; *bad receives the index
+// of the first that is not canonical, whose piece and the ones after it are not
+// sent, or their number.  Copies too small for the ring leave the check to the
+// caller (kUnchecked).
+constexpr size_t kUnchecked = ~(size_t)0;
+int staged_h2d(void* dst, const void* src, size_t bytes, hipStream_t st, size_t* bad = nullptr);
+// Index of the first of n host elements that is not canonical, or n.
+size_t first_not_canonical(const u64* p, size_t n);
 
 // State of the current device, initialised on first use (thread-safe).
 // Returns nullptr and sets the error on failure.

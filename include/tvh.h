@@ -227,7 +227,7 @@ int tvh_trace_coefficients_dev(const uint64_t* d_trace, size_t num_cols, size_t 
  * of coset k is row j*(M/n) + k of the M-point codeword.  d_tail_scratch is
  * accepted for the reference's signature and not used (may be NULL).  Uses the
  * per-device arena for the NTT's transpose step and for the powers of
- * coset_offset that its column step applies to the coefficients as it loads
+ * coset_offset that its first step applies to the coefficients as it loads
  * them.  d_output may equal d_coefficients (in place, which consumes the
  * coefficients) or must not overlap it.
  * Replaces evaluate_coset_from_coefficients_gpu (randomized_lde_kernel.cuh:152-163). */
@@ -545,7 +545,9 @@ int tvh_merkle_tree_host(const uint64_t* leaves, size_t num_leaves, int layout,
 
 /* Whole commit on host buffers (LDETable::compute_lde_and_merkle,
  * src/lde/lde_table.cpp:86-101).  codewords_out (target_len*num_cols,
- * column-major) and digests_out (target_len*5) may be NULL. */
+ * column-major) and digests_out (target_len*5) may be NULL.  An element of trace or
+ * rand that is not canonical is refused (TVH_ERR_NOT_CANONICAL) before the commit is
+ * queued, with the outputs as they were. */
 int tvh_commit_host(const uint64_t* trace, size_t num_cols, size_t trace_len,
                     const uint64_t* rand, size_t rand_len, uint64_t trace_offset,
                     uint64_t target_offset, size_t target_len, uint64_t* codewords_out,

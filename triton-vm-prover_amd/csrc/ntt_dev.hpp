@@ -27,12 +27,12 @@
 // ntt_kernels.hip.
 //
 // Measured on a 2^20 x 379 table to four cosets (3.2 GB in, 12.7 GB out), with
-// radix-16 butterflies on the VALU before: K1 1.49 ms (2.2), K2 12.0 (12.2 in two
+// radix-16 butterflies on the VALU before: K1 1.47 ms (2.2), K2 11.8 (12.2 in two
 // kernels, which wrote and read the coefficients in between), K3 5.4 (7.1).  K1 and
 // K3 move 4.3 and 4.7 TB/s, near what the memory gives a kernel that reads and
 // writes the same amount.  K2 spends most of its time on VALU instructions (per output
 // two products for the twiddles between passes, one for the coset, two for the
-// twiddle on the way out, and 12 operations in each of three DFT passes): 6.7 cycles
+// twiddle on the way out, and 12 operations in each of three DFT passes): 6.6 cycles
 // of a SIMD each, where a saturated SIMD takes 3.7 to 4; the rest is waits on LDS,
 // global loads and barriers.
 #pragma once

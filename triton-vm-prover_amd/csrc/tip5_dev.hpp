@@ -31,7 +31,7 @@
 // What bounds it: VALU issue.  The kernels issue a VALU instruction every 4
 // cycles per SIMD (2 for a few plain 32-bit ones); matrix instructions of one
 // wave run beside the VALU instructions of the others.  Rows of 2^22 x 379
-// (1.6e8 permutations): 18.6 ms, against 28.8 ms with one sponge per lane, the
+// (1.6e8 permutations): 19.3 ms, against 29.2 ms with one sponge per lane, the
 // MDS in f64 FMAs and Montgomery products.
 #pragma once
 
